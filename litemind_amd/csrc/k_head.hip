@@ -177,187 +177,299 @@ __global__ __launch_bounds__(THREADS) void head_logits_kernel(const uint16_t* __
     }
 }
 
-// Weight rows read through the scalar cache (uniform across the lanes).
-typedef const __attribute__((address_space(4))) uint32_t const_u32;
-
-// The same dot products for many tokens, with each token's inputs read from
-// memory once per workgroup rather than once per wave: 64 tokens (one per
-// lane) and four waves of kTokRows rows.  The tokens' inputs pass through LDS in
-// tiles of 64 elements, a kTokStages-slot ring filled by direct-to-LDS buffer
-// loads (each wave a quarter of each tile) and read by all four waves; the rows
-// come through the scalar cache, 16 elements per step.  The steps are
-// pipelined on one wait: at the start of a step everything requested so far is
-// in (lgkmcnt(0)), then the next step's LDS reads and scalar loads are issued,
-// then this step's FMAs run while they land (a scalar load can complete out of
-// order, so no finer wait on the shared counter would be exact).  Every
-// (token, row) pair keeps its 32 chains in one lane and reduces them as
-// head_logits_kernel does, bit for bit.  in_dim % 64 == 0.
-constexpr int kTokRows = 3;    // rows per wave
-constexpr int kTokTile = 64;   // input elements per LDS slot
-constexpr int kTokStages = 4;
-constexpr int kTokStep = 16;   // elements per weight step
+// ---- the same dot products for batches of tokens, on the fp32 matrix cores ----
+//
+// v_mfma_f32_*_f32 forms each output as a chain of fused multiply-adds over k
+// in ascending order, each rounded as fmaf rounds it, subnormals included
+// (checked bit for bit against fmaf on the host over normal, subnormal,
+// overflowing and signed-zero operands for the 32x32x2 and 16x16x4 shapes).
+// dot_bf16's 32 chains are chains of exactly that kind, so one accumulator
+// tile per chain gives every (token, row) pair's chain bit for bit: the k
+// index of one instruction runs over the 2 (or 4) successive 32-element steps
+// of the row, and its operands are one chain's elements of those steps.
+//
+// A workgroup's four waves own 8 chains each (chains 8 w .. 8 w + 7) of one
+// tile of tokens x rows, so a chain's whole sum stays in one register and the
+// four waves share every staged byte.  Tiles: 32 tokens x 32 rows
+// (32x32x2, 128 accumulators per lane), or 16 tokens x 16 NR rows (16x16x4).
+// A stage is 64 (or 128) elements of the tile's rows and tokens, loaded
+// straight to LDS with its 16-byte units XOR-swizzled by row, so that the
+// 16-byte reads of 8 neighbouring lanes fall on distinct banks; DEPTH stages
+// are in flight.  Each wave reads the next stage's operands before this
+// stage's MFMAs, which hide the reads.  At the end the waves exchange their
+// chains through the ring's LDS and reduce them in dot_bf16's order.
+//
+// What bounds it: the fp32 matrix rate (134 TFLOP/s measured for 32x32x2) at
+// 32 and more tokens, the weight stream below.  [102400, 2048] head: 16 tokens
+// 99 us (4.2 TB/s), 32 tokens 139 us (96 TFLOP/s; 8 launches of the few-token
+// kernel: 565 us); [3072, 2048] projection of 77 tokens 14.7 us (VALU chains,
+// one token per lane: about 35).  Small projections end with their longest
+// wave: 16 stages of 8 chains.
 typedef __attribute__((address_space(3))) void head_lds_void;
 constexpr int kHeadBufferWord3 = 0x00020000;  // buffer descriptor word 3, raw 32-bit access
-// s_waitcnt immediates (vmcnt bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8)
-constexpr int kWaitLgkm0 = 0xC07F;             // lgkmcnt(0), the others unconstrained
+// s_waitcnt immediate: vmcnt(n) (bits 3:0 and 15:14), the other counters unconstrained
 constexpr int kWaitVm(int n) { return (n & 15) | ((n >> 4) << 14) | 0x0070 | 0x0F00; }
 
-__global__ __launch_bounds__(256) void matvec_tokens_kernel(const uint16_t* __restrict__ w,
-                                                            const float* __restrict__ x, float* out, int64_t rows,
-                                                            int32_t in_dim, int64_t tokens, float scale,
-                                                            int32_t accumulate) {
-    typedef float f4v __attribute__((ext_vector_type(4)));
-    // slot: 64 tokens x 16 units of 4 elements; unit q of token t at position
-    // t * 16 + (q ^ (t % 16)), so the 16 lanes of each quarter-wave read 16
-    // distinct bank groups.  One array per slot, so the compiler's waits
-    // tell the slots apart.
-    __shared__ __align__(16) float s0[64 * kTokTile], s1[64 * kTokTile], s2[64 * kTokTile], s3[64 * kTokTile];
-    float* const ring[kTokStages] = {s0, s1, s2, s3};
+// 16 bytes per lane straight to LDS (not a template: the host pass checks a
+// template's builtin against its own target, which lacks the 16-byte form).
+__device__ inline void load_lds16(__amdgpu_buffer_rsrc_t from, float* to, unsigned offset, int base) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (head_lds_void*)to, 16, offset, base, 0, 0);
+}
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// One chain's accumulator over the wave's tile: M tokens x (M NR) rows.
+template <int M, int NR>
+struct ChainTile;
+template <int NR>
+struct ChainTile<32, NR> {
+    static_assert(NR == 1);
+    f32x16 v = {};
+    __device__ void step(const float* a, const float (*b)[8], int j) {
+        v = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j], b[0][j], v, 0, 0, 0);
+    }
+    __device__ float get(int quarter, int i) const { return v[4 * quarter + i]; }
+};
+template <int NR>
+struct ChainTile<16, NR> {
+    f32x4 v[NR] = {};
+    __device__ void step(const float* a, const float (*b)[8], int j) {
+#pragma unroll
+        for (int n = 0; n < NR; ++n) {
+            v[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[n][j], v[n], 0, 0, 0);
+        }
+    }
+    __device__ float get(int quarter, int i) const { return v[i][quarter]; }
+};
+
+template <int M, int NR>
+struct ExactTile {
+    static constexpr int kSteps = M == 32 ? 2 : 4;       // 32-element steps per instruction and stage
+    static constexpr int kElems = 32 * kSteps;           // row elements per stage
+    static constexpr int kRowsT = M * NR;                // weight rows per tile
+    static constexpr int kXUnits = kElems / 4;           // 16-byte units of a token's stage
+    static constexpr int kWUnits = kElems / 8;           // 16-byte units of a row's stage
+    static constexpr int kXLoads = M * kXUnits / 256;    // loads per wave and stage
+    static constexpr int kWLoads = kRowsT * kWUnits / 256;
+    static constexpr int kLoads = kXLoads + kWLoads;
+    static constexpr int kStageFloats = M * kElems + kRowsT * kElems / 2;
+    static constexpr int kQuarter = M == 32 ? 4 : NR;    // accumulators of a chain that one wave finishes
+    static_assert(kXLoads >= 1 && kWLoads >= 1);
+};
+
+// in_dim % (32 kSteps) == 0.  `nt` token tiles, `nr` row tiles; workgroups that
+// share rows lie 8 apart in the grid, on one XCD.
+template <int M, int NR, int DEPTH, bool BEST>
+__global__ __launch_bounds__(256, 2) void matvec_exact_kernel(const uint16_t* __restrict__ w,
+                                                              const float* __restrict__ x, float* out,
+                                                              HeadBest* partial, int64_t rows, int32_t in_dim,
+                                                              int32_t tokens, int32_t nt, int32_t nr, float scale,
+                                                              int32_t accumulate) {
+    using T = ExactTile<M, NR>;
+    // One array per stage, so that the compiler's waits tell the stages apart.
+    __shared__ __align__(16) float s0[T::kStageFloats], s1[T::kStageFloats], s2[T::kStageFloats],
+        s3[T::kStageFloats], s4[DEPTH > 4 ? T::kStageFloats : 1], s5[DEPTH > 5 ? T::kStageFloats : 1];
+    static_assert(DEPTH >= 4 && DEPTH <= 6);
+    float* const ring[6] = {s0, s1, s2, s3, s4, s5};
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-    const int64_t t0 = static_cast<int64_t>(blockIdx.x) * 64;
-    const int64_t ntok = std::min<int64_t>(64, tokens - t0);
-    const int64_t row0 = (static_cast<int64_t>(blockIdx.y) * 4 + wave) * kTokRows;
-    const_u32* wr[kTokRows];
-#pragma unroll
-    for (int r = 0; r < kTokRows; ++r) {
-        const int64_t row = row0 + r < rows ? row0 + r : rows - 1;  // rows past the end load the last, store nothing
-        wr[r] = (const_u32*)(w + row * in_dim);
+    const int slot_id = static_cast<int>(blockIdx.x) / 8;
+    const int tt = slot_id % nt;
+    const int rt = slot_id / nt * 8 + static_cast<int>(blockIdx.x) % 8;
+    if (rt >= nr) {
+        return;
     }
-    const int ntiles = in_dim / kTokTile;
-    // this wave's four loads of a tile: load j covers positions (4 wave + j) 64
-    // + lane, i.e. token u / 16 and unit (u % 16) ^ (token % 16); tokens past
-    // the last read the last
+    const int t0 = tt * M;
+    const int ntok = min(M, tokens - t0);
+    const int64_t row0 = static_cast<int64_t>(rt) * T::kRowsT;
+    const int nrow = static_cast<int>(std::min<int64_t>(T::kRowsT, rows - row0));
+    const int stages = in_dim / T::kElems;
     const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(x + t0 * in_dim), 0, static_cast<int>(ntok * in_dim * 4), kHeadBufferWord3);
-    unsigned src[4];
+        (void*)(x + static_cast<int64_t>(t0) * in_dim), 0, ntok * in_dim * 4, kHeadBufferWord3);
+    const __amdgpu_buffer_rsrc_t wres =
+        __builtin_amdgcn_make_buffer_rsrc((void*)(w + row0 * in_dim), 0, nrow * in_dim * 2, kHeadBufferWord3);
+    // Load j of a stage fills 64 consecutive 16-byte positions p; position p of
+    // row (or token) r = p / units holds its unit (p % units) ^ (r % 16), with
+    // the XOR cut to the row's units.  Rows past the end load the last one.
+    unsigned xsrc[T::kXLoads], wsrc[T::kWLoads];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int u = (4 * wave + j) * 64 + lane;
-        const int tt = u >> 4;
-        const int q = (u & 15) ^ (tt & 15);
-        const int ttc = tt < ntok ? tt : static_cast<int>(ntok) - 1;
-        src[j] = static_cast<unsigned>((ttc * in_dim + 4 * q) * 4);
+    for (int j = 0; j < T::kXLoads; ++j) {
+        const int p = (wave * T::kXLoads + j) * 64 + lane;
+        const int r = p / T::kXUnits;
+        const int u = (p % T::kXUnits) ^ (r & 15);
+        xsrc[j] = static_cast<unsigned>((min(r, ntok - 1) * in_dim + 4 * u) * 4);
     }
-    auto issue = [&](int tile, float* slot) {
-        tile = tile < ntiles ? tile : ntiles - 1;  // past the end: reload the last tile (every step issues alike)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(xres, (head_lds_void*)(slot + (4 * wave + j) * 256), 16,
-                                                     src[j] + static_cast<unsigned>(tile * kTokTile * 4), 0, 0, 0);
+    for (int j = 0; j < T::kWLoads; ++j) {
+        const int p = (wave * T::kWLoads + j) * 64 + lane;
+        const int r = p / T::kWUnits;
+        const int u = (p % T::kWUnits) ^ (r & (T::kWUnits - 1));
+        wsrc[j] = static_cast<unsigned>((min(r, nrow - 1) * in_dim + 8 * u) * 2);
+    }
+    auto issue = [&](int stage, float* slot) {
+        stage = stage < stages ? stage : stages - 1;  // past the end: the last again (every stage issues alike)
+#pragma unroll
+        for (int j = 0; j < T::kXLoads; ++j) {
+            load_lds16(xres, slot + (wave * T::kXLoads + j) * 256, xsrc[j], stage * (T::kElems * 4));
+        }
+#pragma unroll
+        for (int j = 0; j < T::kWLoads; ++j) {
+            load_lds16(wres, slot + M * T::kElems + (wave * T::kWLoads + j) * 256, wsrc[j], stage * (T::kElems * 2));
         }
     };
-    float acc[kTokRows][32];
+    // This lane's operands of a stage: step k = lane / M of token and row
+    // lane % M, the wave's 8 chains.
+    const int li = lane % M;
+    const int lk = lane / M;
+    const int xu = 8 * lk + 2 * wave;
+    const int wu = 4 * lk + wave;
+    auto read = [&](const float* slot, f32x4 (&xv)[2], uint4 (&wv)[NR]) {
+        xv[0] = *reinterpret_cast<const f32x4*>(slot + li * T::kElems + 4 * (xu ^ (li & 15)));
+        xv[1] = *reinterpret_cast<const f32x4*>(slot + li * T::kElems + 4 * ((xu + 1) ^ (li & 15)));
 #pragma unroll
-    for (int r = 0; r < kTokRows; ++r) {
-#pragma unroll
-        for (int c = 0; c < 32; ++c) {
-            acc[r][c] = 0.0f;
+        for (int n = 0; n < NR; ++n) {
+            const int r = n * M + li;
+            wv[n] = *reinterpret_cast<const uint4*>(slot + M * T::kElems + r * (T::kElems / 2) +
+                                                    4 * (wu ^ (r & (T::kWUnits - 1))));
         }
-    }
-    f4v xa[4], xb[4];
-    uint32_t wa[kTokRows][8], wb[kTokRows][8];
-    const int sw = lane & 15;
-    // step `st` (0..3) of `tile` from `slot`: the lane's token's 16 inputs and
-    // each row's 16 weights (8 bf16 pairs)
-    auto read = [&](const float* slot, int tile, int st, f4v (&xv)[4], uint32_t (&wv)[kTokRows][8]) {
+    };
+    ChainTile<M, NR> acc[8];
+    auto mfma = [&](const f32x4 (&xv)[2], const uint4 (&wv)[NR]) {
+        float a[8], b[NR][8];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            xv[i] = *reinterpret_cast<const f4v*>(slot + (lane * 16 + ((4 * st + i) ^ sw)) * 4);
+        for (int j = 0; j < 8; ++j) {
+            a[j] = xv[j / 4][j % 4];
         }
-        const int e = (tile < ntiles ? tile : ntiles - 1) * kTokTile + st * kTokStep;
 #pragma unroll
-        for (int r = 0; r < kTokRows; ++r) {
+        for (int n = 0; n < NR; ++n) {
+            const uint32_t pair[4] = {wv[n].x, wv[n].y, wv[n].z, wv[n].w};
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                wv[r][k] = wr[r][e / 2 + k];
+            for (int j = 0; j < 4; ++j) {
+                b[n][2 * j] = bits_float(pair[j] << 16);
+                b[n][2 * j + 1] = bits_float(pair[j] & 0xffff0000u);
             }
         }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            acc[j].step(a, b, j);
+        }
     };
-    // elements e .. e + 15 of a step with parity `half` (e % 32 == 16 half):
-    // element e + m on chain 16 half + m
-    auto fma_step = [&](int half, const f4v (&xv)[4], const uint32_t (&wv)[kTokRows][8]) {
 #pragma unroll
-        for (int r = 0; r < kTokRows; ++r) {
+    for (int d = 0; d < DEPTH - 1; ++d) {
+        issue(d, ring[d]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(kWaitVm(T::kLoads * (DEPTH - 2)));  // stage 0 is in
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 xv[2][2];
+    uint4 wv[2][NR];
+    read(ring[0], xv[0], wv[0]);
+    auto stage_step = [&](int s, int u) {  // u: s modulo kTrip, a constant once unrolled
+        // stage s + 1 is in, and every wave has the operands of s - 1: its slot
+        // takes stage s + DEPTH - 1
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(kWaitVm(T::kLoads * (DEPTH - 3)));
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        issue(s + DEPTH - 1, ring[(u + DEPTH - 1) % DEPTH]);
+        read(ring[(u + 1) % DEPTH], xv[(u + 1) & 1], wv[(u + 1) & 1]);
+        __builtin_amdgcn_sched_barrier(0);  // the reads go out before the MFMAs that hide them
+        mfma(xv[u & 1], wv[u & 1]);
+    };
+    // Whole trips without a branch between stages: where paths join, the
+    // compiler waits for the most recent loads of either.
+    constexpr int kTrip = DEPTH % 2 == 0 ? DEPTH : 2 * DEPTH;  // ring slots and register sets are constants
+    int s = 0;
+    for (; s + kTrip <= stages; s += kTrip) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
+        for (int u = 0; u < kTrip; ++u) {
+            stage_step(s + u, u);
+        }
+    }
 #pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const uint32_t pair = wv[r][2 * i + j];
-                    const int c = 16 * half + 4 * i + 2 * j;
-                    acc[r][c] = __builtin_fmaf(bits_float(pair << 16), xv[i][2 * j], acc[r][c]);
-                    acc[r][c + 1] = __builtin_fmaf(bits_float(pair & 0xffff0000u), xv[i][2 * j + 1], acc[r][c + 1]);
+    for (int u = 0; u < kTrip - 1; ++u) {
+        if (s + u < stages) {
+            stage_step(s + u, u);
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(kWaitVm(0));  // every load to LDS has landed before the ring is reused
+    __syncthreads();
+    // Exchange: wave q finishes quarter q of the accumulators.  `ex` holds, for
+    // each source wave, quarter and accumulator, four chains of 64 lanes; the
+    // stage arrays are carved into 4-KB blocks.
+    constexpr int kBlocksPerStage = T::kStageFloats / 1024;
+    auto block = [&](int b) -> float* {  // b is a constant once unrolled
+        return ring[b / kBlocksPerStage] + b % kBlocksPerStage * 1024;
+    };
+    static_assert(4 * T::kQuarter <= kBlocksPerStage * DEPTH, "a round of the exchange fits the ring");
+    float ls[T::kQuarter][8];
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        // block (quarter, i): source wave s at 256 s + 4 lane
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+#pragma unroll
+            for (int i = 0; i < T::kQuarter; ++i) {
+                f32x4 v;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    v[j] = acc[4 * half + j].get(q, i);
+                }
+                *reinterpret_cast<f32x4*>(block(q * T::kQuarter + i) + wave * 256 + 4 * lane) = v;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (wave == q) {
+#pragma unroll
+                for (int i = 0; i < T::kQuarter; ++i) {
+                    const float* from = block(q * T::kQuarter + i) + 4 * lane;
+                    const f32x4 a0 = *reinterpret_cast<const f32x4*>(from);
+                    const f32x4 a1 = *reinterpret_cast<const f32x4*>(from + 256);
+                    const f32x4 a2 = *reinterpret_cast<const f32x4*>(from + 512);
+                    const f32x4 a3 = *reinterpret_cast<const f32x4*>(from + 768);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        // (a[l] + a[8 + l]) + (a[16 + l] + a[24 + l])
+                        ls[i][4 * half + j] = (a0[j] + a1[j]) + (a2[j] + a3[j]);
+                    }
                 }
             }
         }
-    };
-    auto wait_all_lgkm = [] {
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
-        __builtin_amdgcn_sched_barrier(0);
-    };
-#pragma unroll
-    for (int d = 0; d < kTokStages - 1; ++d) {
-        issue(d, ring[d]);
+        __syncthreads();
     }
-    __builtin_amdgcn_s_waitcnt(kWaitVm(4 * (kTokStages - 2)));  // tile 0 is in
-    __builtin_amdgcn_s_barrier();
-    read(ring[0], 0, 0, xa, wa);
-    for (int tb = 0; tb < ntiles; tb += kTokStages) {
 #pragma unroll
-        for (int j = 0; j < kTokStages; ++j) {
-            const int tile = tb + j;  // tiles past the end load alike and add nothing
-            const float* slot = ring[j];
-            const bool live = tile < ntiles;
-            wait_all_lgkm();
-            read(slot, tile, 1, xb, wb);
-            __builtin_amdgcn_sched_barrier(0);
-            if (live) {
-                fma_step(0, xa, wa);
-            }
-            wait_all_lgkm();
-            read(slot, tile, 2, xa, wa);
-            __builtin_amdgcn_sched_barrier(0);
-            if (live) {
-                fma_step(1, xb, wb);
-            }
-            wait_all_lgkm();
-            read(slot, tile, 3, xb, wb);
-            __builtin_amdgcn_sched_barrier(0);
-            if (live) {
-                fma_step(0, xa, wa);
-            }
-            wait_all_lgkm();
-            // tile + 1 is in (the one issued after it may still be in flight),
-            // and every wave has read all of tile - 1: its slot takes tile + 3
-            __builtin_amdgcn_s_waitcnt(kWaitVm(4 * (kTokStages - 3)));
-            __builtin_amdgcn_s_barrier();
-            issue(tile + kTokStages - 1, ring[(j + kTokStages - 1) % kTokStages]);
-            read(ring[(j + 1) % kTokStages], tile + 1, 0, xa, wa);
-            __builtin_amdgcn_sched_barrier(0);
-            if (live) {
-                fma_step(1, xb, wb);
-            }
-        }
-    }
-    __builtin_amdgcn_s_waitcnt(0);  // every load to LDS has landed before the workgroup ends
-    const int64_t t = t0 + lane;
-#pragma unroll
-    for (int r = 0; r < kTokRows; ++r) {
-        // (a[l] + a[8 + l]) + (a[16 + l] + a[24 + l]), lanes j and j + 4, (h0 + h2) + (h1 + h3)
-        float ls[8];
-#pragma unroll
-        for (int l = 0; l < 8; ++l) {
-            ls[l] = (acc[r][l] + acc[r][8 + l]) + (acc[r][16 + l] + acc[r][24 + l]);
-        }
-        const float h0 = ls[0] + ls[4];
-        const float h1 = ls[1] + ls[5];
-        const float h2 = ls[2] + ls[6];
-        const float h3 = ls[3] + ls[7];
+    for (int i = 0; i < T::kQuarter; ++i) {
+        // lanes j and j + 4, (h0 + h2) + (h1 + h3)
+        const float h0 = ls[i][0] + ls[i][4];
+        const float h1 = ls[i][1] + ls[i][5];
+        const float h2 = ls[i][2] + ls[i][6];
+        const float h3 = ls[i][3] + ls[i][7];
         const float total = (h0 + h2) + (h1 + h3);
-        if (t < tokens && row0 + r < rows) {
-            float* o = out + t * rows + row0 + r;
+        const int t = M == 32 ? 8 * wave + 4 * lk + i : 4 * lk + wave;
+        const int r = M == 32 ? li : M * i + li;
+        const int64_t row = row0 + r;
+        const bool live = t < ntok && r < nrow;
+        if (live) {
+            float* o = out + static_cast<int64_t>(t0 + t) * rows + row;
             *o = accumulate ? __builtin_fmaf(scale, total, *o) : total;
+        }
+        if constexpr (BEST) {
+            // the tile's best row of each token: the M lanes that share it, then
+            // (16-token tiles) one candidate per 16 rows
+            HeadBest b{total, static_cast<int32_t>(row), live && total == total ? 1 : 0};
+#pragma unroll
+            for (int o = M / 2; o >= 1; o >>= 1) {
+                const HeadBest other{__shfl_xor(b.v, o), __shfl_xor(b.i, o), __shfl_xor(b.have, o)};
+                b = better(b, other);
+            }
+            if (li == 0 && t < ntok) {
+                const int64_t per = static_cast<int64_t>(nr) * NR;
+                partial[static_cast<int64_t>(t0 + t) * per + static_cast<int64_t>(rt) * NR + (M == 32 ? 0 : i)] = b;
+            }
         }
     }
 }
@@ -435,19 +547,106 @@ __global__ __launch_bounds__(1024) void argmax_first_kernel(const HeadBest* __re
     }
 }
 
+// Tile shapes of matvec_exact_kernel.
+enum class ExactShape { k32, k16x2, k16x1 };
+
+bool exact_supported(int64_t in_dim) { return in_dim % 64 == 0; }
+
+// The shape with the least expected time: a start-up part plus a part per round
+// of the 256 CUs, in tenths of a microsecond at in_dim 2048 (measured at 576 to
+// 102400 rows and 5 to 128 tokens: one round 14.7 / 10.3 / 8.0, two 22.7 / 14.6
+// / 9.3 us).  Few tiles end sooner as small ones, which spread over more CUs
+// (kv_a, 576 rows x 77 tokens: 6.7 us as 16 x 16 tiles, 14.5 as 32 x 32); many
+// tiles do fewer LDS reads per multiply-add as large ones (102400 rows x 32
+// tokens: 139 us as 32 x 32 tiles, 160 as 16 x 32).
+ExactShape exact_shape(int64_t rows, int64_t in_dim, int64_t tokens) {
+    if (in_dim % 128 != 0) {
+        return ExactShape::k32;
+    }
+    auto rounds = [&](int64_t m, int64_t r) {
+        return (((tokens + m - 1) / m) * ((rows + r - 1) / r) + 255) / 256;
+    };
+    const int64_t c32 = 70 + 76 * rounds(32, 32), c16x2 = 60 + 43 * rounds(16, 32), c16x1 = 50 + 32 * rounds(16, 16);
+    if (c32 <= c16x2 && c32 <= c16x1) {
+        return ExactShape::k32;
+    }
+    return c16x2 <= c16x1 ? ExactShape::k16x2 : ExactShape::k16x1;
+}
+
+template <int M, int NR, int DEPTH>
+hipError_t launch_exact_shape(const uint16_t* w, const float* x, float* out, HeadBest* partial, int64_t rows,
+                              int64_t in_dim, int64_t tokens, float scale, int32_t accumulate, hipStream_t s) {
+    const int64_t nt = (tokens + M - 1) / M;
+    const int64_t nr = (rows + M * NR - 1) / (M * NR);
+    const int64_t grid = (nr + 7) / 8 * 8 * nt;
+    if (grid > INT32_MAX || tokens > INT32_MAX) {
+        return hipErrorInvalidValue;
+    }
+    if (partial != nullptr) {
+        hipLaunchKernelGGL((matvec_exact_kernel<M, NR, DEPTH, true>), dim3(static_cast<unsigned>(grid)), dim3(256), 0,
+                           s, w, x, out, partial, rows, static_cast<int32_t>(in_dim), static_cast<int32_t>(tokens),
+                           static_cast<int32_t>(nt), static_cast<int32_t>(nr), scale, accumulate);
+    } else {
+        hipLaunchKernelGGL((matvec_exact_kernel<M, NR, DEPTH, false>), dim3(static_cast<unsigned>(grid)), dim3(256), 0,
+                           s, w, x, out, partial, rows, static_cast<int32_t>(in_dim), static_cast<int32_t>(tokens),
+                           static_cast<int32_t>(nt), static_cast<int32_t>(nr), scale, accumulate);
+    }
+    return hipGetLastError();
+}
+
+// `blocks`: candidates per token in `partial` (when given).
+hipError_t launch_exact(const uint16_t* w, const float* x, float* out, HeadBest* partial, int64_t* blocks,
+                        int64_t rows, int64_t in_dim, int64_t tokens, float scale, int32_t accumulate,
+                        hipStream_t s) {
+    const ExactShape shape = exact_shape(rows, in_dim, tokens);
+    if (blocks != nullptr) {
+        *blocks = shape == ExactShape::k16x2 ? (rows + 31) / 32 * 2 : shape == ExactShape::k32 ? (rows + 31) / 32
+                                                                                            : (rows + 15) / 16;
+    }
+    switch (shape) {
+        case ExactShape::k32:
+            return launch_exact_shape<32, 1, 6>(w, x, out, partial, rows, in_dim, tokens, scale, accumulate, s);
+        case ExactShape::k16x2:
+            return launch_exact_shape<16, 2, 4>(w, x, out, partial, rows, in_dim, tokens, scale, accumulate, s);
+        default:
+            return launch_exact_shape<16, 1, 4>(w, x, out, partial, rows, in_dim, tokens, scale, accumulate, s);
+    }
+}
+
 }  // namespace
 
-int64_t head_blocks(int64_t rows) { return (rows + kRows - 1) / kRows; }
+int64_t head_batch(int64_t in_dim) {
+    if (exact_supported(in_dim)) {
+        return kHeadBatch;
+    }
+    return std::max<int64_t>(1, std::min<int64_t>(kHeadTokens, 16384 / in_dim));
+}
+
+int64_t head_candidates(int64_t rows, int64_t in_dim) {
+    const int64_t few = kHeadTokens * ((rows + kRows - 1) / kRows);
+    // at most one per 16 rows and token with 16-token tiles, one per 32 with 32-token tiles
+    return exact_supported(in_dim) ? std::max(few, kHeadBatch * 2 * ((rows + 31) / 32)) : few;
+}
 
 hipError_t launch_head(const uint16_t* w, const float* x, float* logits, HeadBest* partial, int32_t* token,
                        int64_t rows, int32_t in_dim, int32_t tokens, hipStream_t s) {
     if (rows <= 0 || tokens <= 0) {
         return hipSuccess;
     }
-    if (tokens > kHeadTokens || in_dim <= 0 || in_dim % 8 != 0 || rows > INT32_MAX) {
+    if (tokens > head_batch(in_dim) || in_dim <= 0 || in_dim % 8 != 0 || rows > INT32_MAX) {
         return hipErrorInvalidValue;
     }
-    const int64_t blocks = head_blocks(rows);
+    int64_t blocks = (rows + kRows - 1) / kRows;
+    if (tokens > kHeadTokens) {
+        const hipError_t err = launch_exact(w, x, logits, token != nullptr ? partial : nullptr, &blocks, rows, in_dim,
+                                            tokens, 1.0f, 0, s);
+        if (err != hipSuccess || token == nullptr) {
+            return err;
+        }
+        hipLaunchKernelGGL(argmax_first_kernel, dim3(static_cast<unsigned>(tokens)), dim3(1024), 0, s, partial,
+                           static_cast<int32_t>(blocks), logits, rows, token);
+        return hipGetLastError();
+    }
     const size_t lds = sizeof(float) * static_cast<size_t>(tokens) * static_cast<size_t>(in_dim);
     if (lds > 64 * 1024) {
         return hipErrorInvalidValue;
@@ -472,7 +671,7 @@ hipError_t launch_matvec_rows(const uint16_t* w, const float* x, float* out, int
     if (!matvec_rows_supported(rows, in_dim)) {
         return hipErrorInvalidValue;
     }
-    hipLaunchKernelGGL(head_logits_kernel<kThreads>, dim3(static_cast<unsigned>(head_blocks(rows))), dim3(kThreads),
+    hipLaunchKernelGGL(head_logits_kernel<kThreads>, dim3(static_cast<unsigned>((rows + kRows - 1) / kRows)), dim3(kThreads),
                        sizeof(float) * static_cast<size_t>(in_dim), s, w, x, out, nullptr, rows,
                        static_cast<int32_t>(in_dim), 1, scale, accumulate);
     return hipGetLastError();
@@ -496,12 +695,12 @@ hipError_t launch_matvec_tokens(const uint16_t* w, const float* x, float* out, i
         }
         return hipGetLastError();
     }
-    if (tokens > kHeadTokens && in_dim % 64 == 0) {
-        const dim3 grid(static_cast<unsigned>((tokens + 63) / 64),
-                        static_cast<unsigned>((rows + 4 * kTokRows - 1) / (4 * kTokRows)));
-        hipLaunchKernelGGL(matvec_tokens_kernel, grid, dim3(256), 0, s, w, x, out, rows,
-                           static_cast<int32_t>(in_dim), tokens, scale, accumulate);
-        return hipGetLastError();
+    // Few tokens on few rows: the tiles spread 2 to 4 tokens over the CUs too
+    // (4096 x 2048, 4 tokens: 8.4 us against 24.7 a row at a time); from some
+    // 20,000 rows on, streaming the rows past the vector units is as fast
+    // (24576 x 2048, 2 tokens: 24.5 us against 25.0).
+    if (exact_supported(in_dim) && (tokens > kHeadTokens || rows <= 16384)) {
+        return launch_exact(w, x, out, nullptr, nullptr, rows, in_dim, tokens, scale, accumulate, s);
     }
     // tokens per launch: at most kHeadTokens, and their rows must fit 64 KiB of LDS
     const int64_t per = std::min<int64_t>(kHeadTokens, std::max<int64_t>(1, 16384 / in_dim));

@@ -196,7 +196,7 @@ struct lm_context {
     float* gemm_out = nullptr;   // output
     size_t gemm_cap = 0;         // floats in each scratch buffer
     // LM head: final norm [H] fp32, head [V, H] BF16, and scratch for one group of
-    // lm::kHeadTokens tokens (normalised hidden states, logits when the caller
+    // lm::head_batch tokens (normalised hidden states, logits when the caller
     // passes none)
     float* head_norm = nullptr;
     uint16_t* head_w = nullptr;
@@ -1395,12 +1395,13 @@ int lm_upload_head(lm_context* ctx, const float* norm_host, const uint16_t* head
     ctx->head_logits = nullptr;
     ctx->head_partial = nullptr;
     ctx->vocab = 0;
+    const size_t batch = static_cast<size_t>(lm::head_batch(ctx->H));
     LM_HIP(hipMalloc(reinterpret_cast<void**>(&ctx->head_norm), sizeof(float) * H));
     LM_HIP(hipMalloc(reinterpret_cast<void**>(&ctx->head_w), sizeof(uint16_t) * V * H));
-    LM_HIP(hipMalloc(reinterpret_cast<void**>(&ctx->head_x), sizeof(float) * lm::kHeadTokens * H));
-    LM_HIP(hipMalloc(reinterpret_cast<void**>(&ctx->head_logits), sizeof(float) * lm::kHeadTokens * V));
+    LM_HIP(hipMalloc(reinterpret_cast<void**>(&ctx->head_x), sizeof(float) * batch * H));
+    LM_HIP(hipMalloc(reinterpret_cast<void**>(&ctx->head_logits), sizeof(float) * batch * V));
     LM_HIP(hipMalloc(reinterpret_cast<void**>(&ctx->head_partial),
-                     sizeof(lm::HeadBest) * lm::kHeadTokens * static_cast<size_t>(lm::head_blocks(vocab))));
+                     sizeof(lm::HeadBest) * static_cast<size_t>(lm::head_candidates(vocab, ctx->H))));
     LM_HIP(hipMemcpy(ctx->head_norm, norm_host, sizeof(float) * H, hipMemcpyHostToDevice));
     LM_HIP(hipMemcpy(ctx->head_w, head_host, sizeof(uint16_t) * V * H, hipMemcpyHostToDevice));
     ctx->vocab = vocab;
@@ -1422,8 +1423,7 @@ int lm_head_forward(lm_context* ctx, const float* hidden_dev, int64_t tokens, fl
         return rc;
     }
     const int64_t H = ctx->H, V = ctx->vocab;
-    // tokens per launch: at most kHeadTokens, and their H floats each within 64 KB of LDS
-    const int64_t group = std::max<int64_t>(1, std::min<int64_t>(lm::kHeadTokens, 16384 / H));
+    const int64_t group = lm::head_batch(H);
     for (int64_t t0 = 0; t0 < tokens; t0 += group) {
         const int32_t n = static_cast<int32_t>(tokens - t0 < group ? tokens - t0 : group);
         float* logits = logits_dev != nullptr ? logits_dev + t0 * V : ctx->head_logits;

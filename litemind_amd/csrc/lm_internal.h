@@ -239,16 +239,20 @@ hipError_t launch_spec_gateup(const RouterArgs& r, const ExpertArgs& e, uint32_t
                               int parity, uint32_t seq, int perturb, uint32_t max_spins, hipStream_t s);
 hipError_t launch_permute(const PermuteArgs& a, hipStream_t s);
 // LM head (k_head.hip): logits [tokens, rows] = w [rows, in_dim] . x [tokens, in_dim]
-// with gemm::dot_bf16's association, tokens <= kHeadTokens, in_dim % 8 == 0; and
-// the greedy choice per token (first maximum of the non-NaN logits).
+// with gemm::dot_bf16's association, tokens <= head_batch(in_dim), in_dim % 8 == 0;
+// and the greedy choice per token (first maximum of the non-NaN logits).  Up to
+// kHeadTokens tokens stream the weights past the vector units; more take the
+// fp32 matrix cores where in_dim allows it (matvec_exact_kernel).
 constexpr int kHeadTokens = 4;
+constexpr int64_t kHeadBatch = 64;
 struct HeadBest {
     float v;
     int32_t i;
     int32_t have;
 };
-// Blocks of the head launch; partial holds kHeadTokens * head_blocks(rows) candidates.
-int64_t head_blocks(int64_t rows);
+// Tokens of one head launch at most, and the candidates that its `partial` holds.
+int64_t head_batch(int64_t in_dim);
+int64_t head_candidates(int64_t rows, int64_t in_dim);
 // token may be null (logits only).
 hipError_t launch_head(const uint16_t* w, const float* x, float* logits, HeadBest* partial, int32_t* token,
                        int64_t rows, int32_t in_dim, int32_t tokens, hipStream_t s);
@@ -258,9 +262,8 @@ hipError_t launch_head(const uint16_t* w, const float* x, float* logits, HeadBes
 bool matvec_rows_supported(int64_t rows, int64_t in_dim);
 hipError_t launch_matvec_rows(const uint16_t* w, const float* x, float* out, int64_t rows, int64_t in_dim, float scale,
                               int32_t accumulate, hipStream_t s);
-// The same kernel over T tokens x [T, in_dim] -> out [T, rows] (or out +=
-// fma(scale, ., out)), one wave per 16 rows, in launches of up to kHeadTokens
-// tokens; conditions as matvec_rows_supported.
+// The same dot products over T tokens x [T, in_dim] -> out [T, rows] (or out +=
+// fma(scale, ., out)); conditions as matvec_rows_supported.
 hipError_t launch_matvec_tokens(const uint16_t* w, const float* x, float* out, int64_t rows, int64_t in_dim,
                                 int64_t tokens, float scale, int32_t accumulate, hipStream_t s);
 // gemm::rms_norm (src/Gemm.cpp:197-207) adds the exact double squares in

@@ -1,0 +1,504 @@
+// k_flash.hip -- the attention core of a batch of query tokens in one launch
+// (fp16 operands, fp32 sums), for heads of 128 + 64 key channels and 128 value
+// channels (DeepSeek-V2 and V2-Lite).
+//
+// Reference: the scores, softmax and context of Attention::forward
+// (src/Attention.cpp:77-98), within the MFMA path's tolerance: queries, keys
+// and values rounded to fp16, every sum in fp32, the probabilities
+// exp(scale (s - m)) rounded to fp16 as the second product's operand and
+// summed unrounded.
+//
+// The scores never leave the registers.  A wave owns 32 query tokens of one
+// head and walks the cached keys in tiles of 64: S^T = K Q^T, so that each
+// lane holds the scores of one query (column lane % 32; the two half waves
+// hold alternate groups of four keys), the running maximum and total are one
+// value per lane, and the probabilities of a lane are already the B operand of
+// ctx^T = V^T P^T, whose K order is free: the values are stored with the keys
+// of each group of 16 in the order in which the lanes hold them.  Waves of a
+// workgroup share the key and value tiles, staged straight to LDS two tiles
+// deep; 16-byte units are XOR-swizzled by row so the fragment reads of 8
+// neighbouring lanes fall on distinct banks.
+//
+// Few query tokens over many keys would leave most CUs idle: the keys are then
+// split over several workgroups, whose unnormalised contexts, maxima and
+// totals flash_combine_kernel joins.
+#include "lm_internal.h"
+
+#include <algorithm>
+
+namespace lm {
+namespace {
+
+constexpr int kNope = 128;
+constexpr int kRope = 64;
+constexpr int kQk = kNope + kRope;
+constexpr int kVh = 128;
+constexpr int kTile = 64;                       // keys per tile
+constexpr int kKeyBytes = kTile * kQk * 2;      // 24 KB
+constexpr int kValueBytes = kTile * kVh * 2;    // 16 KB
+constexpr int kKeyLoads = kKeyBytes / 1024;     // wave loads of 1 KB
+constexpr int kValueLoads = kValueBytes / 1024;
+constexpr int kBufferWord3 = 0x00020000;        // buffer descriptor word 3, raw 32-bit access
+
+typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef __attribute__((address_space(3))) void lds_void;
+
+__device__ inline void load_lds16(__amdgpu_buffer_rsrc_t from, char* to, unsigned offset, int base) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (lds_void*)to, 16, offset, base, 0, 0);
+}
+
+// ---- fp16 copies of the cache ----
+//   keys16    [heads][Kp][192]           row j = [key_nope(h, :, j) | key_rope(:, j)]
+//   values16  [heads][Kp / 64][128][64]  value(h, j, :) transposed per tile of 64
+//                                        keys, each 16 in the order 0-3, 8-11,
+//                                        4-7, 12-15: half wave h's scores are
+//                                        keys 4 h .. + 3 and 8 + 4 h .. + 3, its k
+//                                        indices 8 h .. + 7 of the second product
+// Kp = keys rounded up to 64, zeros past the last key.  Workgroup (tile, head).
+__global__ __launch_bounds__(256) void flash_pack_kernel(const float* __restrict__ key_nope,
+                                                         const float* __restrict__ key_rope,
+                                                         const float* __restrict__ value, _Float16* __restrict__ k16,
+                                                         _Float16* __restrict__ v16, int64_t cap, int64_t keys,
+                                                         int64_t kp) {
+    __shared__ float tile[kTile * (kVh + 1)];  // keys: [64 channels][65]; values: [64 keys][129]
+    const int tid = threadIdx.x;
+    const int64_t j0 = static_cast<int64_t>(blockIdx.x) * kTile;
+    const int h = blockIdx.y;
+    for (int p = 0; p < kQk / 64; ++p) {  // 64 channels at a time
+        float v[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int ch = p * 64 + i * 4 + (tid >> 6);
+            const int64_t j = std::min<int64_t>(j0 + (tid & 63), keys - 1);
+            v[i] = ch < kNope ? key_nope[(static_cast<int64_t>(h) * kNope + ch) * cap + j]
+                              : key_rope[static_cast<int64_t>(ch - kNope) * cap + j];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            tile[(i * 4 + (tid >> 6)) * 65 + (tid & 63)] = v[i];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int kk = (tid >> 3) + 32 * i, part = tid & 7;
+            half8 out;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                out[e] = j0 + kk < keys ? static_cast<_Float16>(tile[(part * 8 + e) * 65 + kk])
+                                        : static_cast<_Float16>(0.0f);
+            }
+            *reinterpret_cast<half8*>(k16 + (static_cast<int64_t>(h) * kp + j0 + kk) * kQk + p * 64 + part * 8) = out;
+        }
+    }
+    f32x4 v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int64_t j = std::min<int64_t>(j0 + i * 8 + (tid >> 5), keys - 1);
+        v[i] = *reinterpret_cast<const f32x4*>(value + (static_cast<int64_t>(h) * cap + j) * kVh + (tid & 31) * 4);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            tile[(i * 8 + (tid >> 5)) * (kVh + 1) + (tid & 31) * 4 + e] = v[i][e];
+        }
+    }
+    __syncthreads();
+    _Float16* const dst = v16 + (static_cast<int64_t>(h) * kp + j0) * kVh;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int c = (tid >> 3) + 32 * i, part = tid & 7;  // positions 8 part .. + 7 of channel c
+        half8 out;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int pos = (part & 1) * 8 + e;  // within the group of 16
+            const int k = part / 2 * 16 + (pos & 3) + (pos & 4) * 2 + (pos & 8) / 2;
+            out[e] = j0 + k < keys ? static_cast<_Float16>(tile[k * (kVh + 1) + c]) : static_cast<_Float16>(0.0f);
+        }
+        *reinterpret_cast<half8*>(dst + c * kTile + part * 8) = out;
+    }
+}
+
+struct FlashArgs {
+    const float* q;        // [T][heads][192], rotary applied
+    const _Float16* k16;
+    const _Float16* v16;
+    _Float16* ctx16;       // panels [ctx_rows][heads 128] (one split)
+    float* part_o;         // [splits][heads][T][128] unnormalised contexts (several splits)
+    float* part_ml;        // [splits][heads][T][2] maximum and total
+    int64_t T, n0, kp;
+    int64_t row0, ctx_rows;
+    int32_t heads, qblocks, splits, split_tiles;
+    float c;               // softmax scale times log2(e)
+};
+
+template <int NW, bool SPLIT>
+__global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_kernel(const FlashArgs a) {
+    __shared__ __align__(16) char k0[kKeyBytes], k1[kKeyBytes], v0[kValueBytes], v1[kValueBytes];
+    char* const kring[2] = {k0, k1};
+    char* const vring[2] = {v0, v1};
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    // Workgroup -> (head, query block, split).  Heads are dealt to the XCDs
+    // (workgroup ids go round robin over them), so a head's tiles come into
+    // one L2; the blocks with the most keys go first, and a launch that fits
+    // the chip at two workgroups per CU pairs them with the lightest.
+    const int xcd = static_cast<int>(blockIdx.x) & 7;
+    int local = static_cast<int>(blockIdx.x) >> 3;
+    const int hpx = (a.heads + 7) / 8;
+    const int h = xcd + 8 * (local % hpx);
+    local /= hpx;
+    const int split = SPLIT ? local % a.splits : 0;
+    const int order = SPLIT ? local / a.splits : local;
+    if (h >= a.heads) {
+        return;
+    }
+    const int heavy = (a.qblocks + 1) / 2;
+    const int qb = order < heavy ? a.qblocks - 1 - order : order - heavy;
+    const int64_t q0 = static_cast<int64_t>(qb) * (32 * NW);
+    const int half = lane >> 5;
+    const int64_t qw = q0 + 32 * wave;                              // the wave's first query
+    const int64_t qi = qw + (lane & 31);                            // this lane's query
+    const int64_t qc = std::min<int64_t>(qi, a.T - 1);
+    const int64_t vis = a.n0 + qc;                                  // last key it sees
+    const int64_t block_keys = a.n0 + std::min<int64_t>(a.T, q0 + 32 * NW);
+    const int all_tiles = static_cast<int>((block_keys + kTile - 1) / kTile);
+    const int tile0 = SPLIT ? split * a.split_tiles : 0;
+    const int tile_end = SPLIT ? std::min(all_tiles, tile0 + a.split_tiles) : all_tiles;
+    // tiles this wave has a visible key in; none for waves past the last query
+    const int wave_end = qw < a.T ? static_cast<int>((a.n0 + std::min<int64_t>(a.T, qw + 32) + kTile - 1) / kTile) : 0;
+    // queries: B operand of S^T, k-step ks holds channels 16 ks + 8 half .. + 7
+    half8 qf[kQk / 16];
+    {
+        const float* qr = a.q + (qc * a.heads + h) * kQk + 8 * half;
+#pragma unroll
+        for (int ks = 0; ks < kQk / 16; ++ks) {
+            const f32x4 lo = *reinterpret_cast<const f32x4*>(qr + 16 * ks);
+            const f32x4 hi = *reinterpret_cast<const f32x4*>(qr + 16 * ks + 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                qf[ks][e] = static_cast<_Float16>(lo[e]);
+                qf[ks][4 + e] = static_cast<_Float16>(hi[e]);
+            }
+        }
+    }
+    // Tile loads: load j of the keys fills 16-byte positions 64 j + lane; a key
+    // row has 24 positions, position p of row r holds unit p ^ (r % 8) (three
+    // loads are 8 rows); a value row (channel) 8, likewise.
+    const int64_t head_keys = static_cast<int64_t>(h) * a.kp;
+    const __amdgpu_buffer_rsrc_t kres = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(a.k16 + head_keys * kQk), 0, static_cast<int>(a.kp * kQk * 2), kBufferWord3);
+    const __amdgpu_buffer_rsrc_t vres = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(a.v16 + head_keys * kVh), 0, static_cast<int>(a.kp * kVh * 2), kBufferWord3);
+    unsigned ksrc[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        const int p = 64 * j + lane;
+        const int r = p / 24, u = p % 24;
+        ksrc[j] = static_cast<unsigned>(r * (kQk * 2) + (u ^ (r & 7)) * 16);
+    }
+    const unsigned vsrc = static_cast<unsigned>((lane >> 3) * (kTile * 2) + ((lane & 7) ^ (lane >> 3)) * 16);
+    auto issue = [&](int tile, char* ks, char* vs) {
+#pragma unroll
+        for (int j = 0; j < kKeyLoads / NW; ++j) {
+            const int at = wave * (kKeyLoads / NW) + j;  // a multiple of three, plus j
+            load_lds16(kres, ks + at * 1024, ksrc[j % 3], tile * kKeyBytes + at / 3 * (8 * kQk * 2));
+        }
+#pragma unroll
+        for (int j = 0; j < kValueLoads / NW; ++j) {
+            const int at = wave * (kValueLoads / NW) + j;
+            load_lds16(vres, vs + at * 1024, vsrc, tile * kValueBytes + at * 1024);
+        }
+    };
+    f32x16 o[kVh / 32] = {};
+    float m = -__builtin_inff();  // running maximum of the raw scores
+    float l = 0.0f;               // this half wave's share of the total
+    auto compute = [&](int tile, const char* ks, const char* vs) {
+        f32x16 s[2] = {};
+        const int r = lane & 31;
+        // Fragments in sets of four (keys: two k-steps of both 32-key halves;
+        // values: one k-step of all channels), each read before the MFMAs of
+        // the set before it.  Rows r + 32 i have r % 8 in common.
+        half8 fa[4], fb[4];
+        auto read_keys = [&](int g, half8 (&f)[4]) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                f[i] = *reinterpret_cast<const half8*>(ks + (32 * (i & 1) + r) * (kQk * 2) +
+                                                       (((4 * g + 2 * (i >> 1)) + half) ^ (r & 7)) * 16);
+            }
+        };
+        auto read_values = [&](int st, half8 (&f)[4]) {
+#pragma unroll
+            for (int vt = 0; vt < 4; ++vt) {
+                f[vt] = *reinterpret_cast<const half8*>(vs + (32 * vt + r) * (kTile * 2) +
+                                                        ((2 * st + half) ^ (r & 7)) * 16);
+            }
+        };
+        auto score = [&](int g, const half8 (&f)[4]) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                s[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[i], qf[2 * g + (i >> 1)], s[i & 1], 0, 0, 0);
+            }
+        };
+        read_keys(0, fa);
+#pragma unroll
+        for (int g = 0; g < kQk / 32; g += 2) {
+            read_keys(g + 1, fb);
+            __builtin_amdgcn_sched_barrier(0);
+            score(g, fa);
+            __builtin_amdgcn_sched_barrier(0);
+            if (g + 2 < kQk / 32) {
+                read_keys(g + 2, fa);
+            } else {
+                read_values(0, fa);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            score(g + 1, fb);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // register e of s[kt] is key 64 tile + 32 kt + 8 (e / 4) + 4 half + e % 4
+        if (static_cast<int64_t>(tile + 1) * kTile > a.n0 + qw + 1) {
+            const int last = static_cast<int>(vis - static_cast<int64_t>(tile) * kTile);
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    if (32 * kt + 8 * (e / 4) + 4 * half + e % 4 > last) {
+                        s[kt][e] = -__builtin_inff();
+                    }
+                }
+            }
+        }
+        float t = fmaxf(s[0][0], s[1][0]);
+#pragma unroll
+        for (int e = 1; e < 16; ++e) {
+            t = fmaxf(t, fmaxf(s[0][e], s[1][e]));
+        }
+        t = fmaxf(t, __shfl_xor(t, 32));
+        const float m_new = fmaxf(m, t);
+        if (__any(m_new > m)) {
+            // no key seen yet: any finite reference, every exponential is 0
+            const float alpha = m_new == -__builtin_inff() ? 1.0f : __builtin_amdgcn_exp2f((m - m_new) * a.c);
+            l *= alpha;
+#pragma unroll
+            for (int vt = 0; vt < kVh / 32; ++vt) {
+                o[vt] *= alpha;
+            }
+            m = m_new;
+        }
+        const float mc = m == -__builtin_inff() ? 0.0f : m * a.c;
+        // ctx^T += V^T P^T: k-step st covers the 16 keys of registers 8 st .. + 7
+        half8 pf;
+        auto weights = [&](int st) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[st / 2][8 * (st & 1) + e], a.c, -mc));
+                l += p;
+                pf[e] = static_cast<_Float16>(p);
+            }
+        };
+        auto context = [&](const half8 (&f)[4]) {
+#pragma unroll
+            for (int vt = 0; vt < 4; ++vt) {
+                o[vt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[vt], pf, o[vt], 0, 0, 0);
+            }
+        };
+#pragma unroll
+        for (int st = 0; st < 4; st += 2) {
+            read_values(st + 1, fb);
+            weights(st);
+            context(fa);
+            if (st + 2 < 4) {
+                read_values(st + 2, fa);
+            }
+            weights(st + 1);
+            context(fb);
+        }
+    };
+    if (tile0 < tile_end) {
+        issue(tile0, k0, v0);
+    }
+    for (int tb = tile0; tb < tile_end; tb += 2) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int tile = tb + u;
+            if (tile < tile_end) {
+                // the tile is in, and every wave is done with the one before it
+                __builtin_amdgcn_sched_barrier(0);
+                __builtin_amdgcn_s_waitcnt(0x0070 | 0x0F00);  // vmcnt(0)
+                __builtin_amdgcn_s_barrier();
+                __builtin_amdgcn_sched_barrier(0);
+                if (tile + 1 < tile_end) {
+                    issue(tile + 1, kring[1 - u], vring[1 - u]);
+                }
+                if (tile < wave_end) {
+                    compute(tile, kring[u], vring[u]);
+                }
+            }
+        }
+    }
+    l += __shfl_xor(l, 32);
+    if (qi >= a.T) {
+        return;
+    }
+    // o[vt] register e: channel 32 vt + 8 (e / 4) + 4 half + e % 4 of query lane % 32
+    if constexpr (SPLIT) {
+        const int64_t at = (static_cast<int64_t>(split) * a.heads + h) * a.T + qi;
+        if (half == 0) {
+            a.part_ml[2 * at] = m;
+            a.part_ml[2 * at + 1] = l;
+        }
+#pragma unroll
+        for (int vt = 0; vt < kVh / 32; ++vt) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                f32x4 out;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    out[e] = o[vt][4 * g + e];
+                }
+                *reinterpret_cast<f32x4*>(a.part_o + at * kVh + 32 * vt + 8 * g + 4 * half) = out;
+            }
+        }
+    } else {
+        const float inv = 1.0f / l;
+#pragma unroll
+        for (int vt = 0; vt < kVh / 32; ++vt) {
+            _Float16* row = a.ctx16 + panel_index(a.row0 + qi, h * kVh + 32 * vt, a.ctx_rows) + 4 * half;
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                half4 out;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    out[e] = static_cast<_Float16>(o[vt][4 * g + e] * inv);
+                }
+                *reinterpret_cast<half4*>(row + 8 * g) = out;
+            }
+        }
+    }
+}
+
+// The splits' contexts of one (token, head) joined: weights exp(scale (m_i -
+// max)), over the weighted total.  32 lanes per (token, head), four channels
+// each.
+__global__ __launch_bounds__(256) void flash_combine_kernel(const FlashArgs a) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * 8 + (threadIdx.x >> 5);
+    const int lane = threadIdx.x & 31;
+    if (i >= a.T * a.heads) {
+        return;
+    }
+    const int64_t t = i / a.heads;
+    const int h = static_cast<int>(i - t * a.heads);
+    const int64_t step = a.heads * a.T;
+    const int64_t at = h * a.T + t;
+    float m = -__builtin_inff();
+    for (int k = 0; k < a.splits; ++k) {
+        m = fmaxf(m, a.part_ml[2 * (at + k * step)]);
+    }
+    f32x4 o = {};
+    float l = 0.0f;
+    for (int k = 0; k < a.splits; ++k) {
+        const float w = __builtin_amdgcn_exp2f((a.part_ml[2 * (at + k * step)] - m) * a.c);
+        l = __builtin_fmaf(w, a.part_ml[2 * (at + k * step) + 1], l);
+        const f32x4 p = *reinterpret_cast<const f32x4*>(a.part_o + (at + k * step) * kVh + 4 * lane);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            o[e] = __builtin_fmaf(w, p[e], o[e]);
+        }
+    }
+    const float inv = 1.0f / l;
+    half4 out;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        out[e] = static_cast<_Float16>(o[e] * inv);
+    }
+    *reinterpret_cast<half4*>(a.ctx16 + panel_index(a.row0 + t, h * kVh + 4 * lane, a.ctx_rows)) = out;
+}
+
+template <int NW>
+hipError_t launch_flash_nw(const FlashArgs& a, hipStream_t s) {
+    const int64_t grid = (a.heads + 7) / 8 * 8 * static_cast<int64_t>(a.qblocks) * a.splits;
+    if (grid > INT32_MAX) {
+        return hipErrorInvalidValue;
+    }
+    if (a.splits > 1) {
+        hipLaunchKernelGGL((flash_kernel<NW, true>), dim3(static_cast<unsigned>(grid)), dim3(64 * NW), 0, s, a);
+    } else {
+        hipLaunchKernelGGL((flash_kernel<NW, false>), dim3(static_cast<unsigned>(grid)), dim3(64 * NW), 0, s, a);
+    }
+    return hipGetLastError();
+}
+
+}  // namespace
+
+bool flash_supported(const AttnShape& a) { return a.nope == kNope && a.rope == kRope && a.vh == kVh; }
+
+int64_t flash_keys(int64_t keys) { return round_up(keys, kTile); }
+
+FlashPlan flash_plan(int32_t heads, int64_t tokens, int64_t keys) {
+    FlashPlan p;
+    p.waves = tokens >= 1024 ? 4 : tokens > 32 ? 2 : 1;
+    const int64_t tiles = (keys + kTile - 1) / kTile;
+    const int64_t blocks = heads * ((tokens + 32 * p.waves - 1) / (32 * p.waves));
+    const int64_t want = std::min<int64_t>({16, (256 + blocks - 1) / blocks, tiles / 4});
+    p.split_tiles = want > 1 ? static_cast<int32_t>((tiles + want - 1) / want) : 0;
+    p.splits = p.split_tiles > 0 ? static_cast<int32_t>((tiles + p.split_tiles - 1) / p.split_tiles) : 1;
+    return p;
+}
+
+int64_t flash_partial_floats(const FlashPlan& p, int32_t heads, int64_t tokens) {
+    return p.splits > 1 ? p.splits * heads * tokens * (kVh + 2) : 0;
+}
+
+hipError_t launch_flash_pack(const AttnShape& a, const KvCacheDev& c, int64_t keys, _Float16* k16, _Float16* v16,
+                             hipStream_t s) {
+    if (keys <= 0) {
+        return hipSuccess;
+    }
+    const int64_t kp = flash_keys(keys);
+    hipLaunchKernelGGL(flash_pack_kernel, dim3(static_cast<unsigned>(kp / kTile), a.heads), dim3(256), 0, s,
+                       c.key_nope, c.key_rope, c.value, k16, v16, a.cap, keys, kp);
+    return hipGetLastError();
+}
+
+hipError_t launch_flash(const AttnShape& a, const FlashPlan& p, const float* q, const _Float16* k16,
+                        const _Float16* v16, float* partial, int64_t T, int64_t n0, int64_t keys, float scale,
+                        _Float16* ctx16, int64_t row0, int64_t ctx_rows, hipStream_t s) {
+    if (T <= 0) {
+        return hipSuccess;
+    }
+    if (!flash_supported(a) || n0 + T > keys || row0 + T > ctx_rows) {
+        return hipErrorInvalidValue;
+    }
+    FlashArgs f;
+    f.q = q;
+    f.k16 = k16;
+    f.v16 = v16;
+    f.ctx16 = ctx16;
+    f.part_o = partial;
+    f.part_ml = partial != nullptr ? partial + p.splits * a.heads * T * kVh : nullptr;
+    f.T = T;
+    f.n0 = n0;
+    f.kp = flash_keys(keys);
+    f.row0 = row0;
+    f.ctx_rows = ctx_rows;
+    f.heads = a.heads;
+    f.qblocks = static_cast<int32_t>((T + 32 * p.waves - 1) / (32 * p.waves));
+    f.splits = p.splits;
+    f.split_tiles = p.split_tiles;
+    f.c = scale * 1.4426950408889634f;
+    hipError_t err = p.waves == 4 ? launch_flash_nw<4>(f, s) : p.waves == 2 ? launch_flash_nw<2>(f, s)
+                                                                           : launch_flash_nw<1>(f, s);
+    if (err != hipSuccess || p.splits == 1) {
+        return err;
+    }
+    hipLaunchKernelGGL(flash_combine_kernel, dim3(static_cast<unsigned>((T * a.heads + 7) / 8)), dim3(256), 0, s, f);
+    return hipGetLastError();
+}
+
+}  // namespace lm

@@ -364,13 +364,19 @@ int attention_tokens(AttnState* st, hipStream_t stream, int32_t layer, const flo
         return at;
     };
     auto halves = [](int64_t n) { return (n + 1) / 2; };
-    const int64_t kp = plan.kp;
+    // the MFMA core in one launch where the shape has it: no scores in memory
+    const bool flash = plan.mfma && lm::flash_supported(a);
+    const bool gemm_core = plan.mfma && !flash;
+    const lm::FlashPlan fp = flash ? lm::flash_plan(a.heads, F, n_total) : lm::FlashPlan{};
+    const int64_t kp = flash ? lm::flash_keys(n_total) : plan.kp;
     const size_t q_at = region(F * heads * qk);
     const size_t ql_at = region(F * ql);
     const size_t lat_at = region(F * (rank + rope));
     const size_t kvn_at = region(F * rank);
     const size_t kvx_at = region(F * heads * (c.qk_nope_head_dim + vh));
-    const size_t s_at = region(plan.mfma ? core * heads * kp : core * heads * n_total);
+    const size_t s_at = region(flash       ? lm::flash_partial_floats(fp, a.heads, core)
+                               : plan.mfma ? core * heads * kp
+                                           : core * heads * n_total);
     const size_t ctx_at = region(F * heads * vh);
     const size_t x16a_at = region(mfma ? halves(F * lm::round_up(H, lm::kPanel)) : 0);
     const size_t x16q_at = region(mfma && ql > 0 ? halves(F * lm::round_up(ql, lm::kPanel)) : 0);
@@ -381,9 +387,9 @@ int attention_tokens(AttnState* st, hipStream_t stream, int32_t layer, const flo
     const size_t partkv_at = region(partkv_f);
     const size_t k16_at = region(plan.mfma ? halves(heads * kp * qk) : 0);
     const size_t v16_at = region(plan.mfma ? halves(heads * vh * kp) : 0);
-    const size_t q16_at = region(plan.mfma ? halves(heads * core * qk) : 0);
-    const size_t p16_at = region(plan.mfma ? halves(heads * core * kp) : 0);
-    const size_t meta_at = region(plan.mfma ? (lm::mfma_heads_meta_bytes(heads) + 3) / 4 : 0);
+    const size_t q16_at = region(gemm_core ? halves(heads * core * qk) : 0);
+    const size_t p16_at = region(gemm_core ? halves(heads * core * kp) : 0);
+    const size_t meta_at = region(gemm_core ? (lm::mfma_heads_meta_bytes(heads) + 3) / 4 : 0);
     int rc = ensure_buffer(&st->ws, &st->ws_floats, stream, total_f);
     if (rc != LM_OK) {
         return rc;
@@ -473,7 +479,18 @@ int attention_tokens(AttnState* st, hipStream_t stream, int32_t layer, const flo
         LM_ATT_HIP(hipStreamWaitEvent(stream, st->join, 0));
     }
     // causal attention over the cache (:77-98), in groups of query tokens
-    if (plan.mfma) {
+    if (flash) {
+        // the context lands in fp16 panels in x16kv as below; a group's
+        // partial contexts (when the keys are split) keep to the budget
+        LM_ATT_HIP(lm::launch_flash_pack(a, L.cache, n_total, h16(k16_at), h16(v16_at), stream));
+        const int64_t step = fp.splits > 1 ? core : F;
+        for (int64_t t0 = 0; t0 < F; t0 += step) {
+            LM_ATT_HIP(lm::launch_flash(a, fp, q + t0 * heads * qk, h16(k16_at), h16(v16_at), S,
+                                        std::min(step, F - t0), n0 + t0, n_total, st->scale, x16kv, t0, F, stream));
+        }
+        pskv.ready = x16kv;
+        pskv.ready_of = ctxv;
+    } else if (plan.mfma) {
         // the context lands in fp16 panels [F, heads vh] in x16kv (free once
         // kv_b has run), the output projection's input; ctxv holds the
         // per-head context of one group

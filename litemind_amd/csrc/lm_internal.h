@@ -542,6 +542,26 @@ hipError_t launch_attention_core_mfma(const AttnShape& a, const float* q, const 
                                       int64_t n0, int64_t keys, float scale, _Float16* ctx16, int64_t row0,
                                       int64_t ctx_rows, hipStream_t s);
 
+// The same core in one launch, scores and probabilities in registers, for
+// heads of 128 + 64 key and 128 value channels (k_flash.hip).
+bool flash_supported(const AttnShape& a);
+// Keys that the fp16 copies k16 [heads][.][192] and v16 [heads][.][128] hold.
+int64_t flash_keys(int64_t keys);
+struct FlashPlan {
+    int32_t waves = 4;        // 32-token waves per workgroup
+    int32_t splits = 1;       // workgroups that share a query block's keys
+    int32_t split_tiles = 0;  // 64-key tiles of each (several splits)
+};
+FlashPlan flash_plan(int32_t heads, int64_t tokens, int64_t keys);
+// Floats of `partial` for `tokens` query tokens (0 with one split).
+int64_t flash_partial_floats(const FlashPlan& p, int32_t heads, int64_t tokens);
+hipError_t launch_flash_pack(const AttnShape& a, const KvCacheDev& c, int64_t keys, _Float16* k16, _Float16* v16,
+                             hipStream_t s);
+// As launch_attention_core_mfma, for T query tokens at slots n0 .. n0 + T - 1.
+hipError_t launch_flash(const AttnShape& a, const FlashPlan& p, const float* q, const _Float16* k16,
+                        const _Float16* v16, float* partial, int64_t T, int64_t n0, int64_t keys, float scale,
+                        _Float16* ctx16, int64_t row0, int64_t ctx_rows, hipStream_t s);
+
 // ---- services of the context (lm_capi.hip) to the attention translation unit ----
 struct AttnState;
 struct ContextInfo {

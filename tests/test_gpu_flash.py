@@ -1,0 +1,109 @@
+"""The one-launch attention core (flash_kernel) at DeepSeek-V2-Lite's head widths,
+through lm_attention_forward on the MFMA path, against float64 attention over
+the same cache: a wave owns 32 query tokens, a tile 64 keys, and few query
+tokens over many keys split the keys over several workgroups.
+
+The reference is fed the cache entries that the call itself wrote (read back),
+so only the core and the query / output projections differ: fp16 operands
+(2^-11 relative each) through a 2048-term product, a softmax over scores of a
+few units and a second product, then the output projection; their independent
+errors stay near 1e-3 of the output's scale, and the bounds are the path's own
+(mean relative 5e-3, maximum 5e-2 at outputs of magnitude 1).
+"""
+import dataclasses
+
+import numpy as np
+import pytest
+
+from conftest import announce, layer_error
+from test_gpu_attention import ATT_MAX_ABS, ATT_MEAN_REL, Mla, tokens
+
+pytestmark = pytest.mark.gpu
+
+
+def _f32(bits):
+    return (np.asarray(bits).astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+
+
+def _reference(m, x, cached):
+    """float64 attention of x [T, H] at positions cached.. over the layer's cache."""
+    from litemind_amd import mla_softmax_scale, rope_tables
+    from litemind_amd import workload as wl
+    d, L, T = m.d, m.L, x.shape[0]
+    n = cached + T
+    kn, kr, v = (a.astype(np.float64) for a in m.ctx.kv_cache_read(0, n))
+    cfg = wl.mla_config(d)
+    cos, sin = (t[cached:n].astype(np.float64)[:, None] for t in rope_tables(cfg, n))
+    q = (x.astype(np.float64) @ _f32(L.q_proj).T).reshape(T, d.heads, d.qk_head)
+    even, odd = q[..., d.qk_nope::2], q[..., d.qk_nope + 1::2]
+    rot = np.concatenate([even * cos - odd * sin, odd * cos + even * sin], axis=-1)
+    scale = float(mla_softmax_scale(cfg))
+    hidden = np.arange(n)[None] > np.arange(cached, n)[:, None]
+    ctx = np.empty((T, d.heads, d.v_head))
+    for h in range(d.heads):
+        s = scale * (q[:, h, :d.qk_nope] @ kn[:, h].T + rot[:, h] @ kr.T)
+        s[hidden] = -np.inf
+        p = np.exp(s - s.max(axis=1, keepdims=True))
+        ctx[:, h] = (p / p.sum(axis=1, keepdims=True)) @ v[:, h]
+    return ctx.reshape(T, -1) @ _f32(L.o_proj).T
+
+
+@pytest.mark.parametrize("heads,cached,T", [
+    (16, 0, 16),      # one wave per workgroup, half of it past the last token
+    (16, 5, 33),      # two waves, one token in the second
+    (16, 63, 65),     # the diagonal crosses tiles, a third wave block
+    (3, 0, 97),       # heads that are no multiple of the eight XCDs
+    (16, 2048, 16),   # keys split over workgroups
+    (16, 1500, 40),   # split, ragged last tile, queries masked in whole tiles
+    (5, 0, 1029),     # four waves, last block of five tokens
+    (16, 130, 1100),  # four waves after cached tokens
+])
+def test_flash_core(heads, cached, T):
+    from litemind_amd import PATH_MFMA
+    from litemind_amd import workload as wl
+    d = dataclasses.replace(wl.V2_LITE_MLA, heads=heads, max_positions=cached + T + 3)
+    announce(f"attention one-launch core heads={heads} cached={cached} T={T}")
+    m = Mla(d, 301 + heads, path=PATH_MFMA)
+    try:
+        rng = np.random.default_rng(T)
+        if cached:
+            m.ctx.kv_cache_write(0, 0, *(rng.standard_normal(s).astype(np.float32) for s in (
+                (cached, heads, d.qk_nope), (cached, d.qk_rope), (cached, heads, d.v_head))))
+        x = tokens(302, T, d.hidden)
+        y = m.forward(x, cached)
+        want = _reference(m, x, cached)
+        assert np.all(np.isfinite(y))
+        mx, rel = layer_error(y, want)
+        print(f"heads={heads} cached={cached} T={T}: max_abs={mx:.3e} mean_rel={rel:.3e}")
+        assert mx <= ATT_MAX_ABS and rel <= ATT_MEAN_REL
+        for t in (0, T - 1):  # no row is off while the mean is fine
+            assert np.abs(y[t] - want[t]).sum() <= 2 * ATT_MEAN_REL * np.abs(want[t]).sum()
+    finally:
+        m.close()
+
+
+def test_flash_core_groups_bit_identical():
+    """A score budget that holds part of the query tokens runs the split core in groups: the
+    same bits as in one launch (the splits depend on the whole call)."""
+    from litemind_amd import PATH_MFMA, attention_plan_core
+    from litemind_amd import workload as wl
+    cached, T = 1500, 130
+    d = dataclasses.replace(wl.V2_LITE_MLA, max_positions=cached + T)
+    rng = np.random.default_rng(9)
+    cache = [rng.standard_normal(s).astype(np.float32) for s in (
+        (cached, d.heads, d.qk_nope), (cached, d.qk_rope), (cached, d.heads, d.v_head))]
+    x = tokens(303, T, d.hidden)
+    budget = 33_600_000
+    plan = attention_plan_core(wl.mla_config(d), cached, T, PATH_MFMA, budget)
+    assert plan.mfma_core == 1 and 1 <= plan.query_group < T
+    announce("attention one-launch core, split keys, query groups against one group")
+    outs = []
+    for b in (budget, 0):
+        m = Mla(d, 304, path=PATH_MFMA)
+        try:
+            m.ctx.attention_set_score_budget(b)
+            m.ctx.kv_cache_write(0, 0, *cache)
+            outs.append(m.forward(x, cached))
+        finally:
+            m.close()
+    np.testing.assert_array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))

@@ -116,7 +116,10 @@ int lm_attention_set_path(lm_context* ctx, int32_t path);
  * runs on MFMA when qk_nope and qk_rope are multiples of 32, v_head_dim of 8
  * and heads * v_head_dim of 32: per head S = Q K^T and ctx = P V with fp16
  * operands over fp16 copies of the cache made once per call, P the causal
- * softmax in fp32 rounded to fp16; within the MFMA path's tolerance.
+ * softmax in fp32 rounded to fp16; within the MFMA path's tolerance.  Heads of
+ * 128 + 64 key and 128 value channels run it in one launch that keeps the
+ * scores in registers (every query token at once; in the plan's groups only
+ * where few query tokens share out the keys of a long cache).
  *
  * The core takes the call's query tokens in groups sized from a byte budget
  * for its scratch (no LiteMind counterpart): the fp32 scores, and for the MFMA

@@ -34,10 +34,9 @@ constexpr int kRope = 64;
 constexpr int kQk = kNope + kRope;
 constexpr int kVh = 128;
 constexpr int kTile = 64;                       // keys per tile
-constexpr int kKeyBytes = kTile * kQk * 2;      // 24 KB
+constexpr int kNopeBytes = kTile * kNope * 2;   // 16 KB
+constexpr int kRopeBytes = kTile * kRope * 2;   // 8 KB
 constexpr int kValueBytes = kTile * kVh * 2;    // 16 KB
-constexpr int kKeyLoads = kKeyBytes / 1024;     // wave loads of 1 KB
-constexpr int kValueLoads = kValueBytes / 1024;
 constexpr int kBufferWord3 = 0x00020000;        // buffer descriptor word 3, raw 32-bit access
 
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
@@ -51,30 +50,35 @@ __device__ inline void load_lds16(__amdgpu_buffer_rsrc_t from, char* to, unsigne
 }
 
 // ---- fp16 copies of the cache ----
-//   keys16    [heads][Kp][192]           row j = [key_nope(h, :, j) | key_rope(:, j)]
+//   nope16    [heads][Kp][128]           row j = key_nope(h, :, j)
+//   rope16    [Kp][64]                   row j = key_rope(:, j), shared by the heads
 //   values16  [heads][Kp / 64][128][64]  value(h, j, :) transposed per tile of 64
 //                                        keys, each 16 in the order 0-3, 8-11,
 //                                        4-7, 12-15: half wave h's scores are
 //                                        keys 4 h .. + 3 and 8 + 4 h .. + 3, its k
 //                                        indices 8 h .. + 7 of the second product
-// Kp = keys rounded up to 64, zeros past the last key.  Workgroup (tile, head).
+// Kp = the call's keys rounded up to 64.  New entries are written as they are
+// computed (k_proj.hip); flash_pack_kernel copies the `keys` older ones, zeros
+// up to the end of their last tile.  Workgroup (tile, head), the head past the
+// last for rope16.
 __global__ __launch_bounds__(256) void flash_pack_kernel(const float* __restrict__ key_nope,
                                                          const float* __restrict__ key_rope,
-                                                         const float* __restrict__ value, _Float16* __restrict__ k16,
-                                                         _Float16* __restrict__ v16, int64_t cap, int64_t keys,
-                                                         int64_t kp) {
+                                                         const float* __restrict__ value, const FlashKv kv,
+                                                         int32_t heads, int64_t cap, int64_t keys) {
     __shared__ float tile[kTile * (kVh + 1)];  // keys: [64 channels][65]; values: [64 keys][129]
     const int tid = threadIdx.x;
     const int64_t j0 = static_cast<int64_t>(blockIdx.x) * kTile;
     const int h = blockIdx.y;
-    for (int p = 0; p < kQk / 64; ++p) {  // 64 channels at a time
+    const bool rope = h == heads;
+    const int width = rope ? kRope : kNope;
+    const float* const src = rope ? key_rope : key_nope + static_cast<int64_t>(h) * kNope * cap;
+    _Float16* const rows = rope ? kv.rope16 + j0 * kRope : kv.nope16 + (static_cast<int64_t>(h) * kv.kp + j0) * kNope;
+    for (int p = 0; p < width / 64; ++p) {  // 64 channels at a time
         float v[16];
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            const int ch = p * 64 + i * 4 + (tid >> 6);
             const int64_t j = std::min<int64_t>(j0 + (tid & 63), keys - 1);
-            v[i] = ch < kNope ? key_nope[(static_cast<int64_t>(h) * kNope + ch) * cap + j]
-                              : key_rope[static_cast<int64_t>(ch - kNope) * cap + j];
+            v[i] = src[(p * 64 + i * 4 + (tid >> 6)) * cap + j];
         }
         __syncthreads();
 #pragma unroll
@@ -91,8 +95,11 @@ __global__ __launch_bounds__(256) void flash_pack_kernel(const float* __restrict
                 out[e] = j0 + kk < keys ? static_cast<_Float16>(tile[(part * 8 + e) * 65 + kk])
                                         : static_cast<_Float16>(0.0f);
             }
-            *reinterpret_cast<half8*>(k16 + (static_cast<int64_t>(h) * kp + j0 + kk) * kQk + p * 64 + part * 8) = out;
+            *reinterpret_cast<half8*>(rows + kk * width + p * 64 + part * 8) = out;
         }
+    }
+    if (rope) {
+        return;
     }
     f32x4 v[8];
 #pragma unroll
@@ -109,7 +116,7 @@ __global__ __launch_bounds__(256) void flash_pack_kernel(const float* __restrict
         }
     }
     __syncthreads();
-    _Float16* const dst = v16 + (static_cast<int64_t>(h) * kp + j0) * kVh;
+    _Float16* const dst = kv.v16 + (static_cast<int64_t>(h) * kv.kp + j0) * kVh;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int c = (tid >> 3) + 32 * i, part = tid & 7;  // positions 8 part .. + 7 of channel c
@@ -125,13 +132,12 @@ __global__ __launch_bounds__(256) void flash_pack_kernel(const float* __restrict
 }
 
 struct FlashArgs {
-    const float* q;        // [T][heads][192], rotary applied
-    const _Float16* k16;
-    const _Float16* v16;
+    const _Float16* q16;   // [T][heads][192], rotary applied
+    FlashKv kv;
     _Float16* ctx16;       // panels [ctx_rows][heads 128] (one split)
     float* part_o;         // [splits][heads][T][128] unnormalised contexts (several splits)
     float* part_ml;        // [splits][heads][T][2] maximum and total
-    int64_t T, n0, kp;
+    int64_t T, n0;
     int64_t row0, ctx_rows;
     int32_t heads, qblocks, splits, split_tiles;
     float c;               // softmax scale times log2(e)
@@ -139,8 +145,10 @@ struct FlashArgs {
 
 template <int NW, bool SPLIT>
 __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_kernel(const FlashArgs a) {
-    __shared__ __align__(16) char k0[kKeyBytes], k1[kKeyBytes], v0[kValueBytes], v1[kValueBytes];
+    __shared__ __align__(16) char k0[kNopeBytes], k1[kNopeBytes], r0[kRopeBytes], r1[kRopeBytes], v0[kValueBytes],
+        v1[kValueBytes];
     char* const kring[2] = {k0, k1};
+    char* const rring[2] = {r0, r1};
     char* const vring[2] = {v0, v1};
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
@@ -175,50 +183,50 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_kernel(const F
     // queries: B operand of S^T, k-step ks holds channels 16 ks + 8 half .. + 7
     half8 qf[kQk / 16];
     {
-        const float* qr = a.q + (qc * a.heads + h) * kQk + 8 * half;
+        const _Float16* qr = a.q16 + (qc * a.heads + h) * kQk + 8 * half;
 #pragma unroll
         for (int ks = 0; ks < kQk / 16; ++ks) {
-            const f32x4 lo = *reinterpret_cast<const f32x4*>(qr + 16 * ks);
-            const f32x4 hi = *reinterpret_cast<const f32x4*>(qr + 16 * ks + 4);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                qf[ks][e] = static_cast<_Float16>(lo[e]);
-                qf[ks][4 + e] = static_cast<_Float16>(hi[e]);
-            }
+            qf[ks] = *reinterpret_cast<const half8*>(qr + 16 * ks);
         }
     }
-    // Tile loads: load j of the keys fills 16-byte positions 64 j + lane; a key
-    // row has 24 positions, position p of row r holds unit p ^ (r % 8) (three
-    // loads are 8 rows); a value row (channel) 8, likewise.
-    const int64_t head_keys = static_cast<int64_t>(h) * a.kp;
+    // Tile loads: a load fills 64 consecutive 16-byte positions; position p of
+    // row r holds unit p ^ (r % 8).  Rows of the nope keys have 16 positions
+    // (four rows a load), of the rotary keys and the values eight.
+    const int64_t head_keys = static_cast<int64_t>(h) * a.kv.kp;
     const __amdgpu_buffer_rsrc_t kres = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(a.k16 + head_keys * kQk), 0, static_cast<int>(a.kp * kQk * 2), kBufferWord3);
+        (void*)(a.kv.nope16 + head_keys * kNope), 0, static_cast<int>(a.kv.kp * kNope * 2), kBufferWord3);
+    const __amdgpu_buffer_rsrc_t rres = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)a.kv.rope16, 0, static_cast<int>(a.kv.kp * kRope * 2), kBufferWord3);
     const __amdgpu_buffer_rsrc_t vres = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(a.v16 + head_keys * kVh), 0, static_cast<int>(a.kp * kVh * 2), kBufferWord3);
-    unsigned ksrc[3];
+        (void*)(a.kv.v16 + head_keys * kVh), 0, static_cast<int>(a.kv.kp * kVh * 2), kBufferWord3);
+    unsigned ksrc[2];  // rows 0..3 and 4..7 of eight
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
-        const int p = 64 * j + lane;
-        const int r = p / 24, u = p % 24;
-        ksrc[j] = static_cast<unsigned>(r * (kQk * 2) + (u ^ (r & 7)) * 16);
+    for (int j = 0; j < 2; ++j) {
+        const int r = 4 * j + (lane >> 4);
+        ksrc[j] = static_cast<unsigned>((lane >> 4) * (kNope * 2) + ((lane & 15) ^ r) * 16);
     }
-    const unsigned vsrc = static_cast<unsigned>((lane >> 3) * (kTile * 2) + ((lane & 7) ^ (lane >> 3)) * 16);
-    auto issue = [&](int tile, char* ks, char* vs) {
+    const unsigned vsrc = static_cast<unsigned>((lane >> 3) * 128 + ((lane & 7) ^ (lane >> 3)) * 16);
+    auto issue = [&](int tile, char* ks, char* rs, char* vs) {
 #pragma unroll
-        for (int j = 0; j < kKeyLoads / NW; ++j) {
-            const int at = wave * (kKeyLoads / NW) + j;  // a multiple of three, plus j
-            load_lds16(kres, ks + at * 1024, ksrc[j % 3], tile * kKeyBytes + at / 3 * (8 * kQk * 2));
+        for (int j = 0; j < 16 / NW; ++j) {
+            const int at = wave * (16 / NW) + j;  // a multiple of four, plus j
+            load_lds16(kres, ks + at * 1024, ksrc[j & 1], tile * kNopeBytes + at * 1024);
         }
 #pragma unroll
-        for (int j = 0; j < kValueLoads / NW; ++j) {
-            const int at = wave * (kValueLoads / NW) + j;
+        for (int j = 0; j < 8 / NW; ++j) {
+            const int at = wave * (8 / NW) + j;
+            load_lds16(rres, rs + at * 1024, vsrc, tile * kRopeBytes + at * 1024);
+        }
+#pragma unroll
+        for (int j = 0; j < 16 / NW; ++j) {
+            const int at = wave * (16 / NW) + j;
             load_lds16(vres, vs + at * 1024, vsrc, tile * kValueBytes + at * 1024);
         }
     };
     f32x16 o[kVh / 32] = {};
     float m = -__builtin_inff();  // running maximum of the raw scores
     float l = 0.0f;               // this half wave's share of the total
-    auto compute = [&](int tile, const char* ks, const char* vs) {
+    auto compute = [&](int tile, const char* ks, const char* rs, const char* vs) {
         f32x16 s[2] = {};
         const int r = lane & 31;
         // Fragments in sets of four (keys: two k-steps of both 32-key halves;
@@ -228,8 +236,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_kernel(const F
         auto read_keys = [&](int g, half8 (&f)[4]) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                f[i] = *reinterpret_cast<const half8*>(ks + (32 * (i & 1) + r) * (kQk * 2) +
-                                                       (((4 * g + 2 * (i >> 1)) + half) ^ (r & 7)) * 16);
+                const int row = 32 * (i & 1) + r, u = 4 * g + 2 * (i >> 1) + half;
+                f[i] = *reinterpret_cast<const half8*>(
+                    g < kNope / 32 ? ks + row * (kNope * 2) + (u ^ (r & 7)) * 16
+                                   : rs + row * (kRope * 2) + ((u - kNope / 8) ^ (r & 7)) * 16);
             }
         };
         auto read_values = [&](int st, half8 (&f)[4]) {
@@ -321,7 +331,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_kernel(const F
         }
     };
     if (tile0 < tile_end) {
-        issue(tile0, k0, v0);
+        issue(tile0, k0, r0, v0);
     }
     for (int tb = tile0; tb < tile_end; tb += 2) {
 #pragma unroll
@@ -334,10 +344,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_kernel(const F
                 __builtin_amdgcn_s_barrier();
                 __builtin_amdgcn_sched_barrier(0);
                 if (tile + 1 < tile_end) {
-                    issue(tile + 1, kring[1 - u], vring[1 - u]);
+                    issue(tile + 1, kring[1 - u], rring[1 - u], vring[1 - u]);
                 }
                 if (tile < wave_end) {
-                    compute(tile, kring[u], vring[u]);
+                    compute(tile, kring[u], rring[u], vring[u]);
                 }
             }
         }
@@ -455,36 +465,32 @@ int64_t flash_partial_floats(const FlashPlan& p, int32_t heads, int64_t tokens) 
     return p.splits > 1 ? p.splits * heads * tokens * (kVh + 2) : 0;
 }
 
-hipError_t launch_flash_pack(const AttnShape& a, const KvCacheDev& c, int64_t keys, _Float16* k16, _Float16* v16,
-                             hipStream_t s) {
+hipError_t launch_flash_pack(const AttnShape& a, const KvCacheDev& c, int64_t keys, const FlashKv& kv, hipStream_t s) {
     if (keys <= 0) {
         return hipSuccess;
     }
-    const int64_t kp = flash_keys(keys);
-    hipLaunchKernelGGL(flash_pack_kernel, dim3(static_cast<unsigned>(kp / kTile), a.heads), dim3(256), 0, s,
-                       c.key_nope, c.key_rope, c.value, k16, v16, a.cap, keys, kp);
+    hipLaunchKernelGGL(flash_pack_kernel, dim3(static_cast<unsigned>((keys + kTile - 1) / kTile), a.heads + 1),
+                       dim3(256), 0, s, c.key_nope, c.key_rope, c.value, kv, a.heads, a.cap, keys);
     return hipGetLastError();
 }
 
-hipError_t launch_flash(const AttnShape& a, const FlashPlan& p, const float* q, const _Float16* k16,
-                        const _Float16* v16, float* partial, int64_t T, int64_t n0, int64_t keys, float scale,
-                        _Float16* ctx16, int64_t row0, int64_t ctx_rows, hipStream_t s) {
+hipError_t launch_flash(const AttnShape& a, const FlashPlan& p, const _Float16* q16, const FlashKv& kv, float* partial,
+                        int64_t T, int64_t n0, float scale, _Float16* ctx16, int64_t row0, int64_t ctx_rows,
+                        hipStream_t s) {
     if (T <= 0) {
         return hipSuccess;
     }
-    if (!flash_supported(a) || n0 + T > keys || row0 + T > ctx_rows) {
+    if (!flash_supported(a) || n0 + T > kv.kp || row0 + T > ctx_rows) {
         return hipErrorInvalidValue;
     }
     FlashArgs f;
-    f.q = q;
-    f.k16 = k16;
-    f.v16 = v16;
+    f.q16 = q16;
+    f.kv = kv;
     f.ctx16 = ctx16;
     f.part_o = partial;
     f.part_ml = partial != nullptr ? partial + p.splits * a.heads * T * kVh : nullptr;
     f.T = T;
     f.n0 = n0;
-    f.kp = flash_keys(keys);
     f.row0 = row0;
     f.ctx_rows = ctx_rows;
     f.heads = a.heads;

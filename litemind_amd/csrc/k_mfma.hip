@@ -44,42 +44,14 @@
 // of 96 rows and more with the small groups in a separate 64-row launch
 // (343: the second launch's tail).
 #include "lm_internal.h"
+#include "mfma_tile.h"
 
 #include <algorithm>
 
 namespace lm {
 namespace {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef __attribute__((address_space(3))) void lds_void;
-
-constexpr int BN = 256;
-constexpr int BK = kPanel;                   // halves: 64-byte rows, 4 chunks of 16 B
-constexpr int kRowBytes = BK * 2;
-constexpr int kBBytes = BN * kRowBytes;      // 16 KB
-constexpr int kXcds = 8;
-constexpr int kBufferWord3 = 0x00020000;     // buffer descriptor word 3: raw 32-bit access
-
-template <int WM, int WN, int MI, int NJ, int STAGES>
-struct Shape {
-    static constexpr int WAVES = WM * WN;
-    static constexpr int kThreads = 64 * WAVES;
-    static constexpr int BM = 32 * WM * MI;
-    static constexpr int kABytes = BM * kRowBytes;
-    static constexpr int kStageBytes = kABytes + kBBytes;
-    static constexpr int AL = kABytes / 1024 / WAVES;  // A loads (1 KB wave instructions) per wave per stage
-    static constexpr int BL = kBBytes / 1024 / WAVES;
-    static constexpr int L = AL + BL;
-    static constexpr int NR = MI + NJ;                 // fragment reads per half step
-    static constexpr int NP = MI * NJ / 2;             // MFMA pairs per half step
-    static_assert(32 * WN * NJ == BN, "the waves cover the 256 columns");
-    static_assert(AL * 1024 * WAVES == kABytes && AL >= 1, "whole A instructions per wave");
-    static_assert(NJ % 2 == 0, "gate/up column blocks come in pairs");
-    static_assert(NR <= 2 * NP && L <= 4 * NP, "reads and loads spread over the MFMA pairs");
-    static_assert(STAGES >= 3 && STAGES <= 4 && (STAGES - 2) * L < 64, "pipeline depth, vmcnt");
-    static_assert(STAGES * kStageBytes <= 80 * 1024, "two workgroups per CU");
-};
+constexpr int BN = 256;  // weight rows per tile
 
 // Launches whose average routed group fits one 64-row tile (T k <= 64 E; a
 // dense layer: T <= 64) take the 64-row shape.  Measured on V2-Lite (one MoE block, 64 experts, k 6): 8-12%
@@ -241,114 +213,6 @@ __device__ inline float silu_fast(float g, float u) {
     return g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * u;
 }
 
-// Chunk permutation of row r (row bits 1..3 only).  A ds_read_b128 serves 16
-// lanes per cycle from 64 banks: lanes 0..15 read rows r0..r0+15 (r0 a
-// multiple of 16) at one logical chunk, and the rows that share a bank phase
-// (r mod 4) get four different chunk positions; the same holds for 8-lane
-// groups over 32 banks.
-__device__ inline int row_swizzle(int r) { return ((r >> 2) & 3) ^ (r & 2); }
-// LDS byte offset of the 16-byte chunk c of row r.
-__device__ inline int chunk_offset(int r, int c) { return r * kRowBytes + ((c ^ row_swizzle(r)) << 4); }
-
-// s_waitcnt with only vmcnt (expcnt and lgkmcnt at their maxima)
-#define LM_WAIT_VM(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | 0x0F70)
-
-// The per-wave state of a tile and the steps of its pipeline.  One type per
-// kernel instantiation (MODE is a parameter): hipcc's host pass left out the
-// launch stub of a second kernel whose body instantiated the same member
-// functions.
-template <int MODE, int WM, int WN, int MI, int NJ, int STAGES>
-struct Tile {
-    using Z = Shape<WM, WN, MI, NJ, STAGES>;
-    __amdgpu_buffer_rsrc_t ra, rb;  // operand A (token rows / activations), operand B (weight rows)
-    unsigned va[Z::AL], vb[Z::BL];  // this lane's byte offset of its row chunk in stage 0
-    unsigned a_step, b_step;        // bytes between consecutive K panels
-    int lane, wave, wm, wn;
-    int blocks;                     // this wave's 32-row blocks holding group rows (0..MI); the rest skip their MFMAs
-    half8 fa[2][MI], fb[2][NJ];     // fragments of the two half steps of a stage
-    floatx16 acc[MI][NJ];
-
-    // Load q of this wave's stage loads (A first, then B): 1 KB, 16 rows of 64
-    // bytes, into LDS by a buffer load (the stage offset is a scalar).
-    __device__ void load1(int ks, char* buf, int q) {
-        if (q < Z::AL) {
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_void*)(buf + (Z::WAVES * q + wave) * 1024), 16, va[q],
-                                                     static_cast<unsigned>(ks) * a_step, 0, 0);
-        } else {
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                rb, (lds_void*)(buf + Z::kABytes + (Z::WAVES * (q - Z::AL) + wave) * 1024), 16, vb[q - Z::AL],
-                static_cast<unsigned>(ks) * b_step, 0, 0);
-        }
-    }
-    // Fragment r of half step kk: A blocks 0..MI-1, then B blocks 0..NJ-1.
-    __device__ void read1(const char* buf, int kk, int r) {
-        const int c = 2 * kk + (lane >> 5);
-        if (r < MI) {
-            fa[kk][r] = *reinterpret_cast<const half8*>(buf + chunk_offset(wm * 32 * MI + 32 * r + (lane & 31), c));
-        } else {
-            fb[kk][r - MI] = *reinterpret_cast<const half8*>(
-                buf + Z::kABytes + chunk_offset(wn * 32 * NJ + 32 * (r - MI) + (lane & 31), c));
-        }
-    }
-    // MFMAs t and t + 1 of half step kk (one A block: NJ is even), skipped for
-    // a block past the group's rows (its accumulators are never stored).
-    __device__ void mma2(int t, int kk) {
-        const int i = t / NJ, j = t % NJ;
-        if (i < blocks) {
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[kk][i], fb[kk][j], acc[i][j], 0, 0, 0);
-            acc[i][j + 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[kk][i], fb[kk][j + 1], acc[i][j + 1], 0, 0, 0);
-        }
-    }
-    // s_waitcnt vmcnt(n L): n later stages of this wave's loads may stay in flight.
-    __device__ void wait_stages(int n) {
-        if (n >= 2) {
-            LM_WAIT_VM(2 * Z::L);
-        } else if (n == 1) {
-            LM_WAIT_VM(Z::L);
-        } else {
-            LM_WAIT_VM(0);
-        }
-    }
-    // Stage ks: wait for this wave's loads of it (`behind` later stages stay in
-    // flight), barrier (every wave's loads visible; the buffer of stage ks - 1,
-    // which the loads of stage ks + STAGES - 1 overwrite, read by every wave),
-    // the first half step's fragments, then its MFMAs with the second half
-    // step's fragment reads and the stage's loads between them, then the second
-    // half step's MFMAs with the remaining loads.  With one read or load
-    // between two MFMAs the wave's MFMA issue never waits for a run of memory
-    // instructions to be accepted (measured on a dense 4096^3 GEMM: 1,150 cycles
-    // per stage against 1,561 with the loads and reads issued in runs).
-    __device__ void stage(int ks, const char* cur, char* tgt, bool issue, int behind) {
-        wait_stages(behind);
-        __builtin_amdgcn_s_barrier();
-#pragma unroll
-        for (int r = 0; r < Z::NR; ++r) {
-            read1(cur, 0, r);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int p = 0; p < 2 * Z::NP; ++p) {
-            if (p < Z::NP) {
-#pragma unroll
-                for (int r = 2 * p; r < 2 * p + 2; ++r) {
-                    if (r < Z::NR) {
-                        read1(cur, 1, r);
-                    }
-                }
-            }
-#pragma unroll
-            for (int q = p * Z::L / (2 * Z::NP); q < (p + 1) * Z::L / (2 * Z::NP); ++q) {
-                if (issue) {
-                    load1(ks + STAGES - 1, tgt, q);
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            mma2(2 * (p % Z::NP), p / Z::NP);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    }
-};
-
 template <int MODE, int WM, int WN, int MI, int NJ, int STAGES>
 __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2, 2))) void mfma_grouped_kernel(
     ExpertArgs a) {
@@ -359,7 +223,7 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
     constexpr int kStage3 = STAGES > 3 ? Z::kStageBytes : 16;
     __shared__ __attribute__((aligned(1024))) char s0[Z::kStageBytes], s1[Z::kStageBytes], s2[Z::kStageBytes],
         s3[kStage3];
-    char* const bufs[4] = {s0, s1, s2, s3};
+    char* const bufs[6] = {s0, s1, s2, s3, s3, s3};
     Tile<MODE, WM, WN, MI, NJ, STAGES> t;
     t.lane = threadIdx.x & 63;
     t.wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
@@ -453,34 +317,7 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
             t.acc[i][j] = floatx16{};
         }
     }
-    // Stages 0 .. STAGES - 2 in flight before the first stage; stage ks lives in
-    // buffer ks % STAGES and the loads of stage ks + STAGES - 1 go to buffer
-    // (ks - 1) % STAGES.  A K shorter than STAGES - 1 stages reloads the last
-    // stage into buffers that are never read, so every path has the same loads
-    // in flight.
-#pragma unroll
-    for (int d = 0; d < STAGES - 1; ++d) {
-#pragma unroll
-        for (int q = 0; q < Z::L; ++q) {
-            t.load1(d < nk ? d : nk - 1, bufs[d], q);
-        }
-    }
-    int ks = 0;
-    for (; ks + 2 * STAGES - 1 <= nk; ks += STAGES) {
-#pragma unroll
-        for (int j = 0; j < STAGES; ++j) {
-            t.stage(ks + j, bufs[j], bufs[(j + STAGES - 1) % STAGES], true, STAGES - 2);
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < 2 * STAGES - 1; ++j) {
-        const int kj = ks + j;
-        if (kj < nk) {
-            const int later = nk - 1 - kj;
-            t.stage(kj, bufs[j % STAGES], bufs[(j + STAGES - 1) % STAGES], kj + STAGES - 1 < nk,
-                    later < STAGES - 2 ? later : STAGES - 2);
-        }
-    }
+    t.run(bufs, nk);
 
     // Epilogue.  Lane l holds column n = l % 32 of each 32 x 32 block, rows
     // m = 8 (r / 4) + 4 (l / 32) + r % 4 for registers r = 0..15.
@@ -516,7 +353,6 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
         }
     }
 }
-#undef LM_WAIT_VM
 
 // Upper bound of the workgroups the tile walk needs (the kernel maps
 // workgroups onto the tiles that exist and the rest return at once): per XCD

@@ -19,7 +19,10 @@
 // results within the tolerance of the MoE block's MFMA path.  With MFMA
 // projections the attention core is MFMA as well where the shape allows it
 // (k_attn.hip): per head S = Q K^T and ctx = P V on the same grouped kernel,
-// over fp16 copies of the cache made once per call.
+// over fp16 copies of the cache made once per call.  Heads of 128 + 64 key and
+// 128 value channels (DeepSeek-V2's) take attention_prompt instead: projections
+// with their next step as epilogue (k_proj.hip) around a one-launch core
+// (k_flash.hip).
 //
 // Query tokens are processed by the core in groups sized from a byte budget
 // (lm_attention_set_score_budget, default 1 GiB) for the scores (and the MFMA
@@ -31,6 +34,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <iterator>
 #include <new>
 #include <string>
 #include <vector>
@@ -60,6 +64,7 @@ struct AttnLayer {
     // of Proj, read by the kernel as its group's weights
     void* slab16 = nullptr;
     const _Float16* const* table16 = nullptr;
+    const _Float16* w16[6] = {};  // the same pointers on the host
     float* input_norm = nullptr;  // [H], lm_decoder_forward
     KvCacheDev cache;
     int64_t count = 0;  // KvCache::token_count
@@ -330,6 +335,116 @@ int project(const AttnLayer& L, int proj, const uint16_t* w, const float* x, int
     return LM_OK;
 }
 
+// attention_tokens for a batch on the MFMA path whose heads have the one-launch
+// core's widths: every projection's next step is its GEMM's epilogue
+// (k_proj.hip), so a call is six launches on one stream (eight with a q LoRA;
+// one more for older cache entries, one more when the core splits its keys):
+//   x -> fp16 | q and kv_a | norm, rotary key | kv_b into cache and copies |
+//   core | o_proj
+// Before, a 512-token V2-Lite prompt took 22 launches on two streams: 108 us
+// against 39, 4096 tokens 1196 us against 263.
+int attention_prompt(AttnState* st, hipStream_t stream, AttnLayer& L, const CorePlan& plan, const float* x, int64_t F,
+                     int64_t pos0, float* out, int32_t accumulate, const float* in_norm) {
+    const lm_mla_config& c = st->cfg;
+    const lm::AttnShape& a = st->shape;
+    const int64_t H = c.hidden_size, heads = c.num_heads, qk = c.qk_nope_head_dim + c.qk_rope_head_dim;
+    const int64_t rank = c.kv_lora_rank, rope = c.qk_rope_head_dim, vh = c.v_head_dim, ql = c.q_lora_rank;
+    const int64_t n0 = L.count;
+    const int64_t kp = lm::flash_keys(n0 + F);
+    const lm::FlashPlan fp = lm::flash_plan(a.heads, F, n0 + F);
+    // query tokens per core launch: all, or when the keys are split (each query
+    // token then has partial contexts) the group that the budget holds
+    const int64_t group = fp.splits > 1 ? plan.group : F;
+    size_t total_f = 0;
+    auto region = [&](int64_t floats) {
+        const size_t at = total_f;
+        total_f += static_cast<size_t>((floats + 63) / 64 * 64);
+        return at;
+    };
+    auto halves = [](int64_t n) { return (n + 1) / 2; };
+    const size_t x16_at = region(halves(F * H));
+    const size_t q16_at = region(halves(F * heads * qk));
+    const size_t ql_at = region(F * ql);
+    const size_t ql16_at = region(halves(F * ql));
+    const size_t lat_at = region(F * (rank + rope));
+    const size_t kvn16_at = region(halves(F * rank));
+    const size_t ctx16_at = region(halves(F * heads * vh));
+    const size_t nope16_at = region(halves(heads * kp * c.qk_nope_head_dim));
+    const size_t rope16_at = region(halves(kp * rope));
+    const size_t v16_at = region(halves(heads * kp * vh));
+    const size_t part_at = region(lm::flash_partial_floats(fp, a.heads, group));
+    const int rc = ensure_buffer(&st->ws, &st->ws_floats, stream, total_f);
+    if (rc != LM_OK) {
+        return rc;
+    }
+    float* const ws = st->ws;
+    auto h16 = [&](size_t at) { return reinterpret_cast<_Float16*>(ws + at); };
+    lm::ProjArgs p;
+    p.tokens = F;
+    p.heads = a.heads;
+    p.q16 = h16(q16_at);
+    p.cache = L.cache;
+    p.kv = lm::FlashKv{h16(nope16_at), h16(rope16_at), h16(v16_at), kp};
+    p.cap = a.cap;
+    p.slot0 = n0;
+    p.pos0 = pos0;
+    p.max_positions = a.max_positions;
+    p.cos_t = a.cos_t;
+    p.sin_t = a.sin_t;
+    auto segment = [&](int proj, int64_t rows, int kind, float* to, int32_t add) {
+        lm::ProjSegment seg;
+        seg.w = L.w16[proj];
+        seg.rows = static_cast<int32_t>(rows);
+        seg.kind = kind;
+        seg.out = to;
+        seg.accumulate = add;
+        return seg;
+    };
+    // older entries first: the copies of the call's own follow into the same tiles
+    LM_ATT_HIP(lm::launch_flash_pack(a, L.cache, n0, p.kv, stream));
+    if (in_norm != nullptr) {
+        LM_ATT_HIP(lm::launch_norm16(x, in_norm, h16(x16_at), F, static_cast<int32_t>(H), c.rms_norm_eps, stream));
+    } else {
+        LM_ATT_HIP(lm::launch_to_f16_rows(x, h16(x16_at), F, static_cast<int32_t>(H), static_cast<int32_t>(H),
+                                          stream));
+    }
+    // queries (src/Attention.cpp:33-48) and the compressed keys and values (:50-56)
+    p.x16 = h16(x16_at);
+    p.width = static_cast<int32_t>(H);
+    p.seg[0] = ql == 0 ? segment(lm::kProjQ, heads * qk, lm::kProjQuery, nullptr, 0)
+                       : segment(lm::kProjQa, ql, lm::kProjPlain, ws + ql_at, 0);
+    p.seg[1] = segment(lm::kProjKva, rank + rope, lm::kProjPlain, ws + lat_at, 0);
+    LM_ATT_HIP(lm::launch_proj(p, stream));
+    p.seg[1] = lm::ProjSegment{};
+    if (ql != 0) {
+        LM_ATT_HIP(lm::launch_norm16(ws + ql_at, L.q_a_norm, h16(ql16_at), F, static_cast<int32_t>(ql),
+                                     c.rms_norm_eps, stream));
+        p.x16 = h16(ql16_at);
+        p.width = static_cast<int32_t>(ql);
+        p.seg[0] = segment(lm::kProjQb, heads * qk, lm::kProjQuery, nullptr, 0);
+        LM_ATT_HIP(lm::launch_proj(p, stream));
+    }
+    // the new entries at slots n0 .. n0 + F - 1 (:57-75)
+    LM_ATT_HIP(lm::launch_kv_prep16(p, ws + lat_at, L.kv_a_norm, h16(kvn16_at), static_cast<int32_t>(rank),
+                                    c.rms_norm_eps, stream));
+    p.x16 = h16(kvn16_at);
+    p.width = static_cast<int32_t>(rank);
+    p.seg[0] = segment(lm::kProjKvb, heads * (c.qk_nope_head_dim + vh), lm::kProjKv, nullptr, 0);
+    LM_ATT_HIP(lm::launch_proj(p, stream));
+    // causal attention over the cache (:77-98)
+    for (int64_t t0 = 0; t0 < F; t0 += group) {
+        LM_ATT_HIP(lm::launch_flash(a, fp, p.q16 + t0 * heads * qk, p.kv, ws + part_at, std::min(group, F - t0),
+                                    n0 + t0, st->scale, h16(ctx16_at), t0, F, stream));
+    }
+    // output projection (:100-101)
+    p.x16 = h16(ctx16_at);
+    p.width = static_cast<int32_t>(heads * vh);
+    p.seg[0] = segment(lm::kProjO, H, lm::kProjPlain, out, accumulate);
+    LM_ATT_HIP(lm::launch_proj(p, stream));
+    L.count = n0 + F;
+    return LM_OK;
+}
+
 // Attention::forward for F tokens that all fit the cache; out = o_proj ctx or
 // out += o_proj ctx.  x [F, H] must not overlap out, except with in_norm: x is
 // then the raw hidden state, normalised here by in_norm (into xn_buf [F, H], or
@@ -350,6 +465,9 @@ int attention_tokens(AttnState* st, hipStream_t stream, int32_t layer, const flo
     const int64_t n_total = n0 + F;
     const bool mfma = L.table16 != nullptr && mfma_projections(path, F);
     const CorePlan plan = plan_core(a, n0, F, mfma, st->score_budget > 0 ? st->score_budget : kScoreBudget);
+    if (plan.mfma && lm::flash_supported(a)) {
+        return attention_prompt(st, stream, L, plan, x, F, pos0, out, accumulate, in_norm);
+    }
     const int64_t core = plan.group;
     // Scratch, each region a multiple of 64 floats: q | q latent | kv latent |
     // kv normalised | kv expanded | scores | context; with MFMA projections
@@ -364,19 +482,13 @@ int attention_tokens(AttnState* st, hipStream_t stream, int32_t layer, const flo
         return at;
     };
     auto halves = [](int64_t n) { return (n + 1) / 2; };
-    // the MFMA core in one launch where the shape has it: no scores in memory
-    const bool flash = plan.mfma && lm::flash_supported(a);
-    const bool gemm_core = plan.mfma && !flash;
-    const lm::FlashPlan fp = flash ? lm::flash_plan(a.heads, F, n_total) : lm::FlashPlan{};
-    const int64_t kp = flash ? lm::flash_keys(n_total) : plan.kp;
+    const int64_t kp = plan.kp;
     const size_t q_at = region(F * heads * qk);
     const size_t ql_at = region(F * ql);
     const size_t lat_at = region(F * (rank + rope));
     const size_t kvn_at = region(F * rank);
     const size_t kvx_at = region(F * heads * (c.qk_nope_head_dim + vh));
-    const size_t s_at = region(flash       ? lm::flash_partial_floats(fp, a.heads, core)
-                               : plan.mfma ? core * heads * kp
-                                           : core * heads * n_total);
+    const size_t s_at = region(plan.mfma ? core * heads * kp : core * heads * n_total);
     const size_t ctx_at = region(F * heads * vh);
     const size_t x16a_at = region(mfma ? halves(F * lm::round_up(H, lm::kPanel)) : 0);
     const size_t x16q_at = region(mfma && ql > 0 ? halves(F * lm::round_up(ql, lm::kPanel)) : 0);
@@ -387,9 +499,9 @@ int attention_tokens(AttnState* st, hipStream_t stream, int32_t layer, const flo
     const size_t partkv_at = region(partkv_f);
     const size_t k16_at = region(plan.mfma ? halves(heads * kp * qk) : 0);
     const size_t v16_at = region(plan.mfma ? halves(heads * vh * kp) : 0);
-    const size_t q16_at = region(gemm_core ? halves(heads * core * qk) : 0);
-    const size_t p16_at = region(gemm_core ? halves(heads * core * kp) : 0);
-    const size_t meta_at = region(gemm_core ? (lm::mfma_heads_meta_bytes(heads) + 3) / 4 : 0);
+    const size_t q16_at = region(plan.mfma ? halves(heads * core * qk) : 0);
+    const size_t p16_at = region(plan.mfma ? halves(heads * core * kp) : 0);
+    const size_t meta_at = region(plan.mfma ? (lm::mfma_heads_meta_bytes(heads) + 3) / 4 : 0);
     int rc = ensure_buffer(&st->ws, &st->ws_floats, stream, total_f);
     if (rc != LM_OK) {
         return rc;
@@ -479,18 +591,7 @@ int attention_tokens(AttnState* st, hipStream_t stream, int32_t layer, const flo
         LM_ATT_HIP(hipStreamWaitEvent(stream, st->join, 0));
     }
     // causal attention over the cache (:77-98), in groups of query tokens
-    if (flash) {
-        // the context lands in fp16 panels in x16kv as below; a group's
-        // partial contexts (when the keys are split) keep to the budget
-        LM_ATT_HIP(lm::launch_flash_pack(a, L.cache, n_total, h16(k16_at), h16(v16_at), stream));
-        const int64_t step = fp.splits > 1 ? core : F;
-        for (int64_t t0 = 0; t0 < F; t0 += step) {
-            LM_ATT_HIP(lm::launch_flash(a, fp, q + t0 * heads * qk, h16(k16_at), h16(v16_at), S,
-                                        std::min(step, F - t0), n0 + t0, n_total, st->scale, x16kv, t0, F, stream));
-        }
-        pskv.ready = x16kv;
-        pskv.ready_of = ctxv;
-    } else if (plan.mfma) {
+if (plan.mfma) {
         // the context lands in fp16 panels [F, heads vh] in x16kv (free once
         // kv_b has run), the output projection's input; ctxv holds the
         // per-head context of one group
@@ -916,6 +1017,7 @@ int lm_upload_attention(lm_context* ctx, int32_t layer, const uint16_t* q_proj_h
         }
         if (overflow == 0) {
             L.table16 = reinterpret_cast<const _Float16* const*>(b16);
+            std::copy(std::begin(table), std::end(table), L.w16);
         } else {
             (void)hipFree(L.slab16);  // a weight outside fp16's range: the layer keeps the BF16 path
             L.slab16 = nullptr;

@@ -545,8 +545,15 @@ hipError_t launch_attention_core_mfma(const AttnShape& a, const float* q, const 
 // The same core in one launch, scores and probabilities in registers, for
 // heads of 128 + 64 key and 128 value channels (k_flash.hip).
 bool flash_supported(const AttnShape& a);
-// Keys that the fp16 copies k16 [heads][.][192] and v16 [heads][.][128] hold.
+// Keys that the core's fp16 copies hold for a cache of `keys`: a multiple of 64.
 int64_t flash_keys(int64_t keys);
+// The copies (layouts: k_flash.hip), kp = flash_keys of the call's last key.
+struct FlashKv {
+    _Float16* nope16;  // [heads][kp][128]
+    _Float16* rope16;  // [kp][64]
+    _Float16* v16;     // [heads][kp / 64][128][64]
+    int64_t kp;
+};
 struct FlashPlan {
     int32_t waves = 4;        // 32-token waves per workgroup
     int32_t splits = 1;       // workgroups that share a query block's keys
@@ -555,12 +562,43 @@ struct FlashPlan {
 FlashPlan flash_plan(int32_t heads, int64_t tokens, int64_t keys);
 // Floats of `partial` for `tokens` query tokens (0 with one split).
 int64_t flash_partial_floats(const FlashPlan& p, int32_t heads, int64_t tokens);
-hipError_t launch_flash_pack(const AttnShape& a, const KvCacheDev& c, int64_t keys, _Float16* k16, _Float16* v16,
-                             hipStream_t s);
-// As launch_attention_core_mfma, for T query tokens at slots n0 .. n0 + T - 1.
-hipError_t launch_flash(const AttnShape& a, const FlashPlan& p, const float* q, const _Float16* k16,
-                        const _Float16* v16, float* partial, int64_t T, int64_t n0, int64_t keys, float scale,
-                        _Float16* ctx16, int64_t row0, int64_t ctx_rows, hipStream_t s);
+// Copies the first `keys` cached entries.
+hipError_t launch_flash_pack(const AttnShape& a, const KvCacheDev& c, int64_t keys, const FlashKv& kv, hipStream_t s);
+// T query tokens q16 [T][heads][192] (rotary applied) at slots n0 .. n0 + T - 1
+// -> the context in fp16 panels ctx16 [ctx_rows][heads 128], rows row0 ..
+hipError_t launch_flash(const AttnShape& a, const FlashPlan& p, const _Float16* q16, const FlashKv& kv, float* partial,
+                        int64_t T, int64_t n0, float scale, _Float16* ctx16, int64_t row0, int64_t ctx_rows,
+                        hipStream_t s);
+// The projections around that core with their next step as epilogue (k_proj.hip).
+enum ProjKind { kProjPlain = 0, kProjQuery = 1, kProjKv = 2 };
+struct ProjSegment {
+    const _Float16* w = nullptr;  // fp16 panels [rows, width]
+    int32_t rows = 0;             // a multiple of 4
+    int32_t kind = kProjPlain;
+    float* out = nullptr;         // plain: [tokens, rows]
+    int32_t accumulate = 0;       // plain: out += instead of out =
+};
+struct ProjArgs {
+    const _Float16* x16 = nullptr;  // fp16 panels [tokens, width]
+    int64_t tokens = 0;
+    int32_t width = 0;
+    int32_t heads = 0;
+    ProjSegment seg[2];
+    _Float16* q16 = nullptr;  // query: [tokens][heads][192]
+    KvCacheDev cache;         // kv
+    FlashKv kv{};
+    int64_t cap = 0, slot0 = 0, pos0 = 0, max_positions = 0;
+    const float* cos_t = nullptr;
+    const float* sin_t = nullptr;
+};
+hipError_t launch_proj(const ProjArgs& a, hipStream_t s);
+// gemm::rms_norm of rows in [rows, cols] into fp16 panels (cols % 32 == 0).
+hipError_t launch_norm16(const float* in, const float* w, _Float16* out16, int64_t rows, int32_t cols, float eps,
+                         hipStream_t s);
+// lat [tokens, rank + 64]: normalised latent into kvn16 panels, rotary keys into
+// the cache and the core's copy, zeros past the last key of its value tile.
+hipError_t launch_kv_prep16(const ProjArgs& a, const float* lat, const float* norm_w, _Float16* kvn16, int32_t rank,
+                            float eps, hipStream_t s);
 
 // ---- services of the context (lm_capi.hip) to the attention translation unit ----
 struct AttnState;

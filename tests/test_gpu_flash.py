@@ -25,8 +25,9 @@ def _f32(bits):
     return (np.asarray(bits).astype(np.uint32) << 16).view(np.float32).astype(np.float64)
 
 
-def _reference(m, x, cached):
-    """float64 attention of x [T, H] at positions cached.. over the layer's cache."""
+def _reference(m, x, cached, rotated=True):
+    """float64 attention of x [T, H] at positions cached.. over the layer's cache (past the
+    rotary table the channels stay as they are)."""
     from litemind_amd import mla_softmax_scale, rope_tables
     from litemind_amd import workload as wl
     d, L, T = m.d, m.L, x.shape[0]
@@ -36,7 +37,7 @@ def _reference(m, x, cached):
     cos, sin = (t[cached:n].astype(np.float64)[:, None] for t in rope_tables(cfg, n))
     q = (x.astype(np.float64) @ _f32(L.q_proj).T).reshape(T, d.heads, d.qk_head)
     even, odd = q[..., d.qk_nope::2], q[..., d.qk_nope + 1::2]
-    rot = np.concatenate([even * cos - odd * sin, odd * cos + even * sin], axis=-1)
+    rot = np.concatenate([even * cos - odd * sin, odd * cos + even * sin], axis=-1) if rotated else q[..., d.qk_nope:]
     scale = float(mla_softmax_scale(cfg))
     hidden = np.arange(n)[None] > np.arange(cached, n)[:, None]
     ctx = np.empty((T, d.heads, d.v_head))
@@ -78,6 +79,23 @@ def test_flash_core(heads, cached, T):
         assert mx <= ATT_MAX_ABS and rel <= ATT_MEAN_REL
         for t in (0, T - 1):  # no row is off while the mean is fine
             assert np.abs(y[t] - want[t]).sum() <= 2 * ATT_MEAN_REL * np.abs(want[t]).sum()
+    finally:
+        m.close()
+
+
+def test_flash_past_the_rotary_table():
+    """Positions at or past the table: queries and keys stay unrotated."""
+    from litemind_amd import PATH_MFMA
+    from litemind_amd import workload as wl
+    d = dataclasses.replace(wl.V2_LITE_MLA, max_positions=40)
+    announce("attention one-launch core past the rotary table")
+    m = Mla(d, 305, path=PATH_MFMA)
+    try:
+        x = tokens(306, 36, d.hidden)
+        y = m.forward(x, 40)
+        want = _reference(m, x, 0, rotated=False)
+        mx, rel = layer_error(y, want)
+        assert mx <= ATT_MAX_ABS and rel <= ATT_MEAN_REL
     finally:
         m.close()
 

@@ -16,8 +16,8 @@
 // ctx^T = V^T P^T, whose K order is free: the values are stored with the keys
 // of each group of 16 in the order in which the lanes hold them.  Waves of a
 // workgroup share the key and value tiles, staged straight to LDS two tiles
-// deep; 16-byte units are XOR-swizzled by row so the fragment reads of 8
-// neighbouring lanes fall on distinct banks.
+// deep, 16-byte units XOR-swizzled by row so that the fragment reads are free
+// of bank conflicts.
 //
 // Few query tokens over many keys would leave most CUs idle: the keys are then
 // split over several workgroups, whose unnormalised contexts, maxima and
@@ -189,9 +189,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_kernel(const F
             qf[ks] = *reinterpret_cast<const half8*>(qr + 16 * ks);
         }
     }
-    // Tile loads: a load fills 64 consecutive 16-byte positions; position p of
-    // row r holds unit p ^ (r % 8).  Rows of the nope keys have 16 positions
-    // (four rows a load), of the rotary keys and the values eight.
+    // Tile loads: a load fills 64 consecutive 16-byte positions.  A 16-byte LDS
+    // read serves 16 lanes, so 16 successive rows go to 16 different columns of
+    // banks: position p of row r holds unit p ^ (r % 16) of the nope keys (256
+    // bytes a row, four rows a load) and p ^ (r / 2 % 8) of the rotary keys and
+    // the values (128 bytes, eight rows).
     const int64_t head_keys = static_cast<int64_t>(h) * a.kv.kp;
     const __amdgpu_buffer_rsrc_t kres = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(a.kv.nope16 + head_keys * kNope), 0, static_cast<int>(a.kv.kp * kNope * 2), kBufferWord3);
@@ -199,54 +201,56 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_kernel(const F
         (void*)a.kv.rope16, 0, static_cast<int>(a.kv.kp * kRope * 2), kBufferWord3);
     const __amdgpu_buffer_rsrc_t vres = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(a.kv.v16 + head_keys * kVh), 0, static_cast<int>(a.kv.kp * kVh * 2), kBufferWord3);
-    unsigned ksrc[2];  // rows 0..3 and 4..7 of eight
+    unsigned ksrc[4], vsrc[2];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        ksrc[j] = static_cast<unsigned>((lane >> 4) * (kNope * 2) + ((lane & 15) ^ (4 * j + (lane >> 4))) * 16);
+    }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-        const int r = 4 * j + (lane >> 4);
-        ksrc[j] = static_cast<unsigned>((lane >> 4) * (kNope * 2) + ((lane & 15) ^ r) * 16);
+        vsrc[j] = static_cast<unsigned>((lane >> 3) * 128 + ((lane & 7) ^ (4 * j + (lane >> 4))) * 16);
     }
-    const unsigned vsrc = static_cast<unsigned>((lane >> 3) * 128 + ((lane & 7) ^ (lane >> 3)) * 16);
     auto issue = [&](int tile, char* ks, char* rs, char* vs) {
 #pragma unroll
         for (int j = 0; j < 16 / NW; ++j) {
             const int at = wave * (16 / NW) + j;  // a multiple of four, plus j
-            load_lds16(kres, ks + at * 1024, ksrc[j & 1], tile * kNopeBytes + at * 1024);
+            load_lds16(kres, ks + at * 1024, ksrc[j & 3], tile * kNopeBytes + at * 1024);
         }
 #pragma unroll
         for (int j = 0; j < 8 / NW; ++j) {
             const int at = wave * (8 / NW) + j;
-            load_lds16(rres, rs + at * 1024, vsrc, tile * kRopeBytes + at * 1024);
+            load_lds16(rres, rs + at * 1024, vsrc[j & 1], tile * kRopeBytes + at * 1024);
         }
 #pragma unroll
         for (int j = 0; j < 16 / NW; ++j) {
             const int at = wave * (16 / NW) + j;
-            load_lds16(vres, vs + at * 1024, vsrc, tile * kValueBytes + at * 1024);
+            load_lds16(vres, vs + at * 1024, vsrc[j & 1], tile * kValueBytes + at * 1024);
         }
     };
     f32x16 o[kVh / 32] = {};
     float m = -__builtin_inff();  // running maximum of the raw scores
-    float l = 0.0f;               // this half wave's share of the total
+    f32x4 l = {};                 // this half wave's share of the total, in four sums
     auto compute = [&](int tile, const char* ks, const char* rs, const char* vs) {
         f32x16 s[2] = {};
         const int r = lane & 31;
         // Fragments in sets of four (keys: two k-steps of both 32-key halves;
         // values: one k-step of all channels), each read before the MFMAs of
-        // the set before it.  Rows r + 32 i have r % 8 in common.
+        // the set before it.
         half8 fa[4], fb[4];
         auto read_keys = [&](int g, half8 (&f)[4]) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int row = 32 * (i & 1) + r, u = 4 * g + 2 * (i >> 1) + half;
                 f[i] = *reinterpret_cast<const half8*>(
-                    g < kNope / 32 ? ks + row * (kNope * 2) + (u ^ (r & 7)) * 16
-                                   : rs + row * (kRope * 2) + ((u - kNope / 8) ^ (r & 7)) * 16);
+                    g < kNope / 32 ? ks + row * (kNope * 2) + (u ^ (r & 15)) * 16
+                                   : rs + row * (kRope * 2) + ((u - kNope / 8) ^ ((r >> 1) & 7)) * 16);
             }
         };
         auto read_values = [&](int st, half8 (&f)[4]) {
 #pragma unroll
             for (int vt = 0; vt < 4; ++vt) {
                 f[vt] = *reinterpret_cast<const half8*>(vs + (32 * vt + r) * (kTile * 2) +
-                                                        ((2 * st + half) ^ (r & 7)) * 16);
+                                                        ((2 * st + half) ^ ((r >> 1) & 7)) * 16);
             }
         };
         auto score = [&](int g, const half8 (&f)[4]) {
@@ -284,11 +288,16 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_kernel(const F
                 }
             }
         }
-        float t = fmaxf(s[0][0], s[1][0]);
+        float t4[4];  // four chains
 #pragma unroll
-        for (int e = 1; e < 16; ++e) {
-            t = fmaxf(t, fmaxf(s[0][e], s[1][e]));
+        for (int e = 0; e < 4; ++e) {
+            t4[e] = fmaxf(s[0][e], s[1][e]);
+#pragma unroll
+            for (int k = 4; k < 16; k += 4) {
+                t4[e] = fmaxf(fmaxf(t4[e], s[0][e + k]), s[1][e + k]);
+            }
         }
+        float t = fmaxf(fmaxf(t4[0], t4[1]), fmaxf(t4[2], t4[3]));
         t = fmaxf(t, __shfl_xor(t, 32));
         const float m_new = fmaxf(m, t);
         if (__any(m_new > m)) {
@@ -308,7 +317,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_kernel(const F
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[st / 2][8 * (st & 1) + e], a.c, -mc));
-                l += p;
+                l[e % 4] += p;
                 pf[e] = static_cast<_Float16>(p);
             }
         };
@@ -352,7 +361,8 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_kernel(const F
             }
         }
     }
-    l += __shfl_xor(l, 32);
+    float total = (l[0] + l[1]) + (l[2] + l[3]);
+    total += __shfl_xor(total, 32);
     if (qi >= a.T) {
         return;
     }
@@ -361,7 +371,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_kernel(const F
         const int64_t at = (static_cast<int64_t>(split) * a.heads + h) * a.T + qi;
         if (half == 0) {
             a.part_ml[2 * at] = m;
-            a.part_ml[2 * at + 1] = l;
+            a.part_ml[2 * at + 1] = total;
         }
 #pragma unroll
         for (int vt = 0; vt < kVh / 32; ++vt) {
@@ -376,7 +386,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_kernel(const F
             }
         }
     } else {
-        const float inv = 1.0f / l;
+        const float inv = 1.0f / total;
 #pragma unroll
         for (int vt = 0; vt < kVh / 32; ++vt) {
             _Float16* row = a.ctx16 + panel_index(a.row0 + qi, h * kVh + 32 * vt, a.ctx_rows) + 4 * half;

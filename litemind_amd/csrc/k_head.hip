@@ -193,9 +193,8 @@ __global__ __launch_bounds__(THREADS) void head_logits_kernel(const uint16_t* __
 // four waves share every staged byte.  Tiles: 32 tokens x 32 rows
 // (32x32x2, 128 accumulators per lane), or 16 tokens x 16 NR rows (16x16x4).
 // A stage is 64 (or 128) elements of the tile's rows and tokens, loaded
-// straight to LDS with its 16-byte units XOR-swizzled by row, so that the
-// 16-byte reads of 8 neighbouring lanes fall on distinct banks; DEPTH stages
-// are in flight.  Each wave reads the next stage's operands before this
+// straight to LDS with its 16-byte units XOR-swizzled by row against bank
+// conflicts; DEPTH stages are in flight.  Each wave reads the next stage's operands before this
 // stage's MFMAs, which hide the reads.  At the end the waves exchange their
 // chains through the ring's LDS and reduce them in dot_bf16's order.
 //
@@ -256,6 +255,9 @@ struct ExactTile {
     static constexpr int kStageFloats = M * kElems + kRowsT * kElems / 2;
     static constexpr int kQuarter = M == 32 ? 4 : NR;    // accumulators of a chain that one wave finishes
     static_assert(kXLoads >= 1 && kWLoads >= 1);
+    // A 16-byte LDS read serves 16 lanes: 16 successive rows take 16 different
+    // columns of banks (rows of 128 bytes alternate between two halves).
+    static __device__ int wswizzle(int r) { return kWUnits == 8 ? (r >> 1) & 7 : r & 15; }
 };
 
 // in_dim % (32 kSteps) == 0.  `nt` token tiles, `nr` row tiles; workgroups that
@@ -290,8 +292,8 @@ __global__ __launch_bounds__(256, 2) void matvec_exact_kernel(const uint16_t* __
     const __amdgpu_buffer_rsrc_t wres =
         __builtin_amdgcn_make_buffer_rsrc((void*)(w + row0 * in_dim), 0, nrow * in_dim * 2, kHeadBufferWord3);
     // Load j of a stage fills 64 consecutive 16-byte positions p; position p of
-    // row (or token) r = p / units holds its unit (p % units) ^ (r % 16), with
-    // the XOR cut to the row's units.  Rows past the end load the last one.
+    // token r = p / units holds its unit (p % units) ^ (r % 16), of a weight row
+    // (p % units) ^ wswizzle(r).  Rows past the end load the last one.
     unsigned xsrc[T::kXLoads], wsrc[T::kWLoads];
 #pragma unroll
     for (int j = 0; j < T::kXLoads; ++j) {
@@ -304,7 +306,7 @@ __global__ __launch_bounds__(256, 2) void matvec_exact_kernel(const uint16_t* __
     for (int j = 0; j < T::kWLoads; ++j) {
         const int p = (wave * T::kWLoads + j) * 64 + lane;
         const int r = p / T::kWUnits;
-        const int u = (p % T::kWUnits) ^ (r & (T::kWUnits - 1));
+        const int u = (p % T::kWUnits) ^ T::wswizzle(r);
         wsrc[j] = static_cast<unsigned>((min(r, nrow - 1) * in_dim + 8 * u) * 2);
     }
     auto issue = [&](int stage, float* slot) {
@@ -331,7 +333,7 @@ __global__ __launch_bounds__(256, 2) void matvec_exact_kernel(const uint16_t* __
         for (int n = 0; n < NR; ++n) {
             const int r = n * M + li;
             wv[n] = *reinterpret_cast<const uint4*>(slot + M * T::kElems + r * (T::kElems / 2) +
-                                                    4 * (wu ^ (r & (T::kWUnits - 1))));
+                                                    4 * (wu ^ T::wswizzle(r)));
         }
     };
     ChainTile<M, NR> acc[8];

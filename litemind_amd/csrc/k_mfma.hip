@@ -29,11 +29,14 @@
 // flight, each in its own LDS array so the compiler can track the asynchronous
 // writes per buffer.  Two workgroups share a CU, so one's memory waits are
 // covered by the other's MFMAs.  Rows past the end of a group (tokens) or of a
-// matrix (weight rows) load a clamped row and are never stored.  Two shapes:
+// matrix (weight rows) load a clamped row and are never stored.  Three shapes
+// (tile_shape):
 //   128 x 256, 2 x 2 waves of 64 x 128, 3 stages (24 KB each): large groups;
 //    64 x 256, 1 x 4 waves of 64 x 64, 4 stages (20 KB each): groups of a few
 //    dozen rows, where the kernel streams weights and the bytes in flight
-//    per CU (two workgroups x (STAGES - 1) x 16 KB of weights) set its rate.
+//    per CU (two workgroups x (STAGES - 1) x 16 KB of weights) set its rate;
+//    64 x 128, 2 x 2 waves of 32 x 64, 5 stages (12 KB each): small groups,
+//    twice the workgroups and a smaller last round.
 //
 // Measured alternatives, not kept (T = 2048 skewed / T = 4096 MoE layer, gate/up
 // µs on one box): 256 x 256 or 192 x 256 tiles of one workgroup per CU with the
@@ -50,14 +53,6 @@
 
 namespace lm {
 namespace {
-
-constexpr int BN = 256;  // weight rows per tile
-
-// Launches whose average routed group fits one 64-row tile (T k <= 64 E; a
-// dense layer: T <= 64) take the 64-row shape.  Measured on V2-Lite (one MoE block, 64 experts, k 6): 8-12%
-// faster from T = 8 to T = 512, 4-13% slower from T = 768 on, where groups
-// span several 64-row tiles and each re-streams the expert's weights.
-constexpr int64_t kNarrowRows = 64;
 
 enum Mode { kGateUp = 0, kDown = 1 };
 
@@ -217,13 +212,13 @@ template <int MODE, int WM, int WN, int MI, int NJ, int STAGES>
 __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2, 2))) void mfma_grouped_kernel(
     ExpertArgs a) {
     using Z = Shape<WM, WN, MI, NJ, STAGES>;
-    constexpr int BM = Z::BM;
+    constexpr int BM = Z::BM, BN = Z::BN;
     // One LDS array per stage: the compiler tracks the asynchronous LDS writes
     // per array.
-    constexpr int kStage3 = STAGES > 3 ? Z::kStageBytes : 16;
+    static_assert(STAGES <= 5);
     __shared__ __attribute__((aligned(1024))) char s0[Z::kStageBytes], s1[Z::kStageBytes], s2[Z::kStageBytes],
-        s3[kStage3];
-    char* const bufs[6] = {s0, s1, s2, s3, s3, s3};
+        s3[STAGES > 3 ? Z::kStageBytes : 16], s4[STAGES > 4 ? Z::kStageBytes : 16];
+    char* const bufs[6] = {s0, s1, s2, s3, s4, s4};
     Tile<MODE, WM, WN, MI, NJ, STAGES> t;
     t.lane = threadIdx.x & 63;
     t.wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
@@ -245,12 +240,13 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
                      MODE == kDown ? kDownGroupM : 0, ti, reinterpret_cast<int*>(bufs[STAGES - 1]))) {
         return;
     }
+    const bool shared = ti.g >= a.experts;
+    const int chunks = shared ? ksplit : 1;  // the routed groups keep their K whole
     int kc = 0;
-    if (ksplit > 1) {
+    if (chunks > 1) {
         kc = ti.nt / nt_shared;
         ti.nt -= kc * nt_shared;
     }
-    const bool shared = ti.g >= a.experts;
     const int width_p = shared ? a.shared_inter_p : inter_p;
     const int n_rows = shared ? n_shared : n_routed;
     const int K = MODE == kGateUp ? a.hidden_p : width_p;
@@ -295,7 +291,7 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
     t.b_step = static_cast<unsigned>(n_rows) * kRowBytes;
     // this tile's K stages [k0, k0 + nk): all of K, or chunk kc of the split
     const int nk_all = K / BK;
-    const int kchunk = (nk_all + ksplit - 1) / ksplit;
+    const int kchunk = (nk_all + chunks - 1) / chunks;
     const int k0 = kc * kchunk;
     const int nk = nk_all - k0 < kchunk ? nk_all - k0 : kchunk;  // >= 1: the launcher's choice of ksplit
 #pragma unroll
@@ -341,7 +337,7 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
                     }
                 }
             } else {
-                float* const dst = ksplit > 1 ? a.partial + static_cast<int64_t>(kc) * a.tokens * a.hidden : a.down_out;
+                float* const dst = a.down_out + static_cast<int64_t>(kc) * a.tokens * a.hidden;
 #pragma unroll
                 for (int j = 0; j < NJ; ++j) {
                     const int h = ti.nt * BN + t.wn * (32 * NJ) + j * 32 + n;
@@ -371,7 +367,7 @@ hipError_t launch_shape(const ExpertArgs& a, hipStream_t s) {
     const int nr = MODE == kGateUp ? 2 * a.inter_p : a.hidden;
     const int ns = MODE == kGateUp ? 2 * a.shared_inter_p : a.hidden;
     const int ksplit = MODE == kDown && a.ksplit > 1 ? a.ksplit : 1;
-    const int64_t grid = tile_bound(a, S::BM, (nr + BN - 1) / BN, (ns + BN - 1) / BN * ksplit);
+    const int64_t grid = tile_bound(a, S::BM, (nr + S::BN - 1) / S::BN, (ns + S::BN - 1) / S::BN * ksplit);
     hipLaunchKernelGGL((mfma_grouped_kernel<MODE, WM, WN, MI, NJ, STAGES>), dim3(static_cast<unsigned>(grid)),
                        dim3(S::kThreads), 0, s, a);
     return hipGetLastError();
@@ -387,6 +383,52 @@ bool offsets_fit(const ExpertArgs& a) {
            2 * widest * a.hidden_p * 2 <= limit && static_cast<int64_t>(a.hidden) * widest * 2 <= limit;
 }
 
+// Tiles of 64 x 128, 64 x 256 or 128 x 256 (tokens x weight rows).
+enum class TileShape { kThin, kNarrow, kWide };
+
+// Which tile a launch takes.  Routed layers stream every active expert's
+// weights: while the average group fits half a 64-row tile the finer 64 x 128
+// tiles leave a smaller last round (V2-Lite, gate/up and down back to back:
+// 8 tokens 128 us against 139 with 64 x 256 tiles, 16 167 / 182, 128 209 / 213,
+// 256 221 / 231, 509 255 / 245); up to one 64-row tile 64 x 256; past that
+// every extra 64-row tile would stream the weights again (768 tokens and more:
+// 4 to 13% slower).  A layer without routed experts is one group of T rows
+// with few column blocks: its gate/up (V2-Lite's dense layer, 8 / 137 / 256
+// tokens) takes 17 / 35 / 43 us with 64 x 128 tiles, 25 / 29 / 47 with 64 x 256
+// and 32 / 37 / 39 with 128 x 256; its down, with K split, 10 / 17 / 21 (64 x
+// 128), 11 / 18 / 20, 11 / 19 / 22, and 35 against 30 us at 512 tokens.
+TileShape tile_shape(const ExpertArgs& a, int mode) {
+    if (a.experts > 0) {
+        const int64_t rows = a.tokens * a.top_k;
+        return rows <= 32 * a.experts ? TileShape::kThin : rows <= 64 * a.experts ? TileShape::kNarrow : TileShape::kWide;
+    }
+    if (mode == kGateUp) {
+        return a.tokens <= 64 ? TileShape::kThin : a.tokens <= 192 ? TileShape::kNarrow : TileShape::kWide;
+    }
+    return a.tokens <= 256 ? TileShape::kThin : TileShape::kWide;
+}
+
+// K chunks of the shared group's down GEMM (hidden columns, K = shared_inter_p).
+// Without routed experts: while its tiles fill less than a round of workgroups
+// (two per CU for the thin tiles, one for the wide ones), at most `most` chunks
+// of at least 8 stages.  Beside routed experts whose weights stream, chunks no
+// longer than their K: the shared tiles are the launch's longest otherwise.
+int32_t down_chunks(const ExpertArgs& a, int64_t most) {
+    const TileShape shape = tile_shape(a, kDown);
+    const int64_t nk = a.shared_inter_p / BK;
+    int64_t ks = 1;
+    if (a.experts > 0) {
+        ks = shape == TileShape::kThin && a.inter_p > 0 ? a.shared_inter_p / a.inter_p : 1;
+    } else {
+        const bool wide = shape == TileShape::kWide;
+        const int64_t tiles = (a.tokens + (wide ? 127 : 63)) / (wide ? 128 : 64) * ((a.hidden + (wide ? 255 : 127)) / (wide ? 256 : 128));
+        ks = (wide ? 256 : 512) / tiles;
+    }
+    ks = std::max<int64_t>(1, std::min({ks, most, nk / 8}));
+    const int64_t chunk = (nk + ks - 1) / ks;
+    return static_cast<int32_t>((nk + chunk - 1) / chunk);  // every chunk holds at least one stage
+}
+
 template <int MODE>
 hipError_t launch(const ExpertArgs& a, hipStream_t s) {
     if (a.tokens <= 0) {
@@ -396,12 +438,14 @@ hipError_t launch(const ExpertArgs& a, hipStream_t s) {
         !offsets_fit(a)) {
         return hipErrorInvalidValue;
     }
-    // A layer without routed experts (the dense FFN) is one group of T rows.
-    const bool narrow = a.experts > 0 ? a.tokens * a.top_k <= kNarrowRows * a.experts : a.tokens <= kNarrowRows;
-    if (narrow) {
-        return launch_shape<MODE, 1, 4, 2, 2, 4>(a, s);
+    switch (tile_shape(a, MODE)) {
+        case TileShape::kThin:
+            return launch_shape<MODE, 2, 2, 1, 2, 5>(a, s);
+        case TileShape::kNarrow:
+            return launch_shape<MODE, 1, 4, 2, 2, 4>(a, s);
+        default:
+            return launch_shape<MODE, 2, 2, 2, 4, 3>(a, s);
     }
-    return launch_shape<MODE, 2, 2, 2, 4, 3>(a, s);
 }
 
 // out[i] = (accumulate ? out[i] : 0) + (p_0[i] + p_1[i] + ... + p_{n-1}[i]), the
@@ -442,26 +486,11 @@ hipError_t launch_mfma_gemm(const _Float16* a16, const _Float16* const* w, float
     ea.inter_p = 0;
     ea.shared_inter_p = Kp;
     ea.has_shared = 1;
-    // Split K while the tiles fill less than half of the workgroup slots (two
-    // per CU), keeping at least 8 stages per chunk and at most 4 chunks.
-    const int64_t bm = M <= kNarrowRows ? 64 : 128;
-    const int64_t tiles = (M + bm - 1) / bm * ((N + BN - 1) / BN);
-    const int nk = Kp / BK;
-    int ks = 1;
-    if (tiles < 256) {
-        ks = static_cast<int>(std::min<int64_t>({(256 + tiles - 1) / tiles, 4, nk / 8}));
-        ks = ks < 1 ? 1 : ks;
-        const int chunk = (nk + ks - 1) / ks;
-        ks = (nk + chunk - 1) / chunk;  // every chunk holds at least one stage
-        if (static_cast<int64_t>(ks) * M * N > scratch_floats) {
-            ks = 1;
-        }
-    }
+    const int32_t ks = std::max<int32_t>(1, down_chunks(ea, std::min<int64_t>(4, scratch_floats / (M * N))));
     const bool via_scratch = ks > 1 || accumulate;
     if (via_scratch) {
         ea.down_out = scratch;
         ea.ksplit = ks;
-        ea.partial = scratch;
     }
     hipError_t e = launch<kDown>(ea, s);
     if (e != hipSuccess || !via_scratch) {
@@ -527,5 +556,12 @@ hipError_t launch_mfma_heads(const _Float16* a16, const _Float16* w16, int64_t w
 hipError_t launch_mfma_gateup(const ExpertArgs& a, hipStream_t s) { return launch<kGateUp>(a, s); }
 
 hipError_t launch_mfma_down(const ExpertArgs& a, hipStream_t s) { return launch<kDown>(a, s); }
+
+int32_t mfma_shared_chunks(const ExpertArgs& a) {
+    if (a.tokens <= 0 || !a.has_shared || a.shared_inter_p < BK) {
+        return 1;
+    }
+    return down_chunks(a, std::min<int64_t>(8, kSplitRows / a.tokens));
+}
 
 }  // namespace lm

@@ -11,6 +11,31 @@ namespace {
 // K > 0 (the top-k known when compiling) the K rows' loads are all in flight
 // before the first addition; K = 0 reads the top-k at run time, one row at a
 // time.  The additions are the same either way.
+
+// Adds chunks 1, 2, ... of the shared row at `row` (column c, one chunk every
+// tokens rows) to chunk 0's `first`, four loads in flight.
+__device__ inline float4 add_chunks(const CombineArgs& a, float4 first, const float* row, int c) {
+    const int64_t step = a.tokens * a.hidden;
+    for (int k0 = 1; k0 < a.shared_chunks; k0 += 4) {
+        float4 d[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int k = k0 + u < a.shared_chunks ? k0 + u : k0;
+            d[u] = *reinterpret_cast<const float4*>(row + k * step + c);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (k0 + u < a.shared_chunks) {
+                first.x = first.x + d[u].x;
+                first.y = first.y + d[u].y;
+                first.z = first.z + d[u].z;
+                first.w = first.w + d[u].w;
+            }
+        }
+    }
+    return first;
+}
+
 template <int K>
 __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a) {
     const int quads = a.hidden / 4;
@@ -49,8 +74,8 @@ __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a) {
         }
     }
     if (a.has_shared) {
-        const int64_t s = a.tokens * a.top_k + t;
-        const float4 d = *reinterpret_cast<const float4*>(a.down_out + s * a.hidden + c);
+        const float* const row = a.down_out + (a.tokens * a.top_k + t) * a.hidden;
+        const float4 d = add_chunks(a, *reinterpret_cast<const float4*>(row + c), row, c);
         acc.x = acc.x + d.x;
         acc.y = acc.y + d.y;
         acc.z = acc.z + d.z;
@@ -134,6 +159,8 @@ __global__ __launch_bounds__(256) void combine_norm_kernel(CombineArgs a) {
 #pragma unroll
         for (int k = 0; k < STEPS; ++k) {
             if (a.has_shared) {
+                const int c = 1024 * k + 4 * tid;
+                sh[k] = add_chunks(a, sh[k], shared_row, c < H ? c : 0);
                 y[k].x = y[k].x + sh[k].x;
                 y[k].y = y[k].y + sh[k].y;
                 y[k].z = y[k].z + sh[k].z;
@@ -167,7 +194,8 @@ __global__ __launch_bounds__(256) void combine_norm_kernel(CombineArgs a) {
             const int c = 1024 * k + 4 * tid;
             if (c < H) {
                 if (a.has_shared) {
-                    const float4 d = *reinterpret_cast<const float4*>(dout + (a.tokens * a.top_k + t) * H + c);
+                    const float* const from = dout + (a.tokens * a.top_k + t) * H;
+                    const float4 d = add_chunks(a, *reinterpret_cast<const float4*>(from + c), from, c);
                     y[k].x = y[k].x + d.x;
                     y[k].y = y[k].y + d.y;
                     y[k].z = y[k].z + d.z;

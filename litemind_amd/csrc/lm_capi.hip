@@ -392,7 +392,8 @@ int ensure_workspace(lm_context* ctx, int64_t tokens) {
     LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.slot_of), sizeof(int32_t) * static_cast<size_t>(TK)));
     LM_HIP(hipMalloc(&w.act, sizeof(float) * act_elems));
     LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.x16), sizeof(_Float16) * static_cast<size_t>(T * ctx->Hp)));
-    LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.down_out), sizeof(float) * static_cast<size_t>((TK + T) * ctx->H)));
+    LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.down_out), 
+                     sizeof(float) * static_cast<size_t>((TK + std::max(T, lm::kSplitRows)) * ctx->H)));
     LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.xnorm), sizeof(float) * static_cast<size_t>(T * ctx->H)));
     LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.ffn), sizeof(float) * static_cast<size_t>(T * ctx->H)));
     LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.zero), sizeof(int32_t) * 4));
@@ -522,7 +523,8 @@ int launch_expert_kernels(lm_context* ctx, const Layer& L, const lm::ExpertArgs&
 int run_experts(lm_context* ctx, Layer& L, const float* x, const _Float16* x16, int64_t T, const lm::RouteBufs& rb,
                 float* y, const float* residual, bool mfma, const float* next_norm = nullptr,
                 bool gateup_done = false) {
-    const lm::ExpertArgs ea = expert_args(ctx, L, x, x16, T, rb);
+    lm::ExpertArgs ea = expert_args(ctx, L, x, x16, T, rb);
+    ea.ksplit = mfma ? lm::mfma_shared_chunks(ea) : 1;
     const int rc = launch_expert_kernels(ctx, L, ea, T, mfma, gateup_done);
     if (rc != LM_OK) {
         return rc;
@@ -538,6 +540,7 @@ int run_experts(lm_context* ctx, Layer& L, const float* x, const _Float16* x16, 
     ca.hidden = ctx->H;
     ca.top_k = ea.top_k;
     ca.has_shared = ea.has_shared;
+    ca.shared_chunks = ea.ksplit;
     ca.next_norm = next_norm;
     ca.xnorm = ctx->ws.xnorm;
     ca.x16 = mfma ? ctx->ws.x16 : nullptr;

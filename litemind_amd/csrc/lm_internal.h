@@ -138,11 +138,10 @@ struct ExpertArgs {
     int32_t hidden, hidden_p, experts, top_k;
     int32_t inter_p, shared_inter_p;   // padded widths (shared 0 = none)
     int32_t has_shared;
-    // Down GEMM of a layer without routed experts only: K split into ksplit
-    // chunks (0 or 1: none), chunk c's partial sums [T, hidden] at
-    // partial + c T hidden instead of down_out.
+    // MFMA down GEMM of the shared expert (or the dense FFN): K split into ksplit
+    // chunks (0 or 1: none), chunk c's partial sums [T, hidden] c T rows past
+    // the shared rows of down_out.
     int32_t ksplit;
-    float* partial;
 };
 
 struct CombineArgs {
@@ -153,6 +152,7 @@ struct CombineArgs {
     const float* residual;   // [T, H] or null: y = residual + ffn
     int64_t tokens;
     int32_t hidden, top_k, has_shared;
+    int32_t shared_chunks;   // partial sums of each shared row (ExpertArgs::ksplit; 0 or 1: one)
     // The next stack layer's RMSNorm applied to y in the same pass (null: none):
     // xnorm [T, H] = rms_norm(y, next_norm), and x16 (or null) its fp16 copy in
     // panel layout [T, hidden_p].
@@ -623,6 +623,10 @@ hipError_t launch_gemv_down(const ExpertArgs& a, int64_t max_groups, hipStream_t
 // Grouped SwiGLU on MFMA (k_mfma.hip): fp16 panel operands, fp32 accumulation.
 hipError_t launch_mfma_gateup(const ExpertArgs& a, hipStream_t s);
 hipError_t launch_mfma_down(const ExpertArgs& a, hipStream_t s);
+// The ksplit worth using for a layer, with T ksplit <= max(T, kSplitRows) so
+// that down_out needs max(T, kSplitRows) rows past the routed ones.
+constexpr int64_t kSplitRows = 4096;
+int32_t mfma_shared_chunks(const ExpertArgs& a);
 // out [M, N] = a16 . W^T (accumulate: out += a16 . W^T) for a16 [M, Kp] and W
 // [N, Kp] fp16 panels (*w, a device pointer to the matrix), fp32 accumulation,
 // on the down kernel as one group of M rows.  With few tiles the K range is

@@ -36,7 +36,7 @@ struct Shape {
     static constexpr int NP = (MI * NJ + 1) / 2;       // MFMA pairs per half step
     static_assert(AL * 1024 * WAVES == kABytes && AL >= 1, "whole A instructions per wave");
     static_assert(BL * 1024 * WAVES == kBBytes && BL >= 1, "whole B instructions per wave");
-    static_assert(NR <= 2 * NP && L <= 4 * NP, "reads and loads spread over the MFMA pairs");
+    static constexpr int RP = NR <= 2 * NP ? 2 : (NR + NP - 1) / NP;  // second half step's reads per MFMA pair
     static_assert(STAGES >= 3 && STAGES <= 6 && (STAGES - 2) * L < 64, "pipeline depth, vmcnt");
     static_assert(STAGES * kStageBytes <= 80 * 1024, "two workgroups per CU");
 };
@@ -145,7 +145,7 @@ struct Tile {
         for (int p = 0; p < 2 * Z::NP; ++p) {
             if (p < Z::NP) {
 #pragma unroll
-                for (int r = 2 * p; r < 2 * p + 2; ++r) {
+                for (int r = Z::RP * p; r < Z::RP * (p + 1); ++r) {
                     if (r < Z::NR) {
                         read1(cur, 1, r);
                     }

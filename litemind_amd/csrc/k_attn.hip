@@ -890,6 +890,119 @@ __global__ __launch_bounds__(256) void context_kernel(const float* __restrict__ 
     }
 }
 
+// The same sums on the fp32 matrix cores, v_head a multiple of 16:
+// v_mfma_f32_16x16x4_f32 forms each output as a chain of fused multiply-adds
+// over its four k in order, rounded as fmaf rounds (as the projections of
+// k_head.hip use it), so with k running over successive cached tokens one
+// accumulator tile holds 16 query tokens x 16 channels of exactly these
+// chains: 8 cycles per cached token for all 256, where context_kernel spends
+// about 50 on 8 tokens of one wave.  The matrix instruction takes the keys that
+// every token of the tile sees; the last few, up to each token's own position,
+// are added on the vector unit with a test per token (a zero probability times
+// an unseen value would not be the same sum for infinite values or negative
+// zeros).  A workgroup is 16 tokens x 64 channels of one head, a wave 16
+// channels; the probabilities pass through LDS in chunks, the values come from
+// L2 kCtxMAhead steps ahead.  Bound by the chains' latency.  V2-Lite: 2 tokens
+// after 1000 58 us for the whole call before, 36 after.
+constexpr int kCtxMTokens = 16;
+constexpr int kCtxMKeys = 512;                  // keys of a chunk
+constexpr int kCtxMStride = kCtxMKeys + 4;      // floats per token's row: 16 rows x 4 keys on 64 banks
+constexpr int kCtxMAhead = 8;                   // value loads in flight per lane, 4 keys each
+
+__global__ __launch_bounds__(256) void context_mfma_kernel(const float* __restrict__ P, const float* __restrict__ value,
+                                                           float* __restrict__ ctx, int32_t heads, int32_t vh,
+                                                           int64_t cap, int64_t n0, int64_t T, int64_t n_stride) {
+    typedef float f4v __attribute__((ext_vector_type(4)));
+    __shared__ float ps[kCtxMTokens * kCtxMStride];
+    const int h = blockIdx.x;
+    const int64_t i0 = static_cast<int64_t>(blockIdx.y) * kCtxMTokens;
+    const int nq = static_cast<int>(std::min<int64_t>(kCtxMTokens, T - i0));
+    const int64_t n_hi = n0 + i0 + nq;             // keys the tile's last token sees
+    const int64_t n_all = n0 + i0 + 1;             // keys every token of the tile sees
+    const int64_t n_mfma = n_all / 4 * 4;          // taken by the matrix instruction
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    const int col = lane & 15, g = lane >> 4;
+    const int c = (static_cast<int>(blockIdx.z) * 4 + wave) * 16 + col;
+    const bool live = c - col < vh;                // whole waves: vh % 16 == 0
+    const float* const vp = value + static_cast<int64_t>(h) * cap * vh + (live ? c : 0);
+    f4v acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int64_t c0 = 0; c0 < n_hi; c0 += kCtxMKeys) {
+        const int cend = static_cast<int>(std::min<int64_t>(kCtxMKeys, n_hi - c0));
+        __syncthreads();
+        // the chunk's probabilities, a row of 16 tokens per wave and step; the
+        // loads are unconditional (tokens past the last read the last, keys
+        // past a token's own are inside its row and not used)
+        for (int r0 = wave; r0 < kCtxMTokens; r0 += 4) {
+            const int64_t t = i0 + (r0 < nq ? r0 : nq - 1);
+            const float* const row = P + (t * heads + h) * n_stride + c0;
+            float v[kCtxMKeys / 64];
+#pragma unroll
+            for (int u = 0; u < kCtxMKeys / 64; ++u) {
+                const int k = 64 * u + lane;
+                v[u] = row[k < cend ? k : cend - 1];
+            }
+#pragma unroll
+            for (int u = 0; u < kCtxMKeys / 64; ++u) {
+                ps[r0 * kCtxMStride + 64 * u + lane] = v[u];
+            }
+        }
+        __syncthreads();
+        const int steps = static_cast<int>(std::max<int64_t>(0, std::min<int64_t>(cend, n_mfma - c0))) / 4;
+        // step s: keys c0 + 4 s .. + 3, this lane's is c0 + 4 s + g; steps past
+        // the last reload it (every group issues the same loads)
+        auto load = [&](int s0, float (&x)[kCtxMAhead]) {
+#pragma unroll
+            for (int u = 0; u < kCtxMAhead; ++u) {
+                const int s = s0 + u < steps ? s0 + u : (steps > 0 ? steps - 1 : 0);
+                const int64_t key = std::min<int64_t>(c0 + 4 * s + g, n_hi - 1);
+                x[u] = vp[key * vh];
+            }
+        };
+        auto add = [&](int s0, const float (&x)[kCtxMAhead]) {
+            float a[kCtxMAhead];
+#pragma unroll
+            for (int u = 0; u < kCtxMAhead; ++u) {
+                a[u] = ps[col * kCtxMStride + std::min(4 * (s0 + u) + g, kCtxMKeys - 1)];
+            }
+#pragma unroll
+            for (int u = 0; u < kCtxMAhead; ++u) {
+                if (s0 + u < steps) {
+                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u], x[u], acc, 0, 0, 0);
+                }
+            }
+        };
+        float x0[kCtxMAhead], x1[kCtxMAhead];
+        load(0, x0);
+        for (int s = 0; s < steps; s += 2 * kCtxMAhead) {
+            load(s + kCtxMAhead, x1);
+            add(s, x0);
+            load(s + 2 * kCtxMAhead, x0);
+            add(s + kCtxMAhead, x1);
+        }
+        // the keys that not every token sees: register r of the tile is token
+        // 4 g + r, column `col`
+        for (int k = static_cast<int>(std::max<int64_t>(0, n_mfma - c0)); k < cend; ++k) {
+            const float x = vp[(c0 + k) * vh];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int t = 4 * g + r;
+                const float sum = __builtin_fmaf(ps[t * kCtxMStride + k], x, acc[r]);
+                acc[r] = c0 + k <= n0 + i0 + t ? sum : acc[r];
+            }
+        }
+    }
+    if (live) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int t = 4 * g + r;
+            if (t < nq) {
+                ctx[((i0 + t) * heads + h) * vh + c] = acc[r];
+            }
+        }
+    }
+}
+
 // The same sum for one query token (decode), T = 1: ctx[h, v] over cached
 // tokens j < n in order.  One workgroup per (head, 16 value channels); lanes
 // 0..15 of wave 0 run the 16 chains from LDS.  The channels' values (64 B per
@@ -1386,6 +1499,13 @@ hipError_t launch_attention_core(const AttnShape& a, const KvCacheDev& c, const 
     } else if (T == 1 && grouped) {
         hipLaunchKernelGGL(scores_grouped_kernel<1>, dim3(tiles, a.heads, 1), dim3(kKeyTile), sizeof(float) * qk, s,
                            q, c.key_nope, c.key_rope, S, a.heads, a.nope, a.rope, a.cap, n0, T, n_stride, scale);
+    } else if (T <= 2 && grouped) {
+        // a block's time grows with its query tokens, padded ones included
+        hipLaunchKernelGGL(scores_grouped_kernel<2>, dim3(tiles, a.heads, 1), dim3(kKeyTile), sizeof(float) * 2 * qk, s,
+                           q, c.key_nope, c.key_rope, S, a.heads, a.nope, a.rope, a.cap, n0, T, n_stride, scale);
+    } else if (T <= 4 && grouped) {
+        hipLaunchKernelGGL(scores_grouped_kernel<4>, dim3(tiles, a.heads, 1), dim3(kKeyTile), sizeof(float) * 4 * qk, s,
+                           q, c.key_nope, c.key_rope, S, a.heads, a.nope, a.rope, a.cap, n0, T, n_stride, scale);
     } else if (grouped) {
         hipLaunchKernelGGL(scores_grouped_kernel<kQueries>, dim3(tiles, a.heads, blocks_of(T, kQueries)),
                            dim3(kKeyTile), sizeof(float) * kQueries * qk, s, q, c.key_nope, c.key_rope, S, a.heads,
@@ -1431,6 +1551,10 @@ hipError_t launch_attention_core(const AttnShape& a, const KvCacheDev& c, const 
     } else if (T == 1) {
         hipLaunchKernelGGL(context_kernel<1>, dim3(a.heads, 1), dim3(threads), 0, s, S, c.value, ctx, a.heads, a.vh,
                            a.cap, n0, T, n_stride);
+    } else if (a.vh % 16 == 0) {
+        hipLaunchKernelGGL(context_mfma_kernel,
+                           dim3(a.heads, blocks_of(T, kCtxMTokens), static_cast<unsigned>((a.vh + 63) / 64)), dim3(256),
+                           0, s, S, c.value, ctx, a.heads, a.vh, a.cap, n0, T, n_stride);
     } else {
         hipLaunchKernelGGL(context_kernel<kQueries>, dim3(a.heads, blocks_of(T, kQueries)), dim3(threads), 0, s, S,
                            c.value, ctx, a.heads, a.vh, a.cap, n0, T, n_stride);

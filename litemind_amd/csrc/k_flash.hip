@@ -33,6 +33,8 @@ constexpr int kNope = 128;
 constexpr int kRope = 64;
 constexpr int kQk = kNope + kRope;
 constexpr int kVh = 128;
+constexpr int NW = 4;                           // waves of 32 query tokens per workgroup
+constexpr int kBlock = 32 * NW;                 // query tokens per workgroup
 constexpr int kTile = 64;                       // keys per tile
 constexpr int kNopeBytes = kTile * kNope * 2;   // 16 KB
 constexpr int kRopeBytes = kTile * kRope * 2;   // 8 KB
@@ -143,8 +145,8 @@ struct FlashArgs {
     float c;               // softmax scale times log2(e)
 };
 
-template <int NW, bool SPLIT>
-__global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_kernel(const FlashArgs a) {
+template <bool SPLIT>
+__global__ __launch_bounds__(64 * NW, 2) void flash_kernel(const FlashArgs a) {
     __shared__ __align__(16) char k0[kNopeBytes], k1[kNopeBytes], r0[kRopeBytes], r1[kRopeBytes], v0[kValueBytes],
         v1[kValueBytes];
     char* const kring[2] = {k0, k1};
@@ -168,16 +170,19 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_kernel(const F
     }
     const int heavy = (a.qblocks + 1) / 2;
     const int qb = order < heavy ? a.qblocks - 1 - order : order - heavy;
-    const int64_t q0 = static_cast<int64_t>(qb) * (32 * NW);
+    const int64_t q0 = static_cast<int64_t>(qb) * kBlock;
     const int half = lane >> 5;
     const int64_t qw = q0 + 32 * wave;                              // the wave's first query
     const int64_t qi = qw + (lane & 31);                            // this lane's query
     const int64_t qc = std::min<int64_t>(qi, a.T - 1);
     const int64_t vis = a.n0 + qc;                                  // last key it sees
-    const int64_t block_keys = a.n0 + std::min<int64_t>(a.T, q0 + 32 * NW);
+    const int64_t block_keys = a.n0 + std::min<int64_t>(a.T, q0 + kBlock);
     const int all_tiles = static_cast<int>((block_keys + kTile - 1) / kTile);
     const int tile0 = SPLIT ? split * a.split_tiles : 0;
     const int tile_end = SPLIT ? std::min(all_tiles, tile0 + a.split_tiles) : all_tiles;
+    if (SPLIT && tile0 >= tile_end) {
+        return;  // the block's keys end before this split (flash_combine_kernel does not read it)
+    }
     // tiles this wave has a visible key in; none for waves past the last query
     const int wave_end = qw < a.T ? static_cast<int>((a.n0 + std::min<int64_t>(a.T, qw + 32) + kTile - 1) / kTile) : 0;
     // queries: B operand of S^T, k-step ks holds channels 16 ks + 8 half .. + 7
@@ -201,30 +206,24 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_kernel(const F
         (void*)a.kv.rope16, 0, static_cast<int>(a.kv.kp * kRope * 2), kBufferWord3);
     const __amdgpu_buffer_rsrc_t vres = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(a.kv.v16 + head_keys * kVh), 0, static_cast<int>(a.kv.kp * kVh * 2), kBufferWord3);
-    unsigned ksrc[4], vsrc[2];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        ksrc[j] = static_cast<unsigned>((lane >> 4) * (kNope * 2) + ((lane & 15) ^ (4 * j + (lane >> 4))) * 16);
-    }
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        vsrc[j] = static_cast<unsigned>((lane >> 3) * 128 + ((lane & 7) ^ (4 * j + (lane >> 4))) * 16);
-    }
+    // Load j of a run: the units of load 0 with bits 2 and 3 (4 j % 16) flipped.
+    const unsigned ksrc = static_cast<unsigned>((lane >> 4) * (kNope * 2) + ((lane & 15) ^ (lane >> 4)) * 16);
+    const unsigned vsrc = static_cast<unsigned>((lane >> 3) * 128 + ((lane & 7) ^ (lane >> 4)) * 16);
     auto issue = [&](int tile, char* ks, char* rs, char* vs) {
 #pragma unroll
         for (int j = 0; j < 16 / NW; ++j) {
             const int at = wave * (16 / NW) + j;  // a multiple of four, plus j
-            load_lds16(kres, ks + at * 1024, ksrc[j & 3], tile * kNopeBytes + at * 1024);
+            load_lds16(kres, ks + at * 1024, ksrc ^ (j & 3) * 64u, tile * kNopeBytes + at * 1024);
         }
 #pragma unroll
         for (int j = 0; j < 8 / NW; ++j) {
             const int at = wave * (8 / NW) + j;
-            load_lds16(rres, rs + at * 1024, vsrc[j & 1], tile * kRopeBytes + at * 1024);
+            load_lds16(rres, rs + at * 1024, vsrc ^ (j & 1) * 64u, tile * kRopeBytes + at * 1024);
         }
 #pragma unroll
         for (int j = 0; j < 16 / NW; ++j) {
             const int at = wave * (16 / NW) + j;
-            load_lds16(vres, vs + at * 1024, vsrc[j & 1], tile * kValueBytes + at * 1024);
+            load_lds16(vres, vs + at * 1024, vsrc ^ (j & 1) * 64u, tile * kValueBytes + at * 1024);
         }
     };
     f32x16 o[kVh / 32] = {};
@@ -339,9 +338,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_kernel(const F
             context(fb);
         }
     };
-    if (tile0 < tile_end) {
-        issue(tile0, k0, r0, v0);
-    }
+    issue(tile0, k0, r0, v0);
     for (int tb = tile0; tb < tile_end; tb += 2) {
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
@@ -416,13 +413,16 @@ __global__ __launch_bounds__(256) void flash_combine_kernel(const FlashArgs a) {
     const int h = static_cast<int>(i - t * a.heads);
     const int64_t step = a.heads * a.T;
     const int64_t at = h * a.T + t;
+    // splits that the token's block of queries has keys in
+    const int64_t keys = a.n0 + std::min<int64_t>(a.T, (t / kBlock + 1) * kBlock);
+    const int splits = static_cast<int>(((keys + kTile - 1) / kTile + a.split_tiles - 1) / a.split_tiles);
     float m = -__builtin_inff();
-    for (int k = 0; k < a.splits; ++k) {
+    for (int k = 0; k < splits; ++k) {
         m = fmaxf(m, a.part_ml[2 * (at + k * step)]);
     }
     f32x4 o = {};
     float l = 0.0f;
-    for (int k = 0; k < a.splits; ++k) {
+    for (int k = 0; k < splits; ++k) {
         const float w = __builtin_amdgcn_exp2f((a.part_ml[2 * (at + k * step)] - m) * a.c);
         l = __builtin_fmaf(w, a.part_ml[2 * (at + k * step) + 1], l);
         const f32x4 p = *reinterpret_cast<const f32x4*>(a.part_o + (at + k * step) * kVh + 4 * lane);
@@ -440,32 +440,25 @@ __global__ __launch_bounds__(256) void flash_combine_kernel(const FlashArgs a) {
     *reinterpret_cast<half4*>(a.ctx16 + panel_index(a.row0 + t, h * kVh + 4 * lane, a.ctx_rows)) = out;
 }
 
-template <int NW>
-hipError_t launch_flash_nw(const FlashArgs& a, hipStream_t s) {
-    const int64_t grid = (a.heads + 7) / 8 * 8 * static_cast<int64_t>(a.qblocks) * a.splits;
-    if (grid > INT32_MAX) {
-        return hipErrorInvalidValue;
-    }
-    if (a.splits > 1) {
-        hipLaunchKernelGGL((flash_kernel<NW, true>), dim3(static_cast<unsigned>(grid)), dim3(64 * NW), 0, s, a);
-    } else {
-        hipLaunchKernelGGL((flash_kernel<NW, false>), dim3(static_cast<unsigned>(grid)), dim3(64 * NW), 0, s, a);
-    }
-    return hipGetLastError();
-}
-
 }  // namespace
 
 bool flash_supported(const AttnShape& a) { return a.nope == kNope && a.rope == kRope && a.vh == kVh; }
 
 int64_t flash_keys(int64_t keys) { return round_up(keys, kTile); }
 
+// Splits while the query blocks leave CUs idle, of at least four tiles on
+// average (a causal block sees half of the call's own keys).  Measured (V2-Lite,
+// 16 heads; us for 1 / 2 / 4 / 8 splits): 16 tokens after 4000 78 / 46 / 28 / 22,
+// 256 after 3000 72 / 45 / 30 / 26, 512 after 3000 77 / 48 / 34 / 37, 512 alone
+// 15 / 17 / 18 / 21, 1024 after 1000 48 / 37 / 37 / 45, 2048 alone 49 / 52 / 50 /
+// 57.  Workgroups of one or two waves were slower throughout (512 alone 17 with
+// two): a tile is staged for fewer query tokens.
 FlashPlan flash_plan(int32_t heads, int64_t tokens, int64_t keys) {
     FlashPlan p;
-    p.waves = tokens >= 1024 ? 4 : tokens > 32 ? 2 : 1;
     const int64_t tiles = (keys + kTile - 1) / kTile;
-    const int64_t blocks = heads * ((tokens + 32 * p.waves - 1) / (32 * p.waves));
-    const int64_t want = std::min<int64_t>({16, (256 + blocks - 1) / blocks, tiles / 4});
+    const int64_t blocks = heads * ((tokens + kBlock - 1) / kBlock);
+    const int64_t mean = (keys - tokens / 2) / kTile;
+    const int64_t want = std::min<int64_t>({16, 256 / blocks, mean / 4});
     p.split_tiles = want > 1 ? static_cast<int32_t>((tiles + want - 1) / want) : 0;
     p.splits = p.split_tiles > 0 ? static_cast<int32_t>((tiles + p.split_tiles - 1) / p.split_tiles) : 1;
     return p;
@@ -504,13 +497,21 @@ hipError_t launch_flash(const AttnShape& a, const FlashPlan& p, const _Float16* 
     f.row0 = row0;
     f.ctx_rows = ctx_rows;
     f.heads = a.heads;
-    f.qblocks = static_cast<int32_t>((T + 32 * p.waves - 1) / (32 * p.waves));
+    f.qblocks = static_cast<int32_t>((T + kBlock - 1) / kBlock);
     f.splits = p.splits;
     f.split_tiles = p.split_tiles;
     f.c = scale * 1.4426950408889634f;
-    hipError_t err = p.waves == 4 ? launch_flash_nw<4>(f, s) : p.waves == 2 ? launch_flash_nw<2>(f, s)
-                                                                           : launch_flash_nw<1>(f, s);
-    if (err != hipSuccess || p.splits == 1) {
+    const int64_t grid = (f.heads + 7) / 8 * 8 * static_cast<int64_t>(f.qblocks) * f.splits;
+    if (grid > INT32_MAX) {
+        return hipErrorInvalidValue;
+    }
+    if (f.splits == 1) {
+        hipLaunchKernelGGL(flash_kernel<false>, dim3(static_cast<unsigned>(grid)), dim3(64 * NW), 0, s, f);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL(flash_kernel<true>, dim3(static_cast<unsigned>(grid)), dim3(64 * NW), 0, s, f);
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess) {
         return err;
     }
     hipLaunchKernelGGL(flash_combine_kernel, dim3(static_cast<unsigned>((T * a.heads + 7) / 8)), dim3(256), 0, s, f);

@@ -264,13 +264,21 @@ __global__ __launch_bounds__(256) void kv_prep16_kernel(const ProjArgs a, const 
     }
 }
 
-// Tile shape: 0: 64 x 64, 1: 128 x 128, 2: 128 x 256.
+// Tile shape (weight rows x tokens): 0: 64 x 64, 1: 64 x 128, 2: 128 x 128,
+// 3: 128 x 256.  The largest that still gives two thirds of the CUs a tile, and
+// 64 x 128 once the 64 x 64 tiles would queue up.  Measured (V2-Lite, us for
+// shapes 0 / 1 / 2 / 3): q and kv_a, 256 tokens 10.6 / 14 / 20 / 33, 777 27 / 24
+// / 23 / 36, 2048 74 / 54 / 43 / 42, 4096 143 / 144 / 89 / 77; o_proj, 512 tokens
+// 8.8 / 11 / 15 / 24, 1024 15 / 13 / 16 / 25, 2048 39 / 24 / 20 / 28.
 int proj_shape(int64_t rows, int64_t tokens) {
     auto tiles = [&](int64_t m, int64_t n) { return ((rows + m - 1) / m) * ((tokens + n - 1) / n); };
-    if (tiles(128, 256) >= 448) {
+    if (tiles(128, 256) >= 170) {
+        return 3;
+    }
+    if (tiles(128, 128) >= 170) {
         return 2;
     }
-    return tiles(128, 128) >= 256 ? 1 : 0;
+    return tiles(64, 64) > 384 ? 1 : 0;
 }
 
 template <int SHAPE, int WM, int WN, int MI, int NJ, int STAGES>
@@ -306,14 +314,15 @@ hipError_t launch_proj(const ProjArgs& a, hipStream_t s) {
         }
         rows += seg.rows;
     }
-    const int shape = proj_shape(rows, a.tokens);
-    switch (shape) {
+    switch (proj_shape(rows, a.tokens)) {
         case 0:
             return launch_proj_shape<0, 2, 2, 1, 1, 6>(a, s);
         case 1:
-            return launch_proj_shape<1, 2, 2, 2, 2, 4>(a, s);
+            return launch_proj_shape<1, 2, 2, 1, 2, 5>(a, s);
+        case 2:
+            return launch_proj_shape<2, 2, 2, 2, 2, 4>(a, s);
         default:
-            return launch_proj_shape<2, 2, 2, 2, 4, 3>(a, s);
+            return launch_proj_shape<3, 2, 2, 2, 4, 3>(a, s);
     }
 }
 

@@ -555,7 +555,6 @@ struct FlashKv {
     int64_t kp;
 };
 struct FlashPlan {
-    int32_t waves = 4;        // 32-token waves per workgroup
     int32_t splits = 1;       // workgroups that share a query block's keys
     int32_t split_tiles = 0;  // 64-key tiles of each (several splits)
 };

@@ -50,14 +50,14 @@ def _reference(m, x, cached, rotated=True):
 
 
 @pytest.mark.parametrize("heads,cached,T", [
-    (16, 0, 16),      # one wave per workgroup, half of it past the last token
-    (16, 5, 33),      # two waves, one token in the second
-    (16, 63, 65),     # the diagonal crosses tiles, a third wave block
+    (16, 0, 16),      # one wave, half of it past the last token
+    (16, 5, 33),      # one token in the second wave
+    (16, 63, 65),     # the diagonal crosses tiles, a third wave
     (3, 0, 97),       # heads that are no multiple of the eight XCDs
     (16, 2048, 16),   # keys split over workgroups
     (16, 1500, 40),   # split, ragged last tile, queries masked in whole tiles
-    (5, 0, 1029),     # four waves, last block of five tokens
-    (16, 130, 1100),  # four waves after cached tokens
+    (5, 0, 1029),     # nine query blocks, the last of five tokens
+    (16, 130, 1100),  # nine query blocks after cached tokens
 ])
 def test_flash_core(heads, cached, T):
     from litemind_amd import PATH_MFMA

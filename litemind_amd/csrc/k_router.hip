@@ -470,7 +470,7 @@ __global__ __launch_bounds__(kDecodeThreads) void router_decode_kernel(RouterArg
 // chains.  Each chunk of 64 gate rows (16 KB of the [H/4][E][4] layout: lane e
 // reads four consecutive rows of its expert with one ds_read_b128) and the
 // tokens' activations for those rows go from global memory straight into a
-// 4-deep LDS ring with global_load_lds, so three chunks are always in flight
+// 4-deep LDS ring with buffer loads, so three chunks are always in flight
 // behind the one the chains consume; every step waits for a constant count and
 // always issues (a chunk past the end reloads the last one into a buffer that
 // is never read), so the waits stay exact.  The selection uses the LDS variant.
@@ -521,6 +521,18 @@ __device__ inline void route_token_lds(float logit, bool valid, int lane, int64_
     }
 }
 
+// Direct-to-LDS buffer loads (not templates: the host pass checks a template's
+// builtin against its own target, which lacks the 16-byte form).  A buffer
+// load, unlike a global load to LDS, is not a pending flat access, after which
+// every wait for an LDS read waits for all of them.
+__device__ inline void router_load16(__amdgpu_buffer_rsrc_t from, char* to, unsigned offset, unsigned base) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (router_lds_void*)to, 16, offset, static_cast<int>(base), 0, 0);
+}
+__device__ inline void router_load4(__amdgpu_buffer_rsrc_t from, char* to, unsigned offset, unsigned base) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (router_lds_void*)to, 4, offset, static_cast<int>(base), 0, 0);
+}
+constexpr int kRouterBufferWord3 = 0x00020000;  // buffer descriptor word 3, raw 32-bit access
+
 template <int TPW, int NW, int DEPTH>
 __global__ __launch_bounds__(NW * 64) void router_wide_kernel(RouterArgs a, const float* __restrict__ x,
                                                                const float* __restrict__ wq4) {
@@ -532,7 +544,7 @@ __global__ __launch_bounds__(NW * 64) void router_wide_kernel(RouterArgs a, cons
     __shared__ __attribute__((aligned(1024))) char r4[kS4], r5[kS4], r6[kS4], r7[kS4];
     char* const ring[8] = {r0, r1, r2, r3, r4, r5, r6, r7};
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const int H = a.hidden;
     const int64_t tb0 = static_cast<int64_t>(blockIdx.x) * NW * TPW;
     const int nchunks = H / kWideRows;
@@ -544,28 +556,29 @@ __global__ __launch_bounds__(NW * 64) void router_wide_kernel(RouterArgs a, cons
     // branch.  With 8 waves, row lane of each of the wave's tokens.
     int64_t xt = tb0 + wave * TPW + (NW == 4 ? ((lane >> 4) % TPW) : 0);
     xt = xt < a.tokens ? xt : a.tokens - 1;
-    const float* xsrc = x + xt * H + (NW == 4 ? 4 * (lane & 15) : lane);
-    const float* wsrc = wq4 + static_cast<int64_t>(wave) * 256 + 4 * lane;
+    const int64_t rows = std::min<int64_t>(NW * TPW, a.tokens - tb0);
+    const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(x + tb0 * H), 0, static_cast<int>(rows * H * 4), kRouterBufferWord3);
+    const __amdgpu_buffer_rsrc_t wres =
+        __builtin_amdgcn_make_buffer_rsrc((void*)wq4, 0, H * 64 * 4, kRouterBufferWord3);
+    const unsigned xsrc = static_cast<unsigned>(((xt - tb0) * H + (NW == 4 ? 4 * (lane & 15) : lane)) * 4);
+    const unsigned wsrc = static_cast<unsigned>((wave * 256 + 4 * lane) * 4);
     auto issue = [&](int c, char* buf) {
         c = c < nchunks ? c : nchunks - 1;
-        const int64_t i0 = static_cast<int64_t>(c) * kWideRows;
+        const unsigned i0 = static_cast<unsigned>(c) * kWideRows;
 #pragma unroll
         for (int j = 0; j < S::kWLoads; ++j) {
             const int n = j * NW + wave;  // 1 KB block n of the chunk's gate rows
-            __builtin_amdgcn_global_load_lds((router_global_void*)(wsrc + i0 * 64 + j * NW * 256),
-                                             (router_lds_void*)(buf + n * 1024), 16, 0, 0);
+            router_load16(wres, buf + n * 1024, wsrc, i0 * 256 + j * NW * 1024);
         }
         if constexpr (NW == 4) {
-            __builtin_amdgcn_global_load_lds((router_global_void*)(xsrc + i0),
-                                             (router_lds_void*)(buf + S::kWBytes + wave * S::kXWave), 16, 0, 0);
+            router_load16(xres, buf + S::kWBytes + wave * S::kXWave, xsrc, i0 * 4);
         } else {
             // token k of the wave: tokens past the batch end repeat the last one
 #pragma unroll
             for (int k = 0; k < TPW; ++k) {
-                const int64_t step = tb0 + wave * TPW + k < a.tokens ? static_cast<int64_t>(k) * H : 0;
-                __builtin_amdgcn_global_load_lds((router_global_void*)(xsrc + step + i0),
-                                                 (router_lds_void*)(buf + S::kWBytes + wave * S::kXWave + k * 256), 4,
-                                                 0, 0);
+                const unsigned step = tb0 + wave * TPW + k < a.tokens ? static_cast<unsigned>(k * H * 4) : 0;
+                router_load4(xres, buf + S::kWBytes + wave * S::kXWave + k * 256, xsrc, step + i0 * 4);
             }
         }
     };
@@ -575,69 +588,104 @@ __global__ __launch_bounds__(NW * 64) void router_wide_kernel(RouterArgs a, cons
     for (int k = 0; k < TPW; ++k) {
         acc[k] = 0.0f;
     }
-    // Rows 4q .. 4q + 3 of a chunk: the four gate values of this lane's expert
-    // (one 16-byte read) and the activations of its tokens (broadcast reads).
-    // The reads of a batch of kBatch rows are issued together and the
-    // additions then run from registers: while LDS-DMA writes are pending the
-    // compiler can only wait for all LDS reads at once, so one wait per batch
-    // is the cheapest arrangement.
+    // Rows 4q .. 4q + 3 of a batch of kBatch: the four gate values of this lane's
+    // expert (one 16-byte read) and the activations of its tokens (broadcast
+    // reads).
     constexpr int kBatch = 32;
-    auto compute = [&](const char* buf) {
+    struct Batch {
+        float4 w[kBatch / 4];
+        float4 x[kBatch / 4][TPW];
+    };
+    auto read = [&](const char* buf, int r0, Batch& b) {
         const float4* wb = reinterpret_cast<const float4*>(buf);
         const float* xb = reinterpret_cast<const float*>(buf + S::kWBytes + wave * S::kXWave);
 #pragma unroll
-        for (int r0 = 0; r0 < kWideRows; r0 += kBatch) {
-            float4 w[kBatch / 4];
-            float4 xv[kBatch / 4][TPW];
+        for (int q = 0; q < kBatch / 4; ++q) {
+            b.w[q] = wb[(r0 / 4 + q) * 64 + lane];
 #pragma unroll
-            for (int q = 0; q < kBatch / 4; ++q) {
-                w[q] = wb[(r0 / 4 + q) * 64 + lane];
-#pragma unroll
-                for (int k = 0; k < TPW; ++k) {
-                    xv[q][k] = *reinterpret_cast<const float4*>(xb + k * kWideRows + r0 + 4 * q);
-                }
+            for (int k = 0; k < TPW; ++k) {
+                b.x[q][k] = *reinterpret_cast<const float4*>(xb + k * kWideRows + r0 + 4 * q);
             }
-#pragma unroll
-            for (int q = 0; q < kBatch / 4; ++q) {
-                // Products first (independent), then the TPW chains' additions
-                // interleaved so consecutive adds never depend on each other.
-                float p[4][TPW];
-#pragma unroll
-                for (int k = 0; k < TPW; ++k) {
-                    p[0][k] = w[q].x * xv[q][k].x;
-                    p[1][k] = w[q].y * xv[q][k].y;
-                    p[2][k] = w[q].z * xv[q][k].z;
-                    p[3][k] = w[q].w * xv[q][k].w;
-                }
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-#pragma unroll
-                    for (int k = 0; k < TPW; ++k) {
-                        acc[k] = acc[k] + p[j][k];
-                    }
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
         }
     };
-    // Chunk c lives in ring[c % depth]; before consuming it, wait until at
-    // most the depth - 2 chunks issued after it are in flight (and this wave's
-    // LDS reads of the previous chunk are done); the barrier then also frees the
-    // buffer consumed in the previous step for chunk c + depth - 1.
-    constexpr int kVm = (DEPTH - 2) * S::kLoads;
-    static_assert(kVm < 64, "vmcnt immediate");
-    constexpr int kWait = 0x0070 | (kVm & 15) | ((kVm >> 4) << 14);  // vmcnt(kVm) lgkmcnt(0)
+    auto add = [&](const Batch& b) {
+#pragma unroll
+        for (int q = 0; q < kBatch / 4; ++q) {
+            // Products first (independent), then the TPW chains' additions
+            // interleaved so consecutive adds never depend on each other.
+            float p[4][TPW];
+#pragma unroll
+            for (int k = 0; k < TPW; ++k) {
+                p[0][k] = b.w[q].x * b.x[q][k].x;
+                p[1][k] = b.w[q].y * b.x[q][k].y;
+                p[2][k] = b.w[q].z * b.x[q][k].z;
+                p[3][k] = b.w[q].w * b.x[q][k].w;
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+#pragma unroll
+                for (int k = 0; k < TPW; ++k) {
+                    acc[k] = acc[k] + p[j][k];
+                }
+            }
+        }
+    };
+    // Chunk c lives in ring[c % depth]; a wait leaves the chunks issued after
+    // the awaited one in flight; the barrier after it also frees the buffer of
+    // the chunk that every wave has consumed, for chunk c + depth - 1.
+    constexpr auto wait_imm = [](int chunks) {  // vmcnt, lgkmcnt unconstrained
+        return 0x0070 | 0x0F00 | ((chunks * S::kLoads) & 15) | (((chunks * S::kLoads) >> 4) << 14);
+    };
+    static_assert((DEPTH - 2) * S::kLoads < 64, "vmcnt immediate");
 #pragma unroll
     for (int d = 0; d < DEPTH - 1; ++d) {
         issue(d, ring[d]);
     }
-    for (int c0 = 0; c0 < nchunks; c0 += DEPTH) {
+    if constexpr (TPW == 1) {
+        // One chain per lane: each batch is read while the one before it is
+        // added, also across chunks, so the chain does not wait for LDS.
+        // V2-Lite router alone: 509 tokens 25.6 us with one wait per batch (global
+        // loads to LDS), 22.7 so; 2048 tokens 31.9 and 28.5; 4096 (two tokens per
+        // wave, the path below with buffer loads) 52.0 and 49.8.
+        static_assert(kWideRows == 2 * kBatch);
+        Batch even, odd;
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(wait_imm(DEPTH - 2));
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        read(ring[0], 0, even);
+        for (int c0 = 0; c0 < nchunks; c0 += DEPTH) {
 #pragma unroll
-        for (int j = 0; j < DEPTH; ++j) {
-            __builtin_amdgcn_s_waitcnt(kWait);
-            __builtin_amdgcn_s_barrier();
-            issue(c0 + j + DEPTH - 1, ring[(j + DEPTH - 1) % DEPTH]);
-            compute(ring[j]);
+            for (int j = 0; j < DEPTH; ++j) {
+                read(ring[j], kBatch, odd);
+                __builtin_amdgcn_sched_barrier(0);
+                add(even);
+                __builtin_amdgcn_sched_barrier(0);
+                __builtin_amdgcn_s_waitcnt(wait_imm(DEPTH - 3));  // chunk c0 + j + 1 is in
+                __builtin_amdgcn_s_barrier();
+                __builtin_amdgcn_sched_barrier(0);
+                issue(c0 + j + DEPTH - 1, ring[(j + DEPTH - 1) % DEPTH]);
+                read(ring[(j + 1) % DEPTH], 0, even);
+                __builtin_amdgcn_sched_barrier(0);
+                add(odd);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    } else {
+        for (int c0 = 0; c0 < nchunks; c0 += DEPTH) {
+#pragma unroll
+            for (int j = 0; j < DEPTH; ++j) {
+                __builtin_amdgcn_s_waitcnt(wait_imm(DEPTH - 2) & ~0x0F00);  // and this wave's reads are done
+                __builtin_amdgcn_s_barrier();
+                issue(c0 + j + DEPTH - 1, ring[(j + DEPTH - 1) % DEPTH]);
+                Batch b;
+#pragma unroll
+                for (int r0 = 0; r0 < kWideRows; r0 += kBatch) {
+                    read(ring[j], r0, b);
+                    add(b);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
         }
     }
     __builtin_amdgcn_s_waitcnt(0x0070);  // drain the clamped reloads
@@ -645,19 +693,31 @@ __global__ __launch_bounds__(NW * 64) void router_wide_kernel(RouterArgs a, cons
 
     // With a.x16, the fp16 panel copy of the wave's tokens for the MFMA path
     // (to_f16_rows_kernel's conversion), from rows the loop above has just
-    // brought into L2.  After the loop: a global store inside it makes the
-    // compiler keep far more registers live (256 VGPRs + 256 AGPRs against 100).
+    // brought into L2, eight loads of a token in flight.  After the loop: a
+    // global store inside it makes the compiler keep far more registers live
+    // (256 VGPRs + 256 AGPRs against 100).
     if (a.x16 != nullptr) {
         typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 #pragma unroll
         for (int k = 0; k < TPW; ++k) {
             const int64_t t = tb0 + wave * TPW + k;
             if (t < a.tokens) {
-                for (int c = 4 * lane; c < H; c += 256) {
-                    const float4 v = *reinterpret_cast<const float4*>(x + t * H + c);
-                    *reinterpret_cast<half4_t*>(a.x16 + panel_index(t, c, a.tokens)) =
-                        half4_t{static_cast<_Float16>(v.x), static_cast<_Float16>(v.y), static_cast<_Float16>(v.z),
-                                static_cast<_Float16>(v.w)};
+                for (int c0 = 4 * lane; c0 < H; c0 += 8 * 256) {
+                    float4 v[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) {
+                        const int c = c0 + 256 * u;
+                        v[u] = *reinterpret_cast<const float4*>(x + t * H + (c < H ? c : c0));
+                    }
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) {
+                        const int c = c0 + 256 * u;
+                        if (c < H) {
+                            *reinterpret_cast<half4_t*>(a.x16 + panel_index(t, c, a.tokens)) =
+                                half4_t{static_cast<_Float16>(v[u].x), static_cast<_Float16>(v[u].y),
+                                        static_cast<_Float16>(v[u].z), static_cast<_Float16>(v[u].w)};
+                        }
+                    }
                 }
             }
         }

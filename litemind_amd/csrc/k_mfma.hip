@@ -387,20 +387,27 @@ bool offsets_fit(const ExpertArgs& a) {
 enum class TileShape { kThin, kNarrow, kWide };
 
 // Which tile a launch takes.  Routed layers stream every active expert's
-// weights: while the average group fits half a 64-row tile the finer 64 x 128
-// tiles leave a smaller last round (V2-Lite, gate/up and down back to back:
-// 8 tokens 128 us against 139 with 64 x 256 tiles, 16 167 / 182, 128 209 / 213,
-// 256 221 / 231, 509 255 / 245); up to one 64-row tile 64 x 256; past that
+// weights, in 64 x 256 tiles up to one 64-row tile per average group; past that
 // every extra 64-row tile would stream the weights again (768 tokens and more:
-// 4 to 13% slower).  A layer without routed experts is one group of T rows
-// with few column blocks: its gate/up (V2-Lite's dense layer, 8 / 137 / 256
-// tokens) takes 17 / 35 / 43 us with 64 x 128 tiles, 25 / 29 / 47 with 64 x 256
-// and 32 / 37 / 39 with 128 x 256; its down, with K split, 10 / 17 / 21 (64 x
-// 128), 11 / 18 / 20, 11 / 19 / 22, and 35 against 30 us at 512 tokens.
+// 4 to 13% slower than 128 x 256).  Where that is only a round or two of
+// workgroups (down tiles of the active experts against 512 slots) the finer
+// 64 x 128 tiles leave a smaller last round, as long as the groups are small
+// (whole V2-Lite layer, 64 x 256 against 64 x 128: 16 tokens 163 / 156 us, 32
+// 186 / 180, 64 204 / 198, 100 203 / 202, 150 209 / 209, 256 220 / 223, 341 230
+// / 239; DeepSeek-V2's, 4 tokens 212 / 204, 16 (four rounds) 582 / 591).
+// A layer without routed experts is one group of T rows with few column blocks:
+// its gate/up (V2-Lite's dense layer, 8 / 137 / 256 tokens) takes 17 / 35 / 43
+// us with 64 x 128 tiles, 25 / 29 / 47 with 64 x 256 and 32 / 37 / 39 with 128 x
+// 256; its down, with K split, 10 / 17 / 21 (64 x 128), 11 / 18 / 20, 11 / 19 /
+// 22, and 35 against 30 us at 512 tokens.
 TileShape tile_shape(const ExpertArgs& a, int mode) {
     if (a.experts > 0) {
         const int64_t rows = a.tokens * a.top_k;
-        return rows <= 32 * a.experts ? TileShape::kThin : rows <= 64 * a.experts ? TileShape::kNarrow : TileShape::kWide;
+        const int64_t groups = std::min<int64_t>(rows, a.experts);
+        if (rows <= 8 * a.experts && groups * ((a.hidden + 255) / 256) <= 1024) {
+            return TileShape::kThin;
+        }
+        return rows <= 64 * a.experts ? TileShape::kNarrow : TileShape::kWide;
     }
     if (mode == kGateUp) {
         return a.tokens <= 64 ? TileShape::kThin : a.tokens <= 192 ? TileShape::kNarrow : TileShape::kWide;

@@ -53,9 +53,9 @@ def test_dense_shapes(dense, T):
     assert mx <= MAX_ABS and rel <= MEAN_REL
 
 
-# 16 experts, top-4: 64-row tiles of 128 columns up to 128 tokens, of 256 up to
+# 16 experts, top-4: 64-row tiles of 128 columns up to 32 tokens, of 256 up to
 # 256, 128-row tiles above; three shared experts chunk their K in three
-@pytest.mark.parametrize("T", [5, 128, 129, 256, 257])
+@pytest.mark.parametrize("T", [5, 32, 33, 256, 257])
 def test_routed_shapes(T):
     from litemind_amd import PATH_MFMA, Context
     from litemind_amd import workload as wl
@@ -79,3 +79,28 @@ def test_routed_shapes(T):
     mx, rel = layer_error(y, want)
     print(f"routed T={T}: max_abs={mx:.3e} mean_rel={rel:.3e}")
     assert mx <= MAX_ABS and rel <= MEAN_REL
+
+
+# heads of other widths than the one-launch core's run the projections and the
+# core as GEMMs of the same grouped kernel: split K with few tiles, 64 x 128 and
+# 128 x 256 tiles
+@pytest.mark.parametrize("q_lora,T", [(0, 40), (96, 40), (0, 300)])
+def test_attention_other_head_widths(q_lora, T):
+    from litemind_amd import PATH_MFMA
+    from litemind_amd import workload as wl
+    from test_gpu_attention import ATT_MAX_ABS, ATT_MEAN_REL, Mla, tokens
+    d = dataclasses.replace(wl.V2_LITE_MLA, hidden=512, heads=4, q_lora_rank=q_lora, kv_lora_rank=256, qk_nope=64,
+                            qk_rope=32, v_head=96, max_positions=T + 8)
+    announce(f"attention MFMA path, other head widths q_lora={q_lora} T={T}")
+    m = Mla(d, 401, path=PATH_MFMA)
+    try:
+        x = tokens(402, T + 5, d.hidden)
+        for lo, hi in ((0, 5), (5, T + 5)):
+            y = m.forward(x[lo:hi], lo)
+            want, n = m.oracle(x[lo:hi], lo)
+            assert n == hi - lo
+            mx, rel = layer_error(y, want)
+            print(f"q_lora={q_lora} {lo}..{hi}: max_abs={mx:.3e} mean_rel={rel:.3e}")
+            assert mx <= ATT_MAX_ABS and rel <= ATT_MEAN_REL
+    finally:
+        m.close()

@@ -903,7 +903,7 @@ __global__ __launch_bounds__(256) void context_kernel(const float* __restrict__ 
 // zeros).  A workgroup is 16 tokens x 64 channels of one head, a wave 16
 // channels; the probabilities pass through LDS in chunks, the values come from
 // L2 kCtxMAhead steps ahead.  Bound by the chains' latency.  V2-Lite: 2 tokens
-// after 1000 58 us for the whole call before, 36 after.
+// after 1000 58 us for the whole call before, 39 after.
 constexpr int kCtxMTokens = 16;
 constexpr int kCtxMKeys = 512;                  // keys of a chunk
 constexpr int kCtxMStride = kCtxMKeys + 4;      // floats per token's row: 16 rows x 4 keys on 64 banks

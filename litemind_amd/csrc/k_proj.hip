@@ -14,9 +14,9 @@
 // one token and groups of four successive channels: rotary pairs meet in a
 // lane, and the key cache (channel-major) is written 32 tokens at a time.
 // Projections of the same input run as segments of one launch.  There is no
-// split of K: tiles of 64 x 64 keep a prompt of a few hundred tokens on all
-// CUs instead (q and kv_a at 512 tokens: 456 tiles), which saves the partial
-// sums' round trip and the launch that adds them.
+// split of K: small tiles keep a prompt of a few hundred tokens on all CUs
+// instead (q and kv_a at 256 tokens: 228 tiles of 64 x 64), which saves the
+// partial sums' round trip and the launch that adds them.
 #include "lm_internal.h"
 #include "mfma_tile.h"
 

@@ -342,7 +342,7 @@ int project(const AttnLayer& L, int proj, const uint16_t* w, const float* x, int
 //   x -> fp16 | q and kv_a | norm, rotary key | kv_b into cache and copies |
 //   core | o_proj
 // Before, a 512-token V2-Lite prompt took 22 launches on two streams: 108 us
-// against 39, 4096 tokens 1196 us against 263.
+// against 32, 4096 tokens 1186 us against 258.
 int attention_prompt(AttnState* st, hipStream_t stream, AttnLayer& L, const CorePlan& plan, const float* x, int64_t F,
                      int64_t pos0, float* out, int32_t accumulate, const float* in_norm) {
     const lm_mla_config& c = st->cfg;

@@ -639,7 +639,14 @@ hipError_t launch_head(const uint16_t* w, const float* x, float* logits, HeadBes
         return hipErrorInvalidValue;
     }
     int64_t blocks = (rows + kRows - 1) / kRows;
-    if (tokens > kHeadTokens) {
+    // The few-token kernel keeps the tokens' rows in LDS.  Where two to four do
+    // not fit (widths above 4096), the tiles take them in one launch:
+    // [102400, 5120], 4 tokens, 217 us (466 as three tokens and one).
+    const size_t lds = sizeof(float) * static_cast<size_t>(tokens) * static_cast<size_t>(in_dim);
+    if (tokens > kHeadTokens || lds > 64 * 1024) {
+        if (!exact_supported(in_dim)) {
+            return hipErrorInvalidValue;
+        }
         const hipError_t err = launch_exact(w, x, logits, token != nullptr ? partial : nullptr, &blocks, rows, in_dim,
                                             tokens, 1.0f, 0, s);
         if (err != hipSuccess || token == nullptr) {
@@ -648,10 +655,6 @@ hipError_t launch_head(const uint16_t* w, const float* x, float* logits, HeadBes
         hipLaunchKernelGGL(argmax_first_kernel, dim3(static_cast<unsigned>(tokens)), dim3(1024), 0, s, partial,
                            static_cast<int32_t>(blocks), logits, rows, token);
         return hipGetLastError();
-    }
-    const size_t lds = sizeof(float) * static_cast<size_t>(tokens) * static_cast<size_t>(in_dim);
-    if (lds > 64 * 1024) {
-        return hipErrorInvalidValue;
     }
     hipLaunchKernelGGL(head_logits_kernel<kThreads>, dim3(static_cast<unsigned>(blocks)), dim3(kThreads), lds, s, w,
                        x, logits, partial, rows, in_dim, tokens, 1.0f, 0);

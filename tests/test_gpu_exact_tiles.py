@@ -44,3 +44,27 @@ def test_head_batches_bit_exact(V, H, T, scale):
     assert np.array_equal(logits.view(np.uint32), want.view(np.uint32))
     assert token.tolist() == [int(np.argmax(want[t])) for t in range(T)]
     assert token2.tolist() == token.tolist()
+
+
+@pytest.mark.parametrize("V,H,T", [
+    (300, 5120, 4),    # four rows of 20 KB
+    (300, 5120, 68),   # 64 tokens, then four
+    (300, 7168, 3),
+    (300, 8192, 67),   # 64 tokens, then three
+    (65, 16384, 2),    # the widest head
+    (65, 4160, 4),     # not a multiple of 128: 32-token tiles
+])
+def test_few_tokens_at_wide_heads(V, H, T):
+    """Two to four tokens, alone or left over from a batch, whose rows exceed the 64 KB of LDS
+    that the few-token kernel keeps them in."""
+    from litemind_amd import Context
+
+    head, norm, hidden = _case(V + H + T, V, H, T)
+    announce(f"head few tokens V={V} H={H} T={T}")
+    with Context(_config(H)) as ctx:
+        ctx.upload_head(norm, head)
+        logits, token, token2 = _gpu(ctx, hidden, V)
+    want = _oracle(head, norm, hidden)
+    assert np.array_equal(logits.view(np.uint32), want.view(np.uint32))
+    assert token.tolist() == [int(np.argmax(want[t])) for t in range(T)]
+    assert token2.tolist() == token.tolist()

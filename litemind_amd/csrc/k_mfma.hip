@@ -415,6 +415,9 @@ TileShape tile_shape(const ExpertArgs& a, int mode) {
     return a.tokens <= 256 ? TileShape::kThin : TileShape::kWide;
 }
 
+// Chunks of the shared expert's K no longer than the routed experts'.
+int64_t routed_chunks(int64_t inter_p, int64_t shared_inter_p) { return inter_p > 0 ? shared_inter_p / inter_p : 1; }
+
 // K chunks of the shared group's down GEMM (hidden columns, K = shared_inter_p).
 // Without routed experts: while its tiles fill less than a round of workgroups
 // (two per CU for the thin tiles, one for the wide ones), at most `most` chunks
@@ -425,7 +428,7 @@ int32_t down_chunks(const ExpertArgs& a, int64_t most) {
     const int64_t nk = a.shared_inter_p / BK;
     int64_t ks = 1;
     if (a.experts > 0) {
-        ks = shape == TileShape::kThin && a.inter_p > 0 ? a.shared_inter_p / a.inter_p : 1;
+        ks = shape == TileShape::kThin ? routed_chunks(a.inter_p, a.shared_inter_p) : 1;
     } else {
         const bool wide = shape == TileShape::kWide;
         const int64_t tiles = (a.tokens + (wide ? 127 : 63)) / (wide ? 128 : 64) * ((a.hidden + (wide ? 255 : 127)) / (wide ? 256 : 128));
@@ -564,11 +567,17 @@ hipError_t launch_mfma_gateup(const ExpertArgs& a, hipStream_t s) { return launc
 
 hipError_t launch_mfma_down(const ExpertArgs& a, hipStream_t s) { return launch<kDown>(a, s); }
 
+int64_t down_rows(int64_t T, int64_t top_k, int64_t inter_p, int64_t shared_inter_p) {
+    const int64_t dense = std::min(kSplitChunks * T, std::max(T, kSplitRows));
+    const int64_t shared = T * std::max<int64_t>(1, routed_chunks(inter_p, shared_inter_p));
+    return std::max(dense, T * top_k + std::min(shared, dense));
+}
+
 int32_t mfma_shared_chunks(const ExpertArgs& a) {
     if (a.tokens <= 0 || !a.has_shared || a.shared_inter_p < BK) {
         return 1;
     }
-    return down_chunks(a, std::min<int64_t>(8, kSplitRows / a.tokens));
+    return down_chunks(a, std::min<int64_t>(kSplitChunks, kSplitRows / a.tokens));
 }
 
 }  // namespace lm

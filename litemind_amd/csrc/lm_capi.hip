@@ -392,8 +392,8 @@ int ensure_workspace(lm_context* ctx, int64_t tokens) {
     LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.slot_of), sizeof(int32_t) * static_cast<size_t>(TK)));
     LM_HIP(hipMalloc(&w.act, sizeof(float) * act_elems));
     LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.x16), sizeof(_Float16) * static_cast<size_t>(T * ctx->Hp)));
-    LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.down_out), 
-                     sizeof(float) * static_cast<size_t>((TK + std::max(T, lm::kSplitRows)) * ctx->H)));
+    LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.down_out),
+                     sizeof(float) * static_cast<size_t>(lm::down_rows(T, ctx->K, ctx->Ip, ctx->Sp) * ctx->H)));
     LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.xnorm), sizeof(float) * static_cast<size_t>(T * ctx->H)));
     LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.ffn), sizeof(float) * static_cast<size_t>(T * ctx->H)));
     LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.zero), sizeof(int32_t) * 4));

@@ -622,9 +622,15 @@ hipError_t launch_gemv_down(const ExpertArgs& a, int64_t max_groups, hipStream_t
 // Grouped SwiGLU on MFMA (k_mfma.hip): fp16 panel operands, fp32 accumulation.
 hipError_t launch_mfma_gateup(const ExpertArgs& a, hipStream_t s);
 hipError_t launch_mfma_down(const ExpertArgs& a, hipStream_t s);
-// The ksplit worth using for a layer, with T ksplit <= max(T, kSplitRows) so
-// that down_out needs max(T, kSplitRows) rows past the routed ones.
+// The ksplit worth using for a layer of T tokens: at most kSplitChunks, with T
+// ksplit <= max(T, kSplitRows).
+constexpr int64_t kSplitChunks = 8;
 constexpr int64_t kSplitRows = 4096;
+// Rows that down_out needs for calls of up to T tokens, of MoE layers and of a
+// dense one.  No more: with 4096 for the chunks whatever T is, a context's
+// first call of one token allocated 34 MB at hidden 2048, 84 MB at 5120, and
+// took 127 and 221 us against 92 and 130.
+int64_t down_rows(int64_t T, int64_t top_k, int64_t inter_p, int64_t shared_inter_p);
 int32_t mfma_shared_chunks(const ExpertArgs& a);
 // out [M, N] = a16 . W^T (accumulate: out += a16 . W^T) for a16 [M, Kp] and W
 // [N, Kp] fp16 panels (*w, a device pointer to the matrix), fp32 accumulation,

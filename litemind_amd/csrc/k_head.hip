@@ -41,6 +41,13 @@ __device__ inline HeadBest better(HeadBest a, HeadBest b) {
     return a;
 }
 
+// Row `row`'s candidate.  A NaN is none, except at index 0, which nothing after
+// it can replace: the largest value at the lowest index.
+__device__ inline HeadBest candidate(float logit, int64_t row, bool live) {
+    const bool nan = logit != logit;
+    return {nan && row == 0 ? __builtin_inff() : logit, static_cast<int32_t>(row), live && (!nan || row == 0) ? 1 : 0};
+}
+
 __device__ inline HeadBest wave_better(HeadBest b) {
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) {
@@ -55,7 +62,9 @@ __device__ inline HeadBest wave_better(HeadBest b) {
 // + 7), and a wave's load covers 64 contiguous bytes of 16 rows.  The tokens
 // (tokens x in_dim floats, dynamic LDS) are staged once per block.  Lane 0 of a
 // row also owns chains 0..7's continuation over the 8-wide remainder.  Then
-// each block's best row per token goes to `partial` (when given).
+// each block's best row per token goes to `partial` (when given; `logits` may
+// then be null: a [102400] head kept 26 MB for the logits of 64 tokens that a
+// caller did not ask for).
 template <int THREADS>
 __global__ __launch_bounds__(THREADS) void head_logits_kernel(const uint16_t* __restrict__ w,
                                                               const float* __restrict__ x, float* logits,
@@ -152,7 +161,7 @@ __global__ __launch_bounds__(THREADS) void head_logits_kernel(const uint16_t* __
         const float h2 = ls[2] + ls[6];
         const float h3 = ls[3] + ls[7];
         const float total = (h0 + h2) + (h1 + h3);
-        if (live && q == 0) {
+        if (live && q == 0 && logits != nullptr) {
             // gemm::matvec_bf16_accumulate folds the row as fma(scale, dot, out) (src/Gemm.cpp:156-175)
             float* o = logits + static_cast<int64_t>(t) * rows + row;
             *o = accumulate ? __builtin_fmaf(scale, total, *o) : total;
@@ -160,7 +169,7 @@ __global__ __launch_bounds__(THREADS) void head_logits_kernel(const uint16_t* __
         if (partial == nullptr) {
             continue;
         }
-        HeadBest b{total, static_cast<int32_t>(row), live && q == 0 && total == total ? 1 : 0};
+        HeadBest b = candidate(total, row, live && q == 0);
         b = wave_better(b);
         if (lane == 0) {
             wave_best[tid >> 6] = b;
@@ -455,14 +464,14 @@ __global__ __launch_bounds__(256, 2) void matvec_exact_kernel(const uint16_t* __
         const int r = M == 32 ? li : M * i + li;
         const int64_t row = row0 + r;
         const bool live = t < ntok && r < nrow;
-        if (live) {
+        if (live && (!BEST || out != nullptr)) {
             float* o = out + static_cast<int64_t>(t0 + t) * rows + row;
             *o = accumulate ? __builtin_fmaf(scale, total, *o) : total;
         }
         if constexpr (BEST) {
             // the tile's best row of each token: the M lanes that share it, then
             // (16-token tiles) one candidate per 16 rows
-            HeadBest b{total, static_cast<int32_t>(row), live && total == total ? 1 : 0};
+            HeadBest b = candidate(total, row, live);
 #pragma unroll
             for (int o = M / 2; o >= 1; o >>= 1) {
                 const HeadBest other{__shfl_xor(b.v, o), __shfl_xor(b.i, o), __shfl_xor(b.have, o)};
@@ -523,10 +532,8 @@ __global__ __launch_bounds__(256) void matvec_one_kernel(const uint16_t* __restr
 // Sampler::select_next's greedy branch over the blocks' candidates:
 // std::max_element keeps the first of equal values and moves only on a strictly
 // larger one, so a NaN never becomes the choice, except at index 0, which
-// nothing after it can replace.  That is the first maximum of the non-NaN
-// logits, or 0 when logit 0 is NaN.
+// nothing after it can replace (`candidate`).  0 when every logit is NaN.
 __global__ __launch_bounds__(1024) void argmax_first_kernel(const HeadBest* __restrict__ partial, int32_t blocks,
-                                                            const float* __restrict__ logits, int64_t vocab,
                                                             int32_t* out) {
     __shared__ HeadBest wave_best[16];
     const HeadBest* p = partial + static_cast<int64_t>(blockIdx.x) * blocks;
@@ -544,8 +551,7 @@ __global__ __launch_bounds__(1024) void argmax_first_kernel(const HeadBest* __re
         for (int k = 1; k < 16; ++k) {
             r = better(r, wave_best[k]);
         }
-        const float first = logits[static_cast<int64_t>(blockIdx.x) * vocab];
-        out[blockIdx.x] = (first != first || !r.have) ? 0 : r.i;
+        out[blockIdx.x] = r.have ? r.i : 0;
     }
 }
 
@@ -653,7 +659,7 @@ hipError_t launch_head(const uint16_t* w, const float* x, float* logits, HeadBes
             return err;
         }
         hipLaunchKernelGGL(argmax_first_kernel, dim3(static_cast<unsigned>(tokens)), dim3(1024), 0, s, partial,
-                           static_cast<int32_t>(blocks), logits, rows, token);
+                           static_cast<int32_t>(blocks), token);
         return hipGetLastError();
     }
     hipLaunchKernelGGL(head_logits_kernel<kThreads>, dim3(static_cast<unsigned>(blocks)), dim3(kThreads), lds, s, w,
@@ -663,7 +669,7 @@ hipError_t launch_head(const uint16_t* w, const float* x, float* logits, HeadBes
         return err;
     }
     hipLaunchKernelGGL(argmax_first_kernel, dim3(static_cast<unsigned>(tokens)), dim3(1024), 0, s, partial,
-                       static_cast<int32_t>(blocks), logits, rows, token);
+                       static_cast<int32_t>(blocks), token);
     return hipGetLastError();
 }
 

@@ -196,13 +196,11 @@ struct lm_context {
     float* gemm_out = nullptr;   // output
     size_t gemm_cap = 0;         // floats in each scratch buffer
     // LM head: final norm [H] fp32, head [V, H] BF16, and scratch for one group of
-    // lm::head_batch tokens (normalised hidden states, logits when the caller
-    // passes none)
+    // lm::head_batch tokens (normalised hidden states)
     float* head_norm = nullptr;
     uint16_t* head_w = nullptr;
     int64_t vocab = 0;
     float* head_x = nullptr;
-    float* head_logits = nullptr;
     lm::HeadBest* head_partial = nullptr;  // per-block candidates of the greedy choice
     lm::AttnState* attention = nullptr;  // lm_attention_configure: MLA weights, rotary tables, KV caches
     int32_t graphs = 0;  // live lm_stack_graph captures (they hold the workspace's pointers)
@@ -1142,7 +1140,6 @@ int lm_context_destroy(lm_context* ctx) {
     (void)hipFree(ctx->head_norm);
     (void)hipFree(ctx->head_w);
     (void)hipFree(ctx->head_x);
-    (void)hipFree(ctx->head_logits);
     (void)hipFree(ctx->head_partial);
     (void)hipFree(ctx->d_overflow);
     (void)hipFree(ctx->d_inexact);
@@ -1388,21 +1385,18 @@ int lm_upload_head(lm_context* ctx, const float* norm_host, const uint16_t* head
         ctx->resident -= sizeof(uint16_t) * static_cast<size_t>(ctx->vocab) * H + sizeof(float) * H;
     }
     for (void* q : {static_cast<void*>(ctx->head_norm), static_cast<void*>(ctx->head_w),
-                    static_cast<void*>(ctx->head_x), static_cast<void*>(ctx->head_logits),
-                    static_cast<void*>(ctx->head_partial)}) {
+                    static_cast<void*>(ctx->head_x), static_cast<void*>(ctx->head_partial)}) {
         LM_HIP(hipFree(q));
     }
     ctx->head_norm = nullptr;
     ctx->head_w = nullptr;
     ctx->head_x = nullptr;
-    ctx->head_logits = nullptr;
     ctx->head_partial = nullptr;
     ctx->vocab = 0;
     const size_t batch = static_cast<size_t>(lm::head_batch(ctx->H));
     LM_HIP(hipMalloc(reinterpret_cast<void**>(&ctx->head_norm), sizeof(float) * H));
     LM_HIP(hipMalloc(reinterpret_cast<void**>(&ctx->head_w), sizeof(uint16_t) * V * H));
     LM_HIP(hipMalloc(reinterpret_cast<void**>(&ctx->head_x), sizeof(float) * batch * H));
-    LM_HIP(hipMalloc(reinterpret_cast<void**>(&ctx->head_logits), sizeof(float) * batch * V));
     LM_HIP(hipMalloc(reinterpret_cast<void**>(&ctx->head_partial),
                      sizeof(lm::HeadBest) * static_cast<size_t>(lm::head_candidates(vocab, ctx->H))));
     LM_HIP(hipMemcpy(ctx->head_norm, norm_host, sizeof(float) * H, hipMemcpyHostToDevice));
@@ -1429,7 +1423,7 @@ int lm_head_forward(lm_context* ctx, const float* hidden_dev, int64_t tokens, fl
     const int64_t group = lm::head_batch(H);
     for (int64_t t0 = 0; t0 < tokens; t0 += group) {
         const int32_t n = static_cast<int32_t>(tokens - t0 < group ? tokens - t0 : group);
-        float* logits = logits_dev != nullptr ? logits_dev + t0 * V : ctx->head_logits;
+        float* logits = logits_dev != nullptr ? logits_dev + t0 * V : nullptr;
         LM_HIP(lm::launch_rms_norm(hidden_dev + t0 * H, ctx->head_norm, ctx->head_x, n, static_cast<int32_t>(H),
                                    ctx->cfg.rms_norm_eps, ctx->stream));
         LM_HIP(lm::launch_head(ctx->head_w, ctx->head_x, logits, ctx->head_partial,

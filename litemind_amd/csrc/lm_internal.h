@@ -253,7 +253,7 @@ struct HeadBest {
 // Tokens of one head launch at most, and the candidates that its `partial` holds.
 int64_t head_batch(int64_t in_dim);
 int64_t head_candidates(int64_t rows, int64_t in_dim);
-// token may be null (logits only).
+// token may be null (logits only), or logits (token only).
 hipError_t launch_head(const uint16_t* w, const float* x, float* logits, HeadBest* partial, int32_t* token,
                        int64_t rows, int32_t in_dim, int32_t tokens, hipStream_t s);
 // The same kernel as one bit-exact gemm::matvec_bf16 (or _accumulate) of a

@@ -99,6 +99,48 @@ def test_head_ties_pick_the_first():
     assert token[0] == min(winners[0], 1500) and token[1] == min(winners[1], 7)
 
 
+@pytest.mark.parametrize("V,H,T", [(900, 512, 1), (900, 512, 3), (900, 512, 20), (5000, 2048, 13), (40, 64, 40)])
+@pytest.mark.parametrize("first", [False, True])
+def test_head_nan_logits(V, H, T, first):
+    """A NaN logit is never the choice, except at index 0, which std::max_element cannot leave;
+    a row of -inf or all NaN ends at 0.  With and without a logits buffer."""
+    from litemind_amd import Context
+
+    head, norm, hidden = _case(V + 3 * T, V, H, T)
+    head = head.copy()
+    head[[V // 2, V - 1, 17], 5] = 0x7FC0  # NaN weights: NaN logits for every token
+    if first:
+        head[0, 5] = 0x7FC0
+    head[9, :] = 0
+    head[9, 3] = 0x7F80                    # an infinite weight: +inf or -inf by the token's sign
+    announce(f"head with NaN logits V={V} H={H} T={T} first={first}")
+    with Context(_config(H)) as ctx:
+        ctx.upload_head(norm, head)
+        logits, token, token2 = _gpu(ctx, hidden, V)
+    want = _oracle(head, norm, hidden)
+    np.testing.assert_array_equal(np.isnan(logits), np.isnan(want))
+    keep = ~np.isnan(want)
+    assert np.array_equal(logits[keep].view(np.uint32), want[keep].view(np.uint32))
+    choice = [0 if first else int(np.nanargmax(want[t])) for t in range(T)]
+    assert token.tolist() == choice and token2.tolist() == choice
+
+
+def test_head_all_nan_takes_index_0():
+    from litemind_amd import Context
+
+    V, H = 300, 512
+    announce("head with every logit NaN")
+    for T in (2, 9):
+        head, norm, hidden = _case(T, V, H, T)
+        hidden[T - 1, 7] = np.nan
+        with Context(_config(H)) as ctx:
+            ctx.upload_head(norm, head)
+            logits, token, token2 = _gpu(ctx, hidden, V)
+        assert np.isnan(logits[T - 1]).all()
+        assert token[T - 1] == 0 and token2[T - 1] == 0
+        assert token[:-1].tolist() == np.argmax(logits[:-1], axis=1).tolist() == token2[:-1].tolist()
+
+
 @pytest.mark.parametrize("tied", [False, True])
 def test_head_from_checkpoint(tmp_path, tied):
     from litemind_amd import Checkpoint, Context

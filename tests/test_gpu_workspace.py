@@ -53,6 +53,31 @@ def test_first_call_of_one_token_stays_small():
     assert took < 40 * MB
 
 
+def test_head_upload_keeps_no_logits():
+    """The head's resident bytes plus what a launch of 64 tokens needs between its kernels: two
+    candidates of 12 bytes per 32 rows and token, and the normalised tokens; the logits only in the caller's
+    buffer."""
+    from litemind_amd import Context, MoeConfig
+    from litemind_amd import workload as wl
+
+    V, H = 102400, 64
+    rng = np.random.default_rng(46)
+    head = wl.f32_to_bf16(rng.standard_normal((V, H)).astype(np.float32))
+    norm = np.ones(H, np.float32)
+    config = MoeConfig(hidden_size=H, moe_intermediate_size=64, n_routed_experts=8, num_experts_per_tok=2,
+                       n_shared_experts=0, intermediate_size=0, norm_topk_prob=0, routed_scaling_factor=1.0,
+                       group_limited=0, n_group=1, topk_group=1, rms_norm_eps=1e-6, num_layers=1)
+    announce(f"upload of a head of {V} rows")
+    for _ in range(2):  # the first upload also takes what copies need
+        with Context(config) as ctx:
+            before = _free()
+            ctx.upload_head(norm, head)
+            took = before - _free()
+    print(f"head of {head.nbytes / MB:.1f} MB: {took / MB:.1f} MB")
+    need = head.nbytes + norm.nbytes + 64 * 4 * H + 12 * 64 * 2 * (V // 32)
+    assert took <= need + 8 * MB  # pages of 2 MB; the logits of 64 tokens would be 25 MB
+
+
 @pytest.mark.parametrize("T", [4, 8, 21, 64])
 def test_shared_chunks_fit_a_workspace_of_the_call(T):
     """A shared expert four times as wide as the routed ones: its K in four chunks, up to 8 rows

@@ -50,6 +50,7 @@
 #include "mfma_tile.h"
 
 #include <algorithm>
+#include <cmath>
 
 namespace lm {
 namespace {
@@ -386,15 +387,35 @@ bool offsets_fit(const ExpertArgs& a) {
 // Tiles of 64 x 128, 64 x 256 or 128 x 256 (tokens x weight rows).
 enum class TileShape { kThin, kNarrow, kWide };
 
+// Chunks of the shared expert's K no longer than the routed experts'.
+int64_t routed_chunks(int64_t inter_p, int64_t shared_inter_p) { return inter_p > 0 ? shared_inter_p / inter_p : 1; }
+
+// Tiles of 64 x 256 of a routed launch, when its tokens choose their experts evenly.
+int64_t even_tiles(const ExpertArgs& a, int mode) {
+    const double missed = std::pow(1.0 - static_cast<double>(a.top_k) / a.experts, static_cast<double>(a.tokens));
+    const int64_t groups = static_cast<int64_t>(std::ceil(a.experts * (1.0 - missed)));
+    auto columns = [&](int64_t inter_p) { return ((mode == kGateUp ? 2 * inter_p : a.hidden) + 255) / 256; };
+    return groups * columns(a.inter_p) + (a.has_shared ? (a.tokens + 63) / 64 * columns(a.shared_inter_p) : 0);
+}
+
 // Which tile a launch takes.  Routed layers stream every active expert's
 // weights, in 64 x 256 tiles up to one 64-row tile per average group; past that
 // every extra 64-row tile would stream the weights again (768 tokens and more:
-// 4 to 13% slower than 128 x 256).  Where that is only a round or two of
-// workgroups (down tiles of the active experts against 512 slots) the finer
-// 64 x 128 tiles leave a smaller last round, as long as the groups are small
-// (whole V2-Lite layer, 64 x 256 against 64 x 128: 16 tokens 163 / 156 us, 32
-// 186 / 180, 64 204 / 198, 100 203 / 202, 150 209 / 209, 256 220 / 223, 341 230
-// / 239; DeepSeek-V2's, 4 tokens 212 / 204, 16 (four rounds) 582 / 591).
+// 4 to 13% slower than 128 x 256).  Where the groups are small and that is only
+// a round or two of workgroups (down tiles of the active experts against 512
+// slots; DeepSeek-V2's layer at 16 tokens, four rounds: 582 us with 64 x 256, 591
+// with 64 x 128), the finer 64 x 128 tiles leave a smaller last round in two cases:
+//  - down, with a shared expert wider than the routed ones: its tiles are the
+//    launch's longest and only the finer ones take K in chunks (V2-Lite's down,
+//    64 x 256 against 64 x 128: 4 tokens 40 / 32 us, 16 71 / 62, 85 82 / 77);
+//  - else where they fill the 256 CUs more evenly: n tiles take the busiest CU
+//    ceil(n / 256) of them, or ceil(2 n / 256) of half the size.  Gate/up with n
+//    tiles (active experts x 11 or 12): n = 264 145 / 132 us, 290 68 / 62, 336
+//    169 / 153, 530 111 / 104; but n = 187 36 / 39, 400 179 / 186, 440 188 / 197,
+//    704 128 / 131.  Down (x 8, no shared expert): n = 64 12.0 / 10.5, 272 49 / 45;
+//    136 25 / 27, 165 26 / 30, 230 33 / 34, 464 61 / 62.  With a short K the
+//    tiles' own start and end count more (K = 512, n = 832: 49 / 55; the sizes
+//    above have 704 to 5120).
 // A layer without routed experts is one group of T rows with few column blocks:
 // its gate/up (V2-Lite's dense layer, 8 / 137 / 256 tokens) takes 17 / 35 / 43
 // us with 64 x 128 tiles, 25 / 29 / 47 with 64 x 256 and 32 / 37 / 39 with 128 x
@@ -404,7 +425,10 @@ TileShape tile_shape(const ExpertArgs& a, int mode) {
     if (a.experts > 0) {
         const int64_t rows = a.tokens * a.top_k;
         const int64_t groups = std::min<int64_t>(rows, a.experts);
-        if (rows <= 8 * a.experts && groups * ((a.hidden + 255) / 256) <= 1024) {
+        const bool few = rows <= 8 * a.experts && groups * ((a.hidden + 255) / 256) <= 1024;
+        const bool chunks = mode == kDown && routed_chunks(a.inter_p, a.shared_inter_p) > 1;
+        const bool deep = (mode == kGateUp ? a.hidden_p : a.inter_p) >= 704;
+        if (few && (chunks || (deep && (even_tiles(a, mode) + 255) % 256 < 128))) {
             return TileShape::kThin;
         }
         return rows <= 64 * a.experts ? TileShape::kNarrow : TileShape::kWide;
@@ -414,9 +438,6 @@ TileShape tile_shape(const ExpertArgs& a, int mode) {
     }
     return a.tokens <= 256 ? TileShape::kThin : TileShape::kWide;
 }
-
-// Chunks of the shared expert's K no longer than the routed experts'.
-int64_t routed_chunks(int64_t inter_p, int64_t shared_inter_p) { return inter_p > 0 ? shared_inter_p / inter_p : 1; }
 
 // K chunks of the shared group's down GEMM (hidden columns, K = shared_inter_p).
 // Without routed experts: while its tiles fill less than a round of workgroups

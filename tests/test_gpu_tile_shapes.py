@@ -53,15 +53,34 @@ def test_dense_shapes(dense, T):
     assert mx <= MAX_ABS and rel <= MEAN_REL
 
 
-# 16 experts, top-4: 64-row tiles of 128 columns up to 32 tokens, of 256 up to
-# 256, 128-row tiles above; three shared experts chunk their K in three
+# 16 experts, top-4: 64-row tiles up to 256 tokens (down's of 128 columns up to
+# 32 tokens: three shared experts chunk their K in three), 128-row tiles above
 @pytest.mark.parametrize("T", [5, 32, 33, 256, 257])
 def test_routed_shapes(T):
+    from litemind_amd import workload as wl
+    _routed(dataclasses.replace(wl.V2_LITE, hidden=320, inter=256, experts=16, top_k=4, n_shared=3), T)
+
+
+# the shape that fills the 256 CUs more evenly, for gate/up (16 x columns / 256
+# tiles of 64 x 256, with K = hidden) and down (K = inter) on their own
+@pytest.mark.parametrize("hidden,inter,n_shared", [
+    (736, 704, 0),    # 96 and 48 tiles: 64 x 128 both
+    (736, 1408, 2),   # 198 tiles: 64 x 256; down 64 x 128 for the shared expert's chunks
+    (2560, 704, 1),   # 102 tiles: 64 x 128; down 170: 64 x 256
+    (2560, 1408, 0),  # 176 and 160: 64 x 256 both
+    (736, 512, 1),    # 68: 64 x 128; down 51 tiles of a short K: 64 x 256
+])
+@pytest.mark.parametrize("T", [13, 32])
+def test_routed_shapes_by_rounds(hidden, inter, n_shared, T):
+    from litemind_amd import workload as wl
+    _routed(dataclasses.replace(wl.V2_LITE, hidden=hidden, inter=inter, experts=16, top_k=4, n_shared=n_shared), T)
+
+
+def _routed(d, T):
     from litemind_amd import PATH_MFMA, Context
     from litemind_amd import workload as wl
-    d = dataclasses.replace(wl.V2_LITE, hidden=320, inter=256, experts=16, top_k=4, n_shared=3)
     L = wl.moe_layer(73, 0, d)
-    announce(f"routed tile shapes T={T}")
+    announce(f"routed tile shapes hidden={d.hidden} inter={d.inter} shared={d.n_shared} T={T}")
     x = wl.tokens(74, T, d.hidden)
     with Context(d.moe_config(num_layers=1)) as ctx:
         wl.upload_moe_layer(ctx, 0, L)
@@ -71,7 +90,7 @@ def test_routed_shapes(T):
         ctx.synchronize()
         y, idx, w = dy.download(), di.download(), dw.download()
     x = x.astype(np.float64)
-    want = _ffn(x, L.shared_gate, L.shared_up, L.shared_down)
+    want = _ffn(x, L.shared_gate, L.shared_up, L.shared_down) if d.n_shared else np.zeros_like(x)
     for e in range(d.experts):
         t, r = np.nonzero(idx == e)
         if t.size:

@@ -118,8 +118,9 @@ int lm_attention_set_path(lm_context* ctx, int32_t path);
  * operands over fp16 copies of the cache made once per call, P the causal
  * softmax in fp32 rounded to fp16; within the MFMA path's tolerance.  Heads of
  * 128 + 64 key and 128 value channels run it in one launch that keeps the
- * scores in registers (every query token at once; in the plan's groups only
- * where few query tokens share out the keys of a long cache).
+ * scores in registers, every query token at once; where few query tokens share
+ * out the keys of a long cache, as many at once as the budget below holds of
+ * their partial contexts (520 bytes per head, token and share) beside the copies.
  *
  * The core takes the call's query tokens in groups sized from a byte budget
  * for its scratch (no LiteMind counterpart): the fp32 scores, and for the MFMA
@@ -136,7 +137,9 @@ typedef struct lm_attention_core_plan {
 } lm_attention_core_plan;
 /* The sizing lm_attention_forward chooses for `tokens` new tokens after
  * `cached` ones on a layer with fp16 weight copies, for a path and a budget
- * (0: the default); host only, no context or GPU. */
+ * (0: the default); host only, no context or GPU.  For heads of 128 + 64 and 128
+ * channels mfma_core is its choice as well; the group and the bytes are those
+ * of the core that keeps its scores in memory. */
 int lm_attention_plan_core(const lm_mla_config* config, int64_t cached, int64_t tokens, int32_t path,
                            int64_t budget_bytes, lm_attention_core_plan* out);
 /* KvCache::clear for every layer (src/DeepSeekRunner.cpp:432-437, DeepSeekRunner::reset). */

@@ -343,7 +343,7 @@ int project(const AttnLayer& L, int proj, const uint16_t* w, const float* x, int
 //   core | o_proj
 // Before, a 512-token V2-Lite prompt took 22 launches on two streams: 108 us
 // against 32, 4096 tokens 1186 us against 258.
-int attention_prompt(AttnState* st, hipStream_t stream, AttnLayer& L, const CorePlan& plan, const float* x, int64_t F,
+int attention_prompt(AttnState* st, hipStream_t stream, AttnLayer& L, int64_t budget, const float* x, int64_t F,
                      int64_t pos0, float* out, int32_t accumulate, const float* in_norm) {
     const lm_mla_config& c = st->cfg;
     const lm::AttnShape& a = st->shape;
@@ -353,8 +353,14 @@ int attention_prompt(AttnState* st, hipStream_t stream, AttnLayer& L, const Core
     const int64_t kp = lm::flash_keys(n0 + F);
     const lm::FlashPlan fp = lm::flash_plan(a.heads, F, n0 + F);
     // query tokens per core launch: all, or when the keys are split (each query
-    // token then has partial contexts) the group that the budget holds
-    const int64_t group = fp.splits > 1 ? plan.group : F;
+    // token then has partial contexts) as many as the budget holds beside the
+    // copies.  Not plan_core's group: the splits fill the CUs with all of the
+    // call's tokens at once, and in launches of at most 512 half of the CUs or
+    // more were idle (V2-Lite, 1024 tokens after 20000: 846 us for the call, 430
+    // in one launch; after 1000 143 and 112; two heads, 8000 tokens 1328 and 411).
+    const int64_t copies = 2 * kp * (heads * (c.qk_nope_head_dim + vh) + rope);
+    const int64_t per = 4 * lm::flash_partial_floats(fp, a.heads, 1);
+    const int64_t group = per > 0 ? std::clamp((budget - copies) / per, int64_t{1}, F) : F;
     size_t total_f = 0;
     auto region = [&](int64_t floats) {
         const size_t at = total_f;
@@ -464,9 +470,10 @@ int attention_tokens(AttnState* st, hipStream_t stream, int32_t layer, const flo
     const int64_t n0 = L.count;
     const int64_t n_total = n0 + F;
     const bool mfma = L.table16 != nullptr && mfma_projections(path, F);
-    const CorePlan plan = plan_core(a, n0, F, mfma, st->score_budget > 0 ? st->score_budget : kScoreBudget);
+    const int64_t budget = st->score_budget > 0 ? st->score_budget : kScoreBudget;
+    const CorePlan plan = plan_core(a, n0, F, mfma, budget);
     if (plan.mfma && lm::flash_supported(a)) {
-        return attention_prompt(st, stream, L, plan, x, F, pos0, out, accumulate, in_norm);
+        return attention_prompt(st, stream, L, budget, x, F, pos0, out, accumulate, in_norm);
     }
     const int64_t core = plan.group;
     // Scratch, each region a multiple of 64 floats: q | q latent | kv latent |
@@ -591,7 +598,7 @@ int attention_tokens(AttnState* st, hipStream_t stream, int32_t layer, const flo
         LM_ATT_HIP(hipStreamWaitEvent(stream, st->join, 0));
     }
     // causal attention over the cache (:77-98), in groups of query tokens
-if (plan.mfma) {
+    if (plan.mfma) {
         // the context lands in fp16 panels [F, heads vh] in x16kv (free once
         // kv_b has run), the output projection's input; ctxv holds the
         // per-head context of one group

@@ -10,6 +10,7 @@ few units and a second product, then the output projection; their independent
 errors stay near 1e-3 of the output's scale, and the bounds are the path's own
 (mean relative 5e-3, maximum 5e-2 at outputs of magnitude 1).
 """
+import ctypes as C
 import dataclasses
 
 import numpy as np
@@ -125,3 +126,92 @@ def test_flash_core_groups_bit_identical():
         finally:
             m.close()
     np.testing.assert_array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+
+
+def _cache(rng, d, cached):
+    return [rng.standard_normal(s).astype(np.float32) for s in (
+        (cached, d.heads, d.qk_nope), (cached, d.qk_rope), (cached, d.heads, d.v_head))]
+
+
+def test_flash_partials_past_the_budget():
+    """One head after 4200 tokens: 15 splits of 520 bytes a query token, and a budget of twice the
+    key and value copies, which holds the partial contexts of some 390 tokens of 600."""
+    from litemind_amd import PATH_MFMA, attention_plan_core
+    from litemind_amd import workload as wl
+    cached, T, budget = 4200, 600, 6_200_000
+    d = dataclasses.replace(wl.V2_LITE_MLA, heads=1, max_positions=cached + T)
+    cache = _cache(np.random.default_rng(19), d, cached)
+    x = tokens(307, T, d.hidden)
+    assert attention_plan_core(wl.mla_config(d), cached, T, PATH_MFMA, budget).mfma_core == 1
+    announce("attention one-launch core, partial contexts in two groups against one")
+    outs = []
+    for b in (budget, 0):
+        m = Mla(d, 308, path=PATH_MFMA)
+        try:
+            m.ctx.attention_set_score_budget(b)
+            m.ctx.kv_cache_write(0, 0, *cache)
+            outs.append(m.forward(x, cached))
+            want = _reference(m, x, cached)
+        finally:
+            m.close()
+    np.testing.assert_array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+    mx, rel = layer_error(outs[0], want)
+    assert mx <= ATT_MAX_ABS and rel <= ATT_MEAN_REL
+
+
+@pytest.mark.parametrize("cached,T,launches", [
+    (2000, 1024, 8),  # copies of the cache, x, q and kv_a, norm, kv_b, core, its splits joined, o_proj
+    (2000, 100, 8),
+    (0, 1024, 7),     # no cache
+    (0, 512, 6),      # nor splits
+])
+def test_prompt_captured(cached, T, launches):
+    """A prompt under stream capture: one launch per step, the core's splits of all query tokens
+    at once, and replays between eager calls that give the eager bits."""
+    from litemind_amd import PATH_MFMA
+    from litemind_amd import workload as wl
+    hip = C.CDLL("libamdhip64.so.7")
+    hip.hipStreamBeginCapture.argtypes = [C.c_void_p, C.c_int]
+    hip.hipStreamEndCapture.argtypes = [C.c_void_p, C.POINTER(C.c_void_p)]
+    hip.hipGraphGetNodes.argtypes = [C.c_void_p, C.c_void_p, C.POINTER(C.c_size_t)]
+    hip.hipGraphInstantiate.argtypes = [C.POINTER(C.c_void_p), C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t]
+    hip.hipGraphLaunch.argtypes = [C.c_void_p, C.c_void_p]
+    hip.hipGraphDestroy.argtypes = hip.hipGraphExecDestroy.argtypes = [C.c_void_p]
+    d = dataclasses.replace(wl.V2_LITE_MLA, max_positions=cached + T)
+    m = Mla(d, 309, path=PATH_MFMA)
+    ctx = m.ctx
+    try:
+        if cached:
+            ctx.kv_cache_write(0, 0, *_cache(np.random.default_rng(20), d, cached))
+        x = tokens(310, T, d.hidden)
+        dx, dout = ctx.to_device(x), ctx.to_device(np.full_like(x, np.nan))
+        stream, graph, run, n = C.c_void_p(ctx.stream()), C.c_void_p(), C.c_void_p(), C.c_size_t()
+
+        def eager():
+            ctx.kv_cache_truncate(0, cached)
+            ctx.attention_forward(0, dx, T, cached, dout)
+
+        announce(f"attention prompt captured cached={cached} T={T}")
+        eager()
+        ctx.synchronize()
+        want = dout.download()
+        assert hip.hipStreamBeginCapture(stream, 2) == 0  # hipStreamCaptureModeRelaxed
+        eager()
+        assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+        assert hip.hipGraphGetNodes(graph, None, C.byref(n)) == 0
+        print(f"cached={cached} T={T}: {n.value} launches")
+        assert n.value == launches
+        assert hip.hipGraphInstantiate(C.byref(run), graph, None, None, 0) == 0
+        for _ in range(3):
+            dout.upload(np.full_like(x, np.nan))
+            assert hip.hipGraphLaunch(run, stream) == 0
+            ctx.synchronize()
+            np.testing.assert_array_equal(dout.download().view(np.uint32), want.view(np.uint32))
+            eager()
+            ctx.synchronize()
+            np.testing.assert_array_equal(dout.download().view(np.uint32), want.view(np.uint32))
+        assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
+        dx.free()
+        dout.free()
+    finally:
+        m.close()

@@ -486,11 +486,11 @@ def test_small_score_budget_groups_bit_exact():
 
 
 def test_mfma_core_small_budget_two_groups():
-    """V2-Lite on the MFMA core: 40 tokens, then 96 with a budget that holds 77
-    query tokens (two core launches, the second of 19 rows per head on the
-    narrow tile); the outputs equal those of one 96-token group bit for bit
-    (every score and context element has the same K order either way) and meet
-    the oracle within the MFMA tolerance."""
+    """V2-Lite on the MFMA path: 40 tokens, then 96 with a budget that the plan fills
+    with the scores of 77 query tokens.  The one-launch core of these head widths
+    keeps no scores and takes all 96 either way: the outputs equal those of the
+    default budget bit for bit and meet the oracle within the MFMA tolerance.
+    (test_score_core_small_budget_two_groups has the core that works in groups.)"""
     from litemind_amd import PATH_AUTO, attention_plan_core
     from litemind_amd import workload as wl
     d = dataclasses.replace(wl.V2_LITE_MLA, max_positions=160)
@@ -518,6 +518,68 @@ def test_mfma_core_small_budget_two_groups():
             m.close()
     for a, b in zip(outs[0], outs[1]):
         np.testing.assert_array_equal(bits(a), bits(b))
+
+
+def test_score_core_small_budget_two_groups():
+    """Other head widths on the MFMA path, whose core keeps its scores in memory: 40
+    tokens, then 96 with a budget that holds 76 query tokens (two core launches,
+    the second of 20 rows per head); the outputs equal those of one 96-token group
+    bit for bit (every score and context element has the same K order either way)
+    and meet the oracle within the MFMA tolerance."""
+    from litemind_amd import PATH_AUTO, attention_plan_core
+    from litemind_amd import workload as wl
+    d = dataclasses.replace(wl.V2_LITE_MLA, hidden=512, kv_lora_rank=128, qk_nope=64, v_head=64, max_positions=160)
+    budget = 2_480_000  # copies 16 x 160 keys x 192 channels x 2 bytes, 19456 bytes per query token
+    plan = attention_plan_core(wl.mla_config(d), 40, 96, PATH_AUTO, budget)
+    assert plan.mfma_core == 1 and plan.query_group == 76
+    assert attention_plan_core(wl.mla_config(d), 40, 96, PATH_AUTO).query_group == 96
+    announce("attention MFMA core of other head widths, 40 + 96 tokens, score budget of 76 query tokens vs default")
+    x = tokens(234, 136, d.hidden)
+    outs = []
+    for b in (budget, 0):
+        m = Mla(d, 233, path=PATH_AUTO)
+        try:
+            m.ctx.attention_set_score_budget(b)
+            y0 = m.forward(x[:40], 0)
+            y1 = m.forward(x[40:], 40)
+            if b:
+                for y, lo, hi in ((y0, 0, 40), (y1, 40, 136)):
+                    want, _ = m.oracle(x[lo:hi], lo)
+                    mx, rel = layer_error(y, want)
+                    print(f"score core {lo}..{hi}: max_abs={mx:.3e} mean_rel={rel:.3e}")
+                    assert mx <= ATT_MAX_ABS and rel <= ATT_MEAN_REL
+            outs.append((y0, y1))
+        finally:
+            m.close()
+    for a, b in zip(outs[0], outs[1]):
+        np.testing.assert_array_equal(bits(a), bits(b))
+
+
+@pytest.mark.parametrize("cached", [2, 509, 511, 512, 1000])
+@pytest.mark.parametrize("T", [2, 3, 4, 17])
+def test_few_tokens_after_a_cache_bit_exact(cached, T):
+    """Two to four query tokens (score blocks of two and four) and 17 (a ragged tile of 16)
+    at V2-Lite's head widths over a cache whose end lies before, at and past the
+    512 keys that the context sums stage at once; the last keys of a tile, which not
+    every token sees, in one chunk or two."""
+    from litemind_amd import workload as wl
+    d = dataclasses.replace(wl.V2_LITE_MLA, hidden=256, heads=3, kv_lora_rank=64, max_positions=1024)
+    announce(f"attention exact path, {T} tokens after {cached}")
+    m = Mla(d, 251)
+    try:
+        rng = np.random.default_rng(1000 * T + cached)
+        for mine in (m.cache.key_nope, m.cache.key_rope, m.cache.value):
+            mine[:cached] = rng.standard_normal(mine[:cached].shape).astype(np.float32)
+        m.cache.count.value = cached
+        m.ctx.kv_cache_write(0, 0, m.cache.key_nope[:cached], m.cache.key_rope[:cached], m.cache.value[:cached])
+        x = tokens(252 + T, T, d.hidden)
+        y = m.forward(x, cached)
+        want, n = m.oracle(x, cached)
+        assert n == T
+        np.testing.assert_array_equal(bits(y), bits(want))
+        m.check_cache()
+    finally:
+        m.close()
 
 
 def test_kv_cache_write_read_range_truncate():

@@ -26,28 +26,29 @@ def _f32(bits):
     return (np.asarray(bits).astype(np.uint32) << 16).view(np.float32).astype(np.float64)
 
 
-def _reference(m, x, cached, rotated=True):
+def _reference(m, x, cached, rotated=True, rows=None):
     """float64 attention of x [T, H] at positions cached.. over the layer's cache (past the
-    rotary table the channels stay as they are)."""
+    rotary table the channels stay as they are), of the given rows only or all."""
     from litemind_amd import mla_softmax_scale, rope_tables
     from litemind_amd import workload as wl
     d, L, T = m.d, m.L, x.shape[0]
     n = cached + T
+    at = np.arange(T) if rows is None else np.asarray(rows)
     kn, kr, v = (a.astype(np.float64) for a in m.ctx.kv_cache_read(0, n))
     cfg = wl.mla_config(d)
-    cos, sin = (t[cached:n].astype(np.float64)[:, None] for t in rope_tables(cfg, n))
-    q = (x.astype(np.float64) @ _f32(L.q_proj).T).reshape(T, d.heads, d.qk_head)
+    cos, sin = (t[cached:n][at].astype(np.float64)[:, None] for t in rope_tables(cfg, n))
+    q = (x[at].astype(np.float64) @ _f32(L.q_proj).T).reshape(len(at), d.heads, d.qk_head)
     even, odd = q[..., d.qk_nope::2], q[..., d.qk_nope + 1::2]
     rot = np.concatenate([even * cos - odd * sin, odd * cos + even * sin], axis=-1) if rotated else q[..., d.qk_nope:]
     scale = float(mla_softmax_scale(cfg))
-    hidden = np.arange(n)[None] > np.arange(cached, n)[:, None]
-    ctx = np.empty((T, d.heads, d.v_head))
+    hidden = np.arange(n)[None] > cached + at[:, None]
+    ctx = np.empty((len(at), d.heads, d.v_head))
     for h in range(d.heads):
         s = scale * (q[:, h, :d.qk_nope] @ kn[:, h].T + rot[:, h] @ kr.T)
         s[hidden] = -np.inf
         p = np.exp(s - s.max(axis=1, keepdims=True))
         ctx[:, h] = (p / p.sum(axis=1, keepdims=True)) @ v[:, h]
-    return ctx.reshape(T, -1) @ _f32(L.o_proj).T
+    return ctx.reshape(len(at), -1) @ _f32(L.o_proj).T
 
 
 @pytest.mark.parametrize("heads,cached,T", [
@@ -80,6 +81,42 @@ def test_flash_core(heads, cached, T):
         assert mx <= ATT_MAX_ABS and rel <= ATT_MEAN_REL
         for t in (0, T - 1):  # no row is off while the mean is fine
             assert np.abs(y[t] - want[t]).sum() <= 2 * ATT_MEAN_REL * np.abs(want[t]).sum()
+    finally:
+        m.close()
+
+
+@pytest.mark.parametrize("T", [700, 1400, 2600])
+def test_prompt_projection_tiles(T):
+    """The projections' larger tiles at V2-Lite's widths: q and kv_a, then kv_b, as 128 x 128 tiles
+    from 641 tokens and 128 x 256 from 1281, o_proj from 1281 and 2561.  Every row of the cache,
+    and the outputs of tokens at the edges of waves and tiles."""
+    from litemind_amd import PATH_MFMA
+    from litemind_amd import workload as wl
+    d = dataclasses.replace(wl.V2_LITE_MLA, max_positions=T)
+    announce(f"attention prompt, projection tiles T={T}")
+    m = Mla(d, 311, path=PATH_MFMA)
+    try:
+        x = tokens(312, T, d.hidden)
+        y = m.forward(x, 0)
+        kn, kr, v = m.ctx.kv_cache_read(0, T)
+        L, cfg = m.L, wl.mla_config(d)
+        kv = x.astype(np.float64) @ _f32(L.kv_a_proj).T
+        c = kv[:, :d.kv_lora_rank]
+        c = c / np.sqrt((c * c).mean(axis=1, keepdims=True) + d.rms_norm_eps) * L.kv_a_layernorm.astype(np.float64)
+        wide = (c @ _f32(L.kv_b_proj).T).reshape(T, d.heads, d.qk_nope + d.v_head)
+        from litemind_amd import rope_tables
+        cos, sin = (t.astype(np.float64) for t in rope_tables(cfg, T))
+        even, odd = kv[:, d.kv_lora_rank::2], kv[:, d.kv_lora_rank + 1::2]
+        rotated = np.concatenate([even * cos - odd * sin, odd * cos + even * sin], axis=1)
+        for got, want in ((kn, wide[..., :d.qk_nope]), (kr, rotated), (v, wide[..., d.qk_nope:])):
+            # fp16 operands in two products: 2^-11 relative each, per row (a wrong row is of order 1)
+            off = np.abs(got - want).reshape(T, -1).sum(axis=1) / np.abs(want).reshape(T, -1).sum(axis=1)
+            assert off.max() <= ATT_MEAN_REL
+        rows = sorted({t for edge in range(0, T + 1, 128) for t in (edge - 1, edge) if 0 <= t < T} | {33, T - 1})
+        want = _reference(m, x, 0, rows=rows)
+        off = np.abs(y[rows] - want).sum(axis=1) / np.abs(want).sum(axis=1)
+        print(f"T={T}: mean_rel by row up to {off.max():.3e}")
+        assert np.all(np.isfinite(y)) and off.max() <= 2 * ATT_MEAN_REL
     finally:
         m.close()
 

@@ -390,32 +390,36 @@ enum class TileShape { kThin, kNarrow, kWide };
 // Chunks of the shared expert's K no longer than the routed experts'.
 int64_t routed_chunks(int64_t inter_p, int64_t shared_inter_p) { return inter_p > 0 ? shared_inter_p / inter_p : 1; }
 
-// Tiles of 64 x 256 of a routed launch, when its tokens choose their experts evenly.
-int64_t even_tiles(const ExpertArgs& a, int mode) {
+// Gate/up tiles of 64 x 256 of a routed layer whose tokens choose their experts evenly.
+int64_t even_tiles(const ExpertArgs& a) {
     const double missed = std::pow(1.0 - static_cast<double>(a.top_k) / a.experts, static_cast<double>(a.tokens));
     const int64_t groups = static_cast<int64_t>(std::ceil(a.experts * (1.0 - missed)));
-    auto columns = [&](int64_t inter_p) { return ((mode == kGateUp ? 2 * inter_p : a.hidden) + 255) / 256; };
-    return groups * columns(a.inter_p) + (a.has_shared ? (a.tokens + 63) / 64 * columns(a.shared_inter_p) : 0);
+    const int64_t shared = a.has_shared ? (a.tokens + 63) / 64 * ((2 * a.shared_inter_p + 255) / 256) : 0;
+    return groups * ((2 * a.inter_p + 255) / 256) + shared;
 }
 
-// Which tile a launch takes.  Routed layers stream every active expert's
-// weights, in 64 x 256 tiles up to one 64-row tile per average group; past that
-// every extra 64-row tile would stream the weights again (768 tokens and more:
-// 4 to 13% slower than 128 x 256).  Where the groups are small and that is only
-// a round or two of workgroups (down tiles of the active experts against 512
-// slots; DeepSeek-V2's layer at 16 tokens, four rounds: 582 us with 64 x 256, 591
-// with 64 x 128), the finer 64 x 128 tiles leave a smaller last round in two cases:
-//  - down, with a shared expert wider than the routed ones: its tiles are the
-//    launch's longest and only the finer ones take K in chunks (V2-Lite's down,
-//    64 x 256 against 64 x 128: 4 tokens 40 / 32 us, 16 71 / 62, 85 82 / 77);
-//  - else where they fill the 256 CUs more evenly: n tiles take the busiest CU
-//    ceil(n / 256) of them, or ceil(2 n / 256) of half the size.  Gate/up with n
-//    tiles (active experts x 11 or 12): n = 264 145 / 132 us, 290 68 / 62, 336
-//    169 / 153, 530 111 / 104; but n = 187 36 / 39, 400 179 / 186, 440 188 / 197,
-//    704 128 / 131.  Down (x 8, no shared expert): n = 64 12.0 / 10.5, 272 49 / 45;
-//    136 25 / 27, 165 26 / 30, 230 33 / 34, 464 61 / 62.  With a short K the
-//    tiles' own start and end count more (K = 512, n = 832: 49 / 55; the sizes
-//    above have 704 to 5120).
+// Which tile a layer's launches take.  Routed layers stream every active
+// expert's weights, in 64 x 256 tiles up to one 64-row tile per average group;
+// past that every extra 64-row tile would stream the weights again (768 tokens
+// and more: 4 to 13% slower than 128 x 256).  Where the groups are small and that
+// is only a round or two of workgroups (down tiles of the active experts against
+// 512 slots; DeepSeek-V2's layer at 16 tokens, four rounds: 582 us with 64 x 256,
+// 591 with 64 x 128), both launches take the finer 64 x 128 tiles: a smaller last
+// round, and the shared expert's K in chunks.  Not where the 256 CUs would just
+// hold one 64 x 256 tile each, or where K is short: there the finer ones only
+// add their own start and end, unless K is long or the shared expert's chunks
+// make up for it.  Whole layers, 64 x 256 against 64 x 128, us of one context's
+// calls in a row and of three contexts' in turn, whose launches overlap:
+//   64 experts of 1408, no shared one, 3 tokens (187 tiles) 75 / 76, 52 / 55; 4
+//     94 / 98, 68 / 67; 16 (560) 167 / 164, 144 / 139; 64 (704) 217 / 222, 189 / 184
+//   32 experts, 3 tokens (165) 69 / 73, 45 / 46; 5 (220) 89 / 94, 66 / 66; 8 (297)
+//     120 / 116, 79 / 77; 128 experts of 768, 4 tokens (174) 78 / 80, 54 / 54
+//   256 experts of 512, 4 tokens (124) 74 / 82, 46 / 45; 16 (412) 158 / 168, 117 /
+//     120; 8 experts of 4096 at hidden 4096, 4 tokens (192) 126 / 107, 87 / 84
+//   V2-Lite, 4 tokens (253) 98 / 91, 66 / 64; 16 201 / 186, 150 / 146; 32 226 / 218,
+//     186 / 180; DeepSeek-V2, 4 tokens 282 / 262, 197 / 193; 6 305 / 323, 270 / 263
+// (gate/up and down each by its own count of tiles was faster in a row, but
+// two shapes overlap badly: V2-Lite, 32 tokens 217 in a row, 185 in turn).
 // A layer without routed experts is one group of T rows with few column blocks:
 // its gate/up (V2-Lite's dense layer, 8 / 137 / 256 tokens) takes 17 / 35 / 43
 // us with 64 x 128 tiles, 25 / 29 / 47 with 64 x 256 and 32 / 37 / 39 with 128 x
@@ -426,9 +430,9 @@ TileShape tile_shape(const ExpertArgs& a, int mode) {
         const int64_t rows = a.tokens * a.top_k;
         const int64_t groups = std::min<int64_t>(rows, a.experts);
         const bool few = rows <= 8 * a.experts && groups * ((a.hidden + 255) / 256) <= 1024;
-        const bool chunks = mode == kDown && routed_chunks(a.inter_p, a.shared_inter_p) > 1;
-        const bool deep = (mode == kGateUp ? a.hidden_p : a.inter_p) >= 704;
-        if (few && (chunks || (deep && (even_tiles(a, mode) + 255) % 256 < 128))) {
+        const int64_t tiles = even_tiles(a), k = std::min(a.hidden_p, a.inter_p);
+        const bool more = k >= 704 && (tiles <= 128 || tiles > 256 || k >= 4096);
+        if (few && (more || routed_chunks(a.inter_p, a.shared_inter_p) > 1)) {
             return TileShape::kThin;
         }
         return rows <= 64 * a.experts ? TileShape::kNarrow : TileShape::kWide;

@@ -53,25 +53,25 @@ def test_dense_shapes(dense, T):
     assert mx <= MAX_ABS and rel <= MEAN_REL
 
 
-# 16 experts, top-4: 64-row tiles up to 256 tokens (down's of 128 columns up to
-# 32 tokens: three shared experts chunk their K in three), 128-row tiles above
+# 16 experts, top-4: 64-row tiles of 128 columns up to 32 tokens, of 256 up to
+# 256, 128-row tiles above; three shared experts chunk their K in three
 @pytest.mark.parametrize("T", [5, 32, 33, 256, 257])
 def test_routed_shapes(T):
     from litemind_amd import workload as wl
     _routed(dataclasses.replace(wl.V2_LITE, hidden=320, inter=256, experts=16, top_k=4, n_shared=3), T)
 
 
-# the shape that fills the 256 CUs more evenly, for gate/up (16 x columns / 256
-# tiles of 64 x 256, with K = hidden) and down (K = inter) on their own
+# small groups by their gate/up tiles of 64 x 256 (16 experts x columns / 256)
 @pytest.mark.parametrize("hidden,inter,n_shared", [
-    (736, 704, 0),    # 96 and 48 tiles: 64 x 128 both
-    (736, 1408, 2),   # 198 tiles: 64 x 256; down 64 x 128 for the shared expert's chunks
-    (2560, 704, 1),   # 102 tiles: 64 x 128; down 170: 64 x 256
-    (2560, 1408, 0),  # 176 and 160: 64 x 256 both
-    (736, 512, 1),    # 68: 64 x 128; down 51 tiles of a short K: 64 x 256
+    (736, 704, 0),    # 96: one per CU or none, 64 x 128
+    (736, 1408, 2),   # 198, but the shared expert's K in two chunks: 64 x 128
+    (2560, 704, 1),   # 102: 64 x 128
+    (2560, 1408, 0),  # 176: one per CU, 64 x 256
+    (736, 2112, 0),   # 272: more, 64 x 128
+    (736, 512, 1),    # 68 of a short K in down: 64 x 256
 ])
 @pytest.mark.parametrize("T", [13, 32])
-def test_routed_shapes_by_rounds(hidden, inter, n_shared, T):
+def test_routed_shapes_by_tiles(hidden, inter, n_shared, T):
     from litemind_amd import workload as wl
     _routed(dataclasses.replace(wl.V2_LITE, hidden=hidden, inter=inter, experts=16, top_k=4, n_shared=n_shared), T)
 

@@ -902,8 +902,9 @@ __global__ __launch_bounds__(256) void context_kernel(const float* __restrict__ 
 // an unseen value would not be the same sum for infinite values or negative
 // zeros).  A workgroup is 16 tokens x 64 channels of one head, a wave 16
 // channels; the probabilities pass through LDS in chunks, the values come from
-// L2 kCtxMAhead steps ahead.  Bound by the chains' latency.  V2-Lite: 2 tokens
-// after 1000 58 us for the whole call before, 39 after.
+// L2 kCtxMAhead steps ahead.  Bound by the chains' latency.  V2-Lite, whole calls
+// in a row on one stream: 2 tokens after 1000 137 us with context_kernel, 78
+// with this one; 77 after 301 121 and 97.
 constexpr int kCtxMTokens = 16;
 constexpr int kCtxMKeys = 512;                  // keys of a chunk
 constexpr int kCtxMStride = kCtxMKeys + 4;      // floats per token's row: 16 rows x 4 keys on 64 banks

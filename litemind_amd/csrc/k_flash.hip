@@ -448,11 +448,12 @@ int64_t flash_keys(int64_t keys) { return round_up(keys, kTile); }
 
 // Splits while the query blocks leave CUs idle, of at least four tiles on
 // average (a causal block sees half of the call's own keys).  Measured (V2-Lite,
-// 16 heads; us for 1 / 2 / 4 / 8 splits): 16 tokens after 4000 78 / 46 / 28 / 22,
-// 256 after 3000 72 / 45 / 30 / 26, 512 after 3000 77 / 48 / 34 / 37, 512 alone
-// 15 / 17 / 18 / 21, 1024 after 1000 48 / 37 / 37 / 45, 2048 alone 49 / 52 / 50 /
-// 57.  Workgroups of one or two waves were slower throughout (512 alone 17 with
-// two): a tile is staged for fewer query tokens.
+// 16 heads, whole calls in a row on one stream; us for 1 / 2 / 4 / 8 splits): 16
+// tokens after 4000 126 / 91 / 73 / 66, 256 after 3000 118 / 89 / 74 / 70, 512
+// after 3000 130 / 101 / 86 / 90, 512 alone 54 / 54 / 54 / 58, 1024 alone 80 / 78
+// / 80 / 85, after 1000 110 / 100 / 101 / 109, after 20000 595 / 413 / 400 / 412,
+// 2048 alone 144 / 146 / 148 / 154.  Workgroups of one or two waves were slower
+// throughout: a tile is staged for fewer query tokens.
 FlashPlan flash_plan(int32_t heads, int64_t tokens, int64_t keys) {
     FlashPlan p;
     const int64_t tiles = (keys + kTile - 1) / kTile;

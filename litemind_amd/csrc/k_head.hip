@@ -208,11 +208,11 @@ __global__ __launch_bounds__(THREADS) void head_logits_kernel(const uint16_t* __
 // chains through the ring's LDS and reduce them in dot_bf16's order.
 //
 // What bounds it: the fp32 matrix rate (134 TFLOP/s measured for 32x32x2) at
-// 32 and more tokens, the weight stream below.  [102400, 2048] head: 16 tokens
-// 99 us (4.2 TB/s), 32 tokens 139 us (96 TFLOP/s; 8 launches of the few-token
-// kernel: 565 us); [3072, 2048] projection of 77 tokens 14.7 us (VALU chains,
-// one token per lane: about 35).  Small projections end with their longest
-// wave: 16 stages of 8 chains.
+// 32 and more tokens, the weight stream below.  [102400, 2048] head, launches in
+// a row: 16 tokens 106 us (4.0 TB/s), 32 tokens 155 us (87 TFLOP/s); whole calls
+// 116 and 166 us, 416 and 833 with the few-token kernel's launches of 4.  [3072,
+// 2048] projection of 77 tokens 15 us (VALU chains, one token per lane: about
+// 35).  Small projections end with their longest wave: 16 stages of 8 chains.
 typedef __attribute__((address_space(3))) void head_lds_void;
 constexpr int kHeadBufferWord3 = 0x00020000;  // buffer descriptor word 3, raw 32-bit access
 // s_waitcnt immediate: vmcnt(n) (bits 3:0 and 15:14), the other counters unconstrained
@@ -566,7 +566,7 @@ bool exact_supported(int64_t in_dim) { return in_dim % 64 == 0; }
 // / 9.3 us).  Few tiles end sooner as small ones, which spread over more CUs
 // (kv_a, 576 rows x 77 tokens: 6.7 us as 16 x 16 tiles, 14.5 as 32 x 32); many
 // tiles do fewer LDS reads per multiply-add as large ones (102400 rows x 32
-// tokens: 139 us as 32 x 32 tiles, 160 as 16 x 32).
+// tokens: 155 us as 32 x 32 tiles, some 15% more as 16 x 32).
 ExactShape exact_shape(int64_t rows, int64_t in_dim, int64_t tokens) {
     if (in_dim % 128 != 0) {
         return ExactShape::k32;

@@ -566,7 +566,7 @@ bool exact_supported(int64_t in_dim) { return in_dim % 64 == 0; }
 // / 9.3 us).  Few tiles end sooner as small ones, which spread over more CUs
 // (kv_a, 576 rows x 77 tokens: 6.7 us as 16 x 16 tiles, 14.5 as 32 x 32); many
 // tiles do fewer LDS reads per multiply-add as large ones (102400 rows x 32
-// tokens: 155 us as 32 x 32 tiles, some 15% more as 16 x 32).
+// tokens, whole calls: 165 us as 32 x 32 tiles, 184 as 16 x 32).
 ExactShape exact_shape(int64_t rows, int64_t in_dim, int64_t tokens) {
     if (in_dim % 128 != 0) {
         return ExactShape::k32;

@@ -14,6 +14,7 @@
 #include <cstdio>
 #include <cstring>
 #include <exception>
+#include <iterator>
 #include <mutex>
 #include <new>
 #include <string>
@@ -84,6 +85,7 @@ struct Layer {
 
 struct Workspace {
     int64_t tokens = 0;
+    void* slab = nullptr;         // one allocation for all up to permute_scratch, decode_* and spec_sync apart
     int32_t* idx = nullptr;
     float* wts = nullptr;
     int32_t* counts = nullptr;
@@ -362,48 +364,53 @@ int ensure_workspace(lm_context* ctx, int64_t tokens) {
                                    " tokens); destroy it before a call with " + std::to_string(tokens));
     }
     LM_HIP(hipStreamSynchronize(ctx->stream));
-    void** ptrs[] = {reinterpret_cast<void**>(&w.idx),     reinterpret_cast<void**>(&w.wts),
-                     reinterpret_cast<void**>(&w.counts),  reinterpret_cast<void**>(&w.offsets),
-                     reinterpret_cast<void**>(&w.active),  reinterpret_cast<void**>(&w.perm),
-                     reinterpret_cast<void**>(&w.slot_of), reinterpret_cast<void**>(&w.act),
-                     reinterpret_cast<void**>(&w.x16),     reinterpret_cast<void**>(&w.down_out),
-                     reinterpret_cast<void**>(&w.xnorm),   reinterpret_cast<void**>(&w.ffn),
-                     reinterpret_cast<void**>(&w.zero),    reinterpret_cast<void**>(&w.logit_scratch),
-                     reinterpret_cast<void**>(&w.ticket),  reinterpret_cast<void**>(&w.permute_scratch)};
-    for (void** p : ptrs) {
-        if (*p != nullptr) {
-            LM_HIP(hipFree(*p));
-            *p = nullptr;
-        }
-    }
     const int64_t T = std::max<int64_t>(tokens, 1);
     const int64_t TK = T * ctx->K;
     const int64_t E = ctx->E;
     const int64_t widest = std::max<int64_t>({ctx->Ip, ctx->Sp, ctx->Dp});
-    const size_t act_elems = static_cast<size_t>(TK * ctx->Ip + T * widest);
-    LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.idx), sizeof(int32_t) * static_cast<size_t>(TK)));
-    LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.wts), sizeof(float) * static_cast<size_t>(TK)));
-    LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.counts), sizeof(int32_t) * static_cast<size_t>(E + 1)));
-    LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.offsets), sizeof(int32_t) * static_cast<size_t>(E + 2)));
-    LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.active), sizeof(int32_t) * static_cast<size_t>(E + 2)));
-    LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.perm), sizeof(int32_t) * static_cast<size_t>(TK)));
-    LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.slot_of), sizeof(int32_t) * static_cast<size_t>(TK)));
-    LM_HIP(hipMalloc(&w.act, sizeof(float) * act_elems));
-    LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.x16), sizeof(_Float16) * static_cast<size_t>(T * ctx->Hp)));
-    LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.down_out),
-                     sizeof(float) * static_cast<size_t>(lm::down_rows(T, ctx->K, ctx->Ip, ctx->Sp) * ctx->H)));
-    LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.xnorm), sizeof(float) * static_cast<size_t>(T * ctx->H)));
-    LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.ffn), sizeof(float) * static_cast<size_t>(T * ctx->H)));
-    LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.zero), sizeof(int32_t) * 4));
-    LM_HIP(hipMemsetAsync(w.zero, 0, sizeof(int32_t) * 4, ctx->stream));
-    LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.logit_scratch),
-                     sizeof(float) * static_cast<size_t>(E) * lm::kRouterSplitTokens));
-    LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.ticket), sizeof(uint32_t) * 4));
-    LM_HIP(hipMemsetAsync(w.ticket, 0, sizeof(uint32_t) * 4, ctx->stream));
-    const size_t permute_bytes = sizeof(int32_t) * static_cast<size_t>(lm::permute_scratch_words(TK));
-    LM_HIP(hipMalloc(reinterpret_cast<void**>(&w.permute_scratch), permute_bytes));
-    LM_HIP(hipMemsetAsync(w.permute_scratch, 0, permute_bytes, ctx->stream));
+    // One allocation: a context's first call waits for each (V2-Lite, one token
+    // 127 us with 16 of them, 107 with one; 509 tokens 1007 and 392), and now and
+    // then 300 us more for one just past 2 MB.
+    struct Part {
+        void** at;
+        size_t bytes;
+    };
+    auto part = [](auto*& at, int64_t count) {
+        return Part{reinterpret_cast<void**>(&at), sizeof(*at) * static_cast<size_t>(count)};
+    };
+    float* act = nullptr;
+    const Part parts[] = {
+        // zeroed: the counter of a dense layer's absent experts, arrival tickets
+        part(w.zero, 4), part(w.ticket, 4), part(w.permute_scratch, lm::permute_scratch_words(TK)),
+        part(w.idx, TK), part(w.wts, TK), part(w.counts, E + 1), part(w.offsets, E + 2), part(w.active, E + 2),
+        part(w.perm, TK), part(w.slot_of, TK), part(w.logit_scratch, E * lm::kRouterSplitTokens),
+        part(act, TK * ctx->Ip + T * widest), part(w.x16, T * ctx->Hp),
+        part(w.down_out, lm::down_rows(T, ctx->K, ctx->Ip, ctx->Sp) * ctx->H), part(w.xnorm, T * ctx->H),
+        part(w.ffn, T * ctx->H)};
+    constexpr size_t kZeroed = 3;
+    auto padded = [](size_t bytes) { return (bytes + 4095) / 4096 * 4096; };
+    size_t total = 0, zeroed = 0;
+    for (size_t i = 0; i < std::size(parts); ++i) {
+        total += padded(parts[i].bytes);
+        zeroed = i < kZeroed ? total : zeroed;
+    }
+    w.tokens = 0;
+    w.idx = nullptr;  // nothing is usable until all is
+    LM_HIP(hipFree(w.slab));
+    w.slab = nullptr;
+    if (const hipError_t err = hipMalloc(&w.slab, total); err != hipSuccess) {
+        w.slab = nullptr;
+        (void)hipGetLastError();  // or the next launch would report it
+        return fail(LM_EHIP, "workspace of " + std::to_string(total) + " bytes: " + hipGetErrorString(err));
+    }
+    LM_HIP(hipMemsetAsync(w.slab, 0, zeroed, ctx->stream));
     LM_HIP(hipStreamSynchronize(ctx->stream));
+    char* next = static_cast<char*>(w.slab);
+    for (const Part& p : parts) {
+        *p.at = next;
+        next += padded(p.bytes);
+    }
+    w.act = act;
     w.tokens = T;
     return LM_OK;
 }
@@ -1125,11 +1132,7 @@ int lm_context_destroy(lm_context* ctx) {
         (void)hipFree(L.table);
     }
     Workspace& w = ctx->ws;
-    void* ptrs[] = {w.idx, w.wts, w.counts, w.offsets, w.active, w.perm, w.slot_of, w.act, w.x16,
-                    w.down_out, w.xnorm, w.ffn, w.zero, w.logit_scratch, w.ticket, w.permute_scratch};
-    for (void* p : ptrs) {
-        (void)hipFree(p);
-    }
+    (void)hipFree(w.slab);
     for (auto& kv : ctx->resident_ptrs) {
         (void)hipFree(kv.second.dev);
     }

@@ -96,6 +96,7 @@ struct Workspace {
     void* act = nullptr;          // fp32 (GEMV) or fp16 (MFMA) activations
     _Float16* x16 = nullptr;
     float* down_out = nullptr;
+    int64_t down_rows = 0;        // of down_out
     float* xnorm = nullptr;       // stack: normalised input
     float* ffn = nullptr;         // stack / dense: FFN output
     int32_t* zero = nullptr;      // a device int holding 0 (dense layers have no routed experts)
@@ -368,6 +369,7 @@ int ensure_workspace(lm_context* ctx, int64_t tokens) {
     const int64_t TK = T * ctx->K;
     const int64_t E = ctx->E;
     const int64_t widest = std::max<int64_t>({ctx->Ip, ctx->Sp, ctx->Dp});
+    const int64_t down_rows = lm::down_rows(T, ctx->K, ctx->Ip, ctx->Sp);
     // One allocation: a context's first call waits for each (V2-Lite, one token
     // 127 us with 16 of them, 107 with one; 509 tokens 1007 and 392), and now and
     // then 300 us more for one just past 2 MB.
@@ -385,7 +387,7 @@ int ensure_workspace(lm_context* ctx, int64_t tokens) {
         part(w.idx, TK), part(w.wts, TK), part(w.counts, E + 1), part(w.offsets, E + 2), part(w.active, E + 2),
         part(w.perm, TK), part(w.slot_of, TK), part(w.logit_scratch, E * lm::kRouterSplitTokens),
         part(act, TK * ctx->Ip + T * widest), part(w.x16, T * ctx->Hp),
-        part(w.down_out, lm::down_rows(T, ctx->K, ctx->Ip, ctx->Sp) * ctx->H), part(w.xnorm, T * ctx->H),
+        part(w.down_out, down_rows * ctx->H), part(w.xnorm, T * ctx->H),
         part(w.ffn, T * ctx->H)};
     constexpr size_t kZeroed = 3;
     auto padded = [](size_t bytes) { return (bytes + 4095) / 4096 * 4096; };
@@ -411,6 +413,7 @@ int ensure_workspace(lm_context* ctx, int64_t tokens) {
         next += padded(p.bytes);
     }
     w.act = act;
+    w.down_rows = down_rows;
     w.tokens = T;
     return LM_OK;
 }
@@ -530,6 +533,9 @@ int run_experts(lm_context* ctx, Layer& L, const float* x, const _Float16* x16, 
                 bool gateup_done = false) {
     lm::ExpertArgs ea = expert_args(ctx, L, x, x16, T, rb);
     ea.ksplit = mfma ? lm::mfma_shared_chunks(ea) : 1;
+    if (T * (ea.top_k + (ea.has_shared ? ea.ksplit : 0)) > ctx->ws.down_rows) {
+        return fail(LM_EINVAL, "the down projection's rows exceed the workspace");
+    }
     const int rc = launch_expert_kernels(ctx, L, ea, T, mfma, gateup_done);
     if (rc != LM_OK) {
         return rc;

@@ -40,17 +40,6 @@ constexpr int kKeyTile = 256;   // keys per score block (one per lane)
 constexpr int kQueries = 8;     // tokens per score / context block when T > 1
 constexpr int kChunk = 1024;    // probabilities staged in LDS per context step (T > 1)
 
-// RotaryEmbedding::apply on one channel pair: the first output is
-// even*cos - odd*sin and the second odd*cos + even*sin, each contracted to one
-// fused multiply-add whose addend is the other product rounded (GCC's
-// contraction of the reference's expressions).
-__device__ inline void rotate_pair(float e, float o, float c, float s, float& lo, float& hi) {
-    const float os = o * s;
-    const float es = e * s;
-    lo = __builtin_fmaf(e, c, -os);
-    hi = __builtin_fmaf(o, c, es);
-}
-
 // q [T, heads, qk_nope + qk_rope]: each head's rotary channels at position
 // pos0 + t (src/Attention.cpp:45-48).  One wave per (token, head); the pair
 // values are read before any is written (the rotation permutes channels).
@@ -1019,7 +1008,6 @@ __global__ __launch_bounds__(256) void context_mfma_kernel(const float* __restri
 // explicit vmcnt.  vh % 16 == 0.
 typedef __attribute__((address_space(3))) void attn_lds_void;
 // buffer descriptor word 3 for raw 32-bit buffer access on gfx950
-constexpr int kBufferWord3 = 0x00020000;
 constexpr int kCtxCh = 16;        // value channels per workgroup
 constexpr int kCtxChunk = 256;    // cached tokens per slot
 constexpr int kCtxDepth = 8;

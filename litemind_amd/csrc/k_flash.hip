@@ -39,17 +39,11 @@ constexpr int kTile = 64;                       // keys per tile
 constexpr int kNopeBytes = kTile * kNope * 2;   // 16 KB
 constexpr int kRopeBytes = kTile * kRope * 2;   // 8 KB
 constexpr int kValueBytes = kTile * kVh * 2;    // 16 KB
-constexpr int kBufferWord3 = 0x00020000;        // buffer descriptor word 3, raw 32-bit access
 
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef __attribute__((address_space(3))) void lds_void;
-
-__device__ inline void load_lds16(__amdgpu_buffer_rsrc_t from, char* to, unsigned offset, int base) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (lds_void*)to, 16, offset, base, 0, 0);
-}
 
 // ---- fp16 copies of the cache ----
 //   nope16    [heads][Kp][128]           row j = key_nope(h, :, j)
@@ -213,17 +207,17 @@ __global__ __launch_bounds__(64 * NW, 2) void flash_kernel(const FlashArgs a) {
 #pragma unroll
         for (int j = 0; j < 16 / NW; ++j) {
             const int at = wave * (16 / NW) + j;  // a multiple of four, plus j
-            load_lds16(kres, ks + at * 1024, ksrc ^ (j & 3) * 64u, tile * kNopeBytes + at * 1024);
+            buffer_lds16(kres, ks + at * 1024, ksrc ^ (j & 3) * 64u, tile * kNopeBytes + at * 1024);
         }
 #pragma unroll
         for (int j = 0; j < 8 / NW; ++j) {
             const int at = wave * (8 / NW) + j;
-            load_lds16(rres, rs + at * 1024, vsrc ^ (j & 1) * 64u, tile * kRopeBytes + at * 1024);
+            buffer_lds16(rres, rs + at * 1024, vsrc ^ (j & 1) * 64u, tile * kRopeBytes + at * 1024);
         }
 #pragma unroll
         for (int j = 0; j < 16 / NW; ++j) {
             const int at = wave * (16 / NW) + j;
-            load_lds16(vres, vs + at * 1024, vsrc ^ (j & 1) * 64u, tile * kValueBytes + at * 1024);
+            buffer_lds16(vres, vs + at * 1024, vsrc ^ (j & 1) * 64u, tile * kValueBytes + at * 1024);
         }
     };
     f32x16 o[kVh / 32] = {};

@@ -213,16 +213,8 @@ __global__ __launch_bounds__(THREADS) void head_logits_kernel(const uint16_t* __
 // 116 and 166 us, 416 and 833 with the few-token kernel's launches of 4.  [3072,
 // 2048] projection of 77 tokens 15 us (VALU chains, one token per lane: about
 // 35).  Small projections end with their longest wave: 16 stages of 8 chains.
-typedef __attribute__((address_space(3))) void head_lds_void;
-constexpr int kHeadBufferWord3 = 0x00020000;  // buffer descriptor word 3, raw 32-bit access
 // s_waitcnt immediate: vmcnt(n) (bits 3:0 and 15:14), the other counters unconstrained
 constexpr int kWaitVm(int n) { return (n & 15) | ((n >> 4) << 14) | 0x0070 | 0x0F00; }
-
-// 16 bytes per lane straight to LDS (not a template: the host pass checks a
-// template's builtin against its own target, which lacks the 16-byte form).
-__device__ inline void load_lds16(__amdgpu_buffer_rsrc_t from, float* to, unsigned offset, int base) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (head_lds_void*)to, 16, offset, base, 0, 0);
-}
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -297,9 +289,9 @@ __global__ __launch_bounds__(256, 2) void matvec_exact_kernel(const uint16_t* __
     const int nrow = static_cast<int>(std::min<int64_t>(T::kRowsT, rows - row0));
     const int stages = in_dim / T::kElems;
     const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(x + static_cast<int64_t>(t0) * in_dim), 0, ntok * in_dim * 4, kHeadBufferWord3);
+        (void*)(x + static_cast<int64_t>(t0) * in_dim), 0, ntok * in_dim * 4, kBufferWord3);
     const __amdgpu_buffer_rsrc_t wres =
-        __builtin_amdgcn_make_buffer_rsrc((void*)(w + row0 * in_dim), 0, nrow * in_dim * 2, kHeadBufferWord3);
+        __builtin_amdgcn_make_buffer_rsrc((void*)(w + row0 * in_dim), 0, nrow * in_dim * 2, kBufferWord3);
     // Load j of a stage fills 64 consecutive 16-byte positions p; position p of
     // token r = p / units holds its unit (p % units) ^ (r % 16), of a weight row
     // (p % units) ^ wswizzle(r).  Rows past the end load the last one.
@@ -322,11 +314,11 @@ __global__ __launch_bounds__(256, 2) void matvec_exact_kernel(const uint16_t* __
         stage = stage < stages ? stage : stages - 1;  // past the end: the last again (every stage issues alike)
 #pragma unroll
         for (int j = 0; j < T::kXLoads; ++j) {
-            load_lds16(xres, slot + (wave * T::kXLoads + j) * 256, xsrc[j], stage * (T::kElems * 4));
+            buffer_lds16(xres, slot + (wave * T::kXLoads + j) * 256, xsrc[j], stage * (T::kElems * 4));
         }
 #pragma unroll
         for (int j = 0; j < T::kWLoads; ++j) {
-            load_lds16(wres, slot + M * T::kElems + (wave * T::kWLoads + j) * 256, wsrc[j], stage * (T::kElems * 2));
+            buffer_lds16(wres, slot + M * T::kElems + (wave * T::kWLoads + j) * 256, wsrc[j], stage * (T::kElems * 2));
         }
     };
     // This lane's operands of a stage: step k = lane / M of token and row

@@ -4,14 +4,6 @@
 namespace lm {
 namespace {
 
-// y[t] = sum over ranks r of w[t,r] * down[slot(t,r)], accumulated in rank order
-// as out += w * dot (src/DeepSeekRunner.cpp:277-284, src/Gemm.cpp:172, which GCC
-// fuses), then + shared (:285-288), optionally + residual (gemm::axpy, :290).
-// A gather in a fixed order per token: deterministic, no float atomics.  With
-// K > 0 (the top-k known when compiling) the K rows' loads are all in flight
-// before the first addition; K = 0 reads the top-k at run time, one row at a
-// time.  The additions are the same either way.
-
 // Adds chunks 1, 2, ... of the shared row at `row` (column c, one chunk every
 // tokens rows) to chunk 0's `first`, four loads in flight.
 __device__ inline float4 add_chunks(const CombineArgs& a, float4 first, const float* row, int c) {
@@ -36,6 +28,13 @@ __device__ inline float4 add_chunks(const CombineArgs& a, float4 first, const fl
     return first;
 }
 
+// y[t] = sum over ranks r of w[t,r] * down[slot(t,r)], accumulated in rank order
+// as out += w * dot (src/DeepSeekRunner.cpp:277-284, src/Gemm.cpp:172, which GCC
+// fuses), then + shared (:285-288), optionally + residual (gemm::axpy, :290).
+// A gather in a fixed order per token: deterministic, no float atomics.  With
+// K > 0 (the top-k known when compiling) the K rows' loads are all in flight
+// before the first addition; K = 0 reads the top-k at run time, one row at a
+// time.  The additions are the same either way.
 template <int K>
 __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a) {
     const int quads = a.hidden / 4;

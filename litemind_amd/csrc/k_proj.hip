@@ -42,14 +42,6 @@ __device__ inline half4 to_half4(f32x4 v) {
 // Where key slot j of a 64-key tile lies in the core's value rows (k_flash.hip).
 __device__ inline int value_slot(int j) { return (j & 48) + (j & 4) * 2 + (j & 8) / 2 + (j & 3); }
 
-// RotaryEmbedding::apply on one pair, as k_attn.hip's rotate_pair.
-__device__ inline void rotate_pair(float e, float o, float c, float s, float& lo, float& hi) {
-    const float os = o * s;
-    const float es = e * s;
-    lo = __builtin_fmaf(e, c, -os);
-    hi = __builtin_fmaf(o, c, es);
-}
-
 // Four channels n .. n + 3 (n % 4 == 0) of token t.
 __device__ inline void store_query(const ProjArgs& a, int64_t t, int n, f32x4 v) {
     const int h = n / kQk, d = n - h * kQk;

@@ -521,18 +521,6 @@ __device__ inline void route_token_lds(float logit, bool valid, int lane, int64_
     }
 }
 
-// Direct-to-LDS buffer loads (not templates: the host pass checks a template's
-// builtin against its own target, which lacks the 16-byte form).  A buffer
-// load, unlike a global load to LDS, is not a pending flat access, after which
-// every wait for an LDS read waits for all of them.
-__device__ inline void router_load16(__amdgpu_buffer_rsrc_t from, char* to, unsigned offset, unsigned base) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (router_lds_void*)to, 16, offset, static_cast<int>(base), 0, 0);
-}
-__device__ inline void router_load4(__amdgpu_buffer_rsrc_t from, char* to, unsigned offset, unsigned base) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (router_lds_void*)to, 4, offset, static_cast<int>(base), 0, 0);
-}
-constexpr int kRouterBufferWord3 = 0x00020000;  // buffer descriptor word 3, raw 32-bit access
-
 template <int TPW, int NW, int DEPTH>
 __global__ __launch_bounds__(NW * 64) void router_wide_kernel(RouterArgs a, const float* __restrict__ x,
                                                                const float* __restrict__ wq4) {
@@ -558,9 +546,9 @@ __global__ __launch_bounds__(NW * 64) void router_wide_kernel(RouterArgs a, cons
     xt = xt < a.tokens ? xt : a.tokens - 1;
     const int64_t rows = std::min<int64_t>(NW * TPW, a.tokens - tb0);
     const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(x + tb0 * H), 0, static_cast<int>(rows * H * 4), kRouterBufferWord3);
+        (void*)(x + tb0 * H), 0, static_cast<int>(rows * H * 4), kBufferWord3);
     const __amdgpu_buffer_rsrc_t wres =
-        __builtin_amdgcn_make_buffer_rsrc((void*)wq4, 0, H * 64 * 4, kRouterBufferWord3);
+        __builtin_amdgcn_make_buffer_rsrc((void*)wq4, 0, H * 64 * 4, kBufferWord3);
     const unsigned xsrc = static_cast<unsigned>(((xt - tb0) * H + (NW == 4 ? 4 * (lane & 15) : lane)) * 4);
     const unsigned wsrc = static_cast<unsigned>((wave * 256 + 4 * lane) * 4);
     auto issue = [&](int c, char* buf) {
@@ -569,16 +557,16 @@ __global__ __launch_bounds__(NW * 64) void router_wide_kernel(RouterArgs a, cons
 #pragma unroll
         for (int j = 0; j < S::kWLoads; ++j) {
             const int n = j * NW + wave;  // 1 KB block n of the chunk's gate rows
-            router_load16(wres, buf + n * 1024, wsrc, i0 * 256 + j * NW * 1024);
+            buffer_lds16(wres, buf + n * 1024, wsrc, i0 * 256 + j * NW * 1024);
         }
         if constexpr (NW == 4) {
-            router_load16(xres, buf + S::kWBytes + wave * S::kXWave, xsrc, i0 * 4);
+            buffer_lds16(xres, buf + S::kWBytes + wave * S::kXWave, xsrc, i0 * 4);
         } else {
             // token k of the wave: tokens past the batch end repeat the last one
 #pragma unroll
             for (int k = 0; k < TPW; ++k) {
                 const unsigned step = tb0 + wave * TPW + k < a.tokens ? static_cast<unsigned>(k * H * 4) : 0;
-                router_load4(xres, buf + S::kWBytes + wave * S::kXWave + k * 256, xsrc, step + i0 * 4);
+                buffer_lds4(xres, buf + S::kWBytes + wave * S::kXWave + k * 256, xsrc, step + i0 * 4);
             }
         }
     };

@@ -52,6 +52,20 @@ __device__ inline void lds_barrier() {
     __builtin_amdgcn_s_barrier();
 }
 
+// Buffer loads straight to LDS, 16 or 4 bytes per lane (not templates: the host
+// pass checks a template's builtin against its own target, which lacks the
+// 16-byte form), and word 3 of their descriptor: raw 32-bit access.  Unlike a
+// global load to LDS they are no pending flat access, after which every wait for
+// an LDS read waits for all of them.
+typedef __attribute__((address_space(3))) void lds_void;
+constexpr int kBufferWord3 = 0x00020000;
+__device__ inline void buffer_lds16(__amdgpu_buffer_rsrc_t from, void* to, unsigned offset, unsigned base) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (lds_void*)to, 16, offset, static_cast<int>(base), 0, 0);
+}
+__device__ inline void buffer_lds4(__amdgpu_buffer_rsrc_t from, void* to, unsigned offset, unsigned base) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (lds_void*)to, 4, offset, static_cast<int>(base), 0, 0);
+}
+
 // 16-byte load of streamed weights: global address space (pointers read from a
 // table would otherwise compile to flat loads) and non-temporal, since every
 // weight byte is used once per step.
@@ -323,6 +337,17 @@ __device__ inline float rms_inverse_exact(double total, int n, float eps, double
     const double sum = part[0];
     barrier();  // read before a later call writes `part` or the stage again
     return static_cast<float>(1.0 / __builtin_sqrt(sum / static_cast<double>(n) + static_cast<double>(eps)));
+}
+
+// RotaryEmbedding::apply on one channel pair: the first output is
+// even*cos - odd*sin and the second odd*cos + even*sin, each contracted to one
+// fused multiply-add whose addend is the other product rounded (GCC's
+// contraction of the reference's expressions).
+__device__ inline void rotate_pair(float e, float o, float c, float s, float& lo, float& hi) {
+    const float os = o * s;
+    const float es = e * s;
+    lo = __builtin_fmaf(e, c, -os);
+    hi = __builtin_fmaf(o, c, es);
 }
 
 // gemm::rms_norm's inverse for x[0 .. n) with 256 threads: thread t sums the

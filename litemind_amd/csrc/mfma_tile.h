@@ -13,12 +13,10 @@ namespace {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef __attribute__((address_space(3))) void lds_void;
 
 constexpr int BK = kPanel;                   // halves: 64-byte rows, 4 chunks of 16 B
 constexpr int kRowBytes = BK * 2;
 constexpr int kXcds = 8;
-constexpr int kBufferWord3 = 0x00020000;     // buffer descriptor word 3: raw 32-bit access
 
 template <int WM, int WN, int MI, int NJ, int STAGES>
 struct Shape {
@@ -53,12 +51,6 @@ __device__ inline int chunk_offset(int r, int c) { return r * kRowBytes + ((c ^ 
 // s_waitcnt with only vmcnt (expcnt and lgkmcnt at their maxima)
 #define LM_WAIT_VM(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | 0x0F70)
 
-// 16 bytes per lane straight to LDS (not a template: the host pass checks a
-// template's builtin against its own target, which lacks the 16-byte form).
-__device__ inline void tile_load16(__amdgpu_buffer_rsrc_t from, char* to, unsigned offset, unsigned base) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (lds_void*)to, 16, offset, static_cast<int>(base), 0, 0);
-}
-
 // The per-wave state of a tile and the steps of its pipeline.  One type per
 // kernel instantiation (MODE is a parameter).
 template <int MODE, int WM, int WN, int MI, int NJ, int STAGES>
@@ -76,9 +68,9 @@ struct Tile {
     // bytes, into LDS by a buffer load (the stage offset is a scalar).
     __device__ void load1(int ks, char* buf, int q) {
         if (q < Z::AL) {
-            tile_load16(ra, buf + (Z::WAVES * q + wave) * 1024, va[q], static_cast<unsigned>(ks) * a_step);
+            buffer_lds16(ra, buf + (Z::WAVES * q + wave) * 1024, va[q], static_cast<unsigned>(ks) * a_step);
         } else {
-            tile_load16(rb, buf + Z::kABytes + (Z::WAVES * (q - Z::AL) + wave) * 1024, vb[q - Z::AL],
+            buffer_lds16(rb, buf + Z::kABytes + (Z::WAVES * (q - Z::AL) + wave) * 1024, vb[q - Z::AL],
                         static_cast<unsigned>(ks) * b_step);
         }
     }
